@@ -60,6 +60,33 @@ def test_query_add_view(kvm_state, dt, layout):
     assert not got[0].any() and list(host(qa.q_count)) == [0, int(keep.sum()) + 3]
 
 
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n", [32, 33, 128, 257, 600])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_query_add_view_long_runs(kvm_state, dt, n, offset):
+    """Row counts around the long-run form's threshold and LDS buffers, and the
+    same rows from a base that is not 16-byte aligned (the general form), bit for
+    bit: both keep the row order, and a row the mask leaves out is never added
+    (it holds NaN here)."""
+    rng = np.random.default_rng(n * 3 + offset)
+    heads, D = 3, 128
+    x = torch.from_numpy((rng.standard_normal((n, heads * D)) * 3).astype(np.float32)).to(DT[dt])
+    keep = rng.random(n) < 0.7
+    keep[: min(n, 70)] &= rng.random(min(n, 70)) < 0.1
+    keep[n // 2] = True
+    x[torch.from_numpy(~keep)] = float("nan")
+    flat = torch.empty(n * heads * D + 1, dtype=DT[dt], device="cuda")
+    q = flat[offset:offset + n * heads * D].view(n, heads, D)
+    q.copy_(x.view(n, heads, D))
+    qa = api.QueryAcc(kvm_state, 1, heads, D)
+    qa.reset()
+    qa.add_view(0, q, keep)
+    rows = _f32_rows(q)
+    want = _ordered_sum(np.zeros(heads * D, np.float32), list(rows[keep]))
+    assert np.array_equal(host(qa.q_sum)[0].view(np.uint32), want.view(np.uint32))
+    assert int(qa.q_count[0]) == int(keep.sum())
+
+
 def test_query_add_view_more_rows_than_one_launch(kvm_state):
     rng = np.random.default_rng(5)
     qa = api.QueryAcc(kvm_state, 1, 2, 128)
