@@ -120,19 +120,30 @@ __global__ void __launch_bounds__(256) k_query_add_rows(qview_args a) {
         if (more) load(row0 + RB);
         if (tid < 64u) {
             const uint8_t *x = &s_rows[b][tid * ES];
-            for (uint32_t c = 0; c < RB && row0 + c < a.n_rows; c += 32u) {
-                const uint32_t k = a.keep[(row0 + c) >> 5];
-                if (k == 0u) continue;
-                float v[32];
+            const uint32_t nr = a.n_rows - row0 < RB ? a.n_rows - row0 : RB;
+            // the LDS reads of the next 32 rows run under the adds of these 32
+            float v[2][32];
+            auto read = [&](float (&o)[32], uint32_t c) {
 #pragma unroll
-                for (uint32_t i = 0; i < 32; ++i) v[i] = view_value<T>(x + (c + i) * SEG);
+                for (uint32_t i = 0; i < 32; ++i) o[i] = view_value<T>(x + (c + i) * SEG);
+            };
+            auto add = [&](const float (&o)[32], uint32_t c) {
+                const uint32_t k = a.keep[(row0 + c) >> 5];     // bits past n_rows are 0
                 if (k == 0xffffffffu) {
 #pragma unroll
-                    for (uint32_t i = 0; i < 32; ++i) s = kvm_fadd(s, v[i]);
+                    for (uint32_t i = 0; i < 32; ++i) s = kvm_fadd(s, o[i]);
                 } else {
 #pragma unroll
-                    for (uint32_t i = 0; i < 32; ++i) s = (k >> i) & 1u ? kvm_fadd(s, v[i]) : s;
+                    for (uint32_t i = 0; i < 32; ++i) s = (k >> i) & 1u ? kvm_fadd(s, o[i]) : s;
                 }
+            };
+            read(v[0], 0);
+            for (uint32_t c = 0; c < nr; c += 64u) {
+                read(v[1], c + 32u < RB ? c + 32u : 0u);
+                add(v[0], c);
+                if (c + 32u >= nr) break;
+                read(v[0], c + 64u < RB ? c + 64u : 0u);
+                add(v[1], c + 32u);
             }
         }
         if (more) store(b ^ 1u);
@@ -322,28 +333,63 @@ extern "C" size_t kvm_meank_k_sum_floats(const kvm_meank_index *ix) {
     return (size_t)ix->n_layer * tiles * KVM_MEANK_TILE * ix->n_head_kv * ix->head_dim;
 }
 
-// One block's share (chunk ci of the positions pos0 .. pos0+n-1) per
-// blockIdx.y; the view's token pos - pos0 + tok0 holds position pos.
-__global__ void k_meank_add(float *k_sum, uint32_t *mean_tokens, uint8_t *present, uint32_t cap,
-                            uint32_t n_embd, uint32_t bt, uint32_t pos0, uint32_t n, view_args v, uint32_t tok0) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+// One block's share (chunk ci = blockIdx.y of the positions pos0 .. pos0+n-1)
+// of 256 embeddings per workgroup; the view's token pos - pos0 + tok0 holds
+// position pos.  What bounds it is the memory round trips of a block's ordered
+// rows, so the loads of 64 rows are issued together (unconditional: rows past
+// the share re-read its last one): two round trips for a 128-token block.  TD:
+// 0, or the head_dim (128, 256) of an index that carries the block terms, whose
+// new nk the workgroup then forms from its sums (256 / TD heads) as
+// k_meank_terms does, without a launch of its own.  A 2,048-token bf16 chunk of
+// 4 x 256 values took 40 us with a load in flight at a time, and 4.8 for the
+// terms' launch.
+struct meank_add_args {
+    float *k_sum;
+    uint32_t *mean_tokens;
+    uint8_t *present;
+    float *k_norm;               // the layer's [H][cap] (TD > 0)
+    view_args v;
+    uint32_t cap, n_embd, bt, pos0, n, tok0;
+};
+template <int T, int TD>
+__global__ void __launch_bounds__(256) k_meank_add(meank_add_args a) {
+    constexpr uint32_t B = 64;
+    const uint32_t tid = threadIdx.x, e = blockIdx.x * 256u + tid;
     const uint32_t ci = blockIdx.y;                  // chunk = one block's share
-    const uint32_t bid = pos0 / bt + ci;
-    const uint32_t start = ci == 0 ? pos0 : bid * bt;
-    const uint32_t end_blk = (bid + 1) * bt;
-    const uint32_t end = pos0 + n < end_blk ? pos0 + n : end_blk;
-    if (bid >= cap || start >= end) return;
-    const uint32_t off = start - bid * bt, take = end - start;
-    if (e < n_embd) {
-        float *p = k_sum + kvm_meank_off(n_embd, e, bid);
-        float s = off == 0 ? 0.0f : *p;
-        for (uint32_t t = start; t < end; ++t) s = kvm_fadd(s, view_load(v, t - pos0 + tok0, e));
+    const uint32_t bid = a.pos0 / a.bt + ci;
+    const uint32_t start = ci == 0 ? a.pos0 : bid * a.bt;
+    const uint32_t end_blk = (bid + 1) * a.bt;
+    const uint32_t end = a.pos0 + a.n < end_blk ? a.pos0 + a.n : end_blk;
+    if (bid >= a.cap || start >= end) return;
+    const uint32_t off = start - bid * a.bt, take = end - start;
+    // (off > 0: another workgroup of the block may have stored its new count
+    // already, which gives the same maximum)
+    const uint32_t mt = off == 0 ? 0u : a.mean_tokens[bid];
+    const uint32_t cnt = mt > off + take ? mt : off + take;
+    float s = 0.0f;
+    if (e < a.n_embd) {
+        float *p = a.k_sum + kvm_meank_off(a.n_embd, e, bid);
+        const uint8_t *x0 = a.v.data + (size_t)(start - a.pos0 + a.tok0) * a.v.nb2 + view_off(a.v, e);
+        if (off != 0) s = *p;
+        for (uint32_t t0 = 0; t0 < take; t0 += B) {
+            float x[B];
+#pragma unroll
+            for (uint32_t i = 0; i < B; ++i) x[i] = view_value<T>(x0 + (size_t)(t0 + i < take ? t0 + i : take - 1) * a.v.nb2);
+#pragma unroll
+            for (uint32_t i = 0; i < B; ++i) s = t0 + i < take ? kvm_fadd(s, x[i]) : s;
+        }
         *p = s;
     }
     if (e == 0) {
-        const uint32_t mt = mean_tokens[bid];
-        mean_tokens[bid] = off == 0 ? take : (mt > off + take ? mt : off + take);
-        if (present) present[bid] = 1;
+        a.mean_tokens[bid] = cnt;
+        if (a.present) a.present[bid] = 1;
+    }
+    if constexpr (TD > 0) {
+        __shared__ __align__(16) float s_sq[256];
+        const float kh = kvm_fmul(s, kvm_recip_or0((float)cnt));        // cnt > 0
+        s_sq[tid] = kvm_fmul(kh, kh);
+        __syncthreads();
+        if (tid % TD == 0 && e < a.n_embd) a.k_norm[(uint64_t)(e / TD) * a.cap + bid] = ordered_sum<TD>(s_sq + tid);
     }
 }
 
@@ -359,29 +405,22 @@ static uint64_t meank_layer_floats(const kvm_meank_index *ix) {
 }
 
 // The index's block terms (k_norm) of blocks b0 .. b0 + gridDim.x - 1, kv head
-// blockIdx.y, layer il0 + blockIdx.z, one wave each: lane l forms kh of dims
-// l, l + 64, ... as the scorer does (k_sum * (1 / mean_tokens), 0 without
-// tokens), then lane 0 sums kh^2 over the dims in order from LDS.
+// blockIdx.y, layer il0 + blockIdx.z: thread d forms kh of dim d as the scorer
+// does (k_sum * (1 / mean_tokens), 0 without tokens), then one lane sums kh^2
+// over the dims in order from LDS.
 template <int D>
-__global__ void __launch_bounds__(64) k_meank_terms(const float *k_sum, const uint32_t *mean_tokens, float *k_norm,
-                                                    uint64_t layer_floats, uint32_t cap, uint32_t H, uint32_t il0,
-                                                    uint32_t b0) {
-    const uint32_t b = b0 + blockIdx.x, h = blockIdx.y, il = il0 + blockIdx.z, l = threadIdx.x, n_embd = H * D;
-    __shared__ float s_sq[D];
+__global__ void __launch_bounds__(D) k_meank_terms(const float *k_sum, const uint32_t *mean_tokens, float *k_norm,
+                                                   uint64_t layer_floats, uint32_t cap, uint32_t H, uint32_t il0,
+                                                   uint32_t b0) {
+    const uint32_t b = b0 + blockIdx.x, h = blockIdx.y, il = il0 + blockIdx.z, d = threadIdx.x;
+    __shared__ __align__(16) float s_sq[D];
     const uint32_t mt = mean_tokens[(uint64_t)il * cap + b];
-    const float inv = kvm_recip_or0((float)mt);
+    const float ks = k_sum[(uint64_t)il * layer_floats + kvm_meank_off(H * D, h * D + d, b)];
     const uint32_t keep = mt ? 0xffffffffu : 0u;
-    const float *ks = k_sum + (uint64_t)il * layer_floats;
-    for (uint32_t d = l; d < (uint32_t)D; d += 64u) {
-        const float kh = __uint_as_float(__float_as_uint(kvm_fmul(ks[kvm_meank_off(n_embd, h * D + d, b)], inv)) & keep);
-        s_sq[d] = kvm_fmul(kh, kh);
-    }
+    const float kh = __uint_as_float(__float_as_uint(kvm_fmul(ks, kvm_recip_or0((float)mt))) & keep);
+    s_sq[d] = kvm_fmul(kh, kh);
     __syncthreads();
-    if (l == 0) {
-        float nk = 0.0f;
-        for (uint32_t d = 0; d < (uint32_t)D; ++d) nk = kvm_fadd(nk, s_sq[d]);
-        k_norm[((uint64_t)il * H + h) * cap + b] = nk;
-    }
+    if (d == 0) k_norm[((uint64_t)il * H + h) * cap + b] = ordered_sum<D>(s_sq);
 }
 
 // Forms k_norm of layers [il0, il0 + n_lay) and blocks [b0, b1) on the state's stream.
@@ -390,10 +429,10 @@ static int meank_terms_launch(kvm_state *st, const kvm_meank_index *ix, uint32_t
     if (!ix->k_norm || n_lay == 0 || b1 <= b0) return KVM_OK;
     const dim3 grid(b1 - b0, ix->n_head_kv, n_lay);
     if (ix->head_dim == 256)
-        hipLaunchKernelGGL(k_meank_terms<256>, grid, dim3(64), 0, st->stream, ix->k_sum, ix->mean_tokens, ix->k_norm,
+        hipLaunchKernelGGL(k_meank_terms<256>, grid, dim3(256), 0, st->stream, ix->k_sum, ix->mean_tokens, ix->k_norm,
                            meank_layer_floats(ix), ix->n_blocks, ix->n_head_kv, il0, b0);
     else
-        hipLaunchKernelGGL(k_meank_terms<128>, grid, dim3(64), 0, st->stream, ix->k_sum, ix->mean_tokens, ix->k_norm,
+        hipLaunchKernelGGL(k_meank_terms<128>, grid, dim3(128), 0, st->stream, ix->k_sum, ix->mean_tokens, ix->k_norm,
                            meank_layer_floats(ix), ix->n_blocks, ix->n_head_kv, il0, b0);
     KVM_LAUNCH_CHECK(st, "meank_terms");
     return KVM_OK;
@@ -431,12 +470,21 @@ static int meank_add_view(kvm_state *st, const kvm_meank_index *ix, uint32_t il,
                                               (unsigned long long)last, ix->n_blocks);
     KVM_HIP(st, hipSetDevice(st->device));
     const uint32_t n_chunks = (uint32_t)(last - pos0 / bt + 1);
-    hipLaunchKernelGGL(k_meank_add, dim3(kvm_cdiv(n_embd, 256), n_chunks), dim3(256), 0, st->stream,
-                       ix->k_sum + (uint64_t)il * meank_layer_floats(ix),
-                       ix->mean_tokens + (uint64_t)il * ix->n_blocks, ix->present, ix->n_blocks, n_embd,
-                       bt, pos0, n, view_of(k), tok0);
+    const meank_add_args a{ix->k_sum + (uint64_t)il * meank_layer_floats(ix), ix->mean_tokens + (uint64_t)il * ix->n_blocks,
+                           ix->present, ix->k_norm ? ix->k_norm + (uint64_t)il * ix->n_head_kv * ix->n_blocks : nullptr,
+                           view_of(k), ix->n_blocks, n_embd, bt, pos0, n, tok0};
+    const dim3 grid(kvm_cdiv(n_embd, 256), n_chunks);
+    auto go = [&](auto t) {
+        constexpr int T = decltype(t)::value;
+        if (!ix->k_norm) hipLaunchKernelGGL((k_meank_add<T, 0>), grid, dim3(256), 0, st->stream, a);
+        else if (ix->head_dim == 256) hipLaunchKernelGGL((k_meank_add<T, 256>), grid, dim3(256), 0, st->stream, a);
+        else hipLaunchKernelGGL((k_meank_add<T, 128>), grid, dim3(256), 0, st->stream, a);
+    };
+    if (k->type == KVM_TYPE_F16) go(std::integral_constant<int, KVM_TYPE_F16>{});
+    else if (k->type == KVM_TYPE_BF16) go(std::integral_constant<int, KVM_TYPE_BF16>{});
+    else go(std::integral_constant<int, KVM_TYPE_F32>{});
     KVM_LAUNCH_CHECK(st, "meank_add");
-    return meank_terms_launch(st, ix, il, 1, pos0 / bt, (uint32_t)last + 1);
+    return KVM_OK;
 }
 
 extern "C" int kvm_meank_add_view(kvm_state *st, const kvm_meank_index *ix, uint32_t il, uint32_t pos0,
@@ -460,11 +508,22 @@ extern "C" int kvm_meank_add(kvm_state *st, const kvm_meank_index *ix, uint32_t 
 // (RawKvStore::write_layer_mean_sum, raw_kv_store.cpp:707-731, as
 // decode_mean_flush applies it, llama-memory-kvmem.cpp:3939-3993).
 // ---------------------------------------------------------------------------
-__global__ void k_meank_acc_add(float *acc, uint32_t n_embd, view_args v, uint32_t tok0, uint32_t n_keep) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+// One thread per embedding, the loads of eight tokens in flight (a decode
+// step's tokens in one round trip).
+template <int T>
+__global__ void __launch_bounds__(64) k_meank_acc_add(float *acc, uint32_t n_embd, view_args v, uint32_t tok0,
+                                                      uint32_t n_keep) {
+    const uint32_t e = blockIdx.x * 64u + threadIdx.x;
     if (e >= n_embd) return;
+    const uint8_t *p = v.data + (size_t)tok0 * v.nb2 + view_off(v, e);
     float s = acc[e];
-    for (uint32_t t = 0; t < n_keep; ++t) s = kvm_fadd(s, view_load(v, tok0 + t, e));
+    for (uint32_t t0 = 0; t0 < n_keep; t0 += 8) {
+        float x[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) x[i] = view_value<T>(p + (size_t)(t0 + i < n_keep ? t0 + i : n_keep - 1) * v.nb2);
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) s = t0 + i < n_keep ? kvm_fadd(s, x[i]) : s;
+    }
     acc[e] = s;
 }
 
@@ -507,8 +566,13 @@ extern "C" int kvm_meank_acc_add(kvm_state *st, const kvm_meank_index *ix, uint3
     if (n_keep == 0) return KVM_OK;
     if ((uint64_t)tok0 + n_keep > (uint64_t)k->ne2) return kvm_fail(st, KVM_ERANGE, "meank_acc_add: tokens past the view");
     KVM_HIP(st, hipSetDevice(st->device));
-    hipLaunchKernelGGL(k_meank_acc_add, dim3(kvm_cdiv(n_embd, 256)), dim3(256), 0, st->stream,
-                       ix->acc + (uint64_t)il * n_embd, n_embd, view_of(k), tok0, n_keep);
+    auto go = [&](auto t) {
+        hipLaunchKernelGGL(k_meank_acc_add<decltype(t)::value>, dim3(kvm_cdiv(n_embd, 64)), dim3(64), 0, st->stream,
+                           ix->acc + (uint64_t)il * n_embd, n_embd, view_of(k), tok0, n_keep);
+    };
+    if (k->type == KVM_TYPE_F16) go(std::integral_constant<int, KVM_TYPE_F16>{});
+    else if (k->type == KVM_TYPE_BF16) go(std::integral_constant<int, KVM_TYPE_BF16>{});
+    else go(std::integral_constant<int, KVM_TYPE_F32>{});
     KVM_LAUNCH_CHECK(st, "meank_acc_add");
     return KVM_OK;
 }

@@ -120,6 +120,30 @@ def test_meank_add_view(kvm_state, dt, layout):
     assert list(host(ix.present)[:5]) == [1, 1, 1, 1, 0]
 
 
+@pytest.mark.parametrize("H,D,bt", [(4, 256, 128), (3, 128, 64), (1, 128, 192)])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_meank_add_forms_block_terms(kvm_state, H, D, bt, dt):
+    """An add over ragged position ranges (a part of one block, whole blocks, the
+    block continued) leaves the sums of an index without terms and the terms
+    kvm_meank_refresh forms from those sums, bit for bit; blocks it did not
+    touch keep theirs."""
+    rng = np.random.default_rng(H * D + bt)
+    nb = 6
+    ix = api.MeanKIndex(kvm_state, 1, nb, H, D, bt, norms=True)
+    plain = api.MeanKIndex(kvm_state, 1, nb, H, D, bt)
+    ix.k_norm.fill_(-1.0)
+    for pos0, n in ((0, 1), (bt + 5, 2 * bt), (3 * bt + 5, bt - 5 + 3)):
+        k = _captured(rng, n, H, D, dt, "contiguous")
+        ix.add_view(0, pos0, k)
+        plain.add_view(0, pos0, k)
+    assert torch.equal(ix.k_sum.view(torch.int32), plain.k_sum.view(torch.int32))
+    assert torch.equal(ix.mean_tokens, plain.mean_tokens)
+    got = ix.k_norm.clone()
+    assert bool((got[0, :, 5] == -1.0).all())
+    ix.refresh()
+    assert torch.equal(got[0, :, :5].contiguous().view(torch.int32), ix.k_norm[0, :, :5].contiguous().view(torch.int32))
+
+
 def test_meank_decode_running_sum_and_flush(kvm_state):
     """Accepted decode tokens go to the running sum (two commits, the second
     keeping 2 of 3 MTP tokens), which is flushed into a block the prompt left
