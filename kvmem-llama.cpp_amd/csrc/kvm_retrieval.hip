@@ -38,6 +38,18 @@ __device__ __forceinline__ float view_value(const uint8_t *p) {
     else if constexpr (T == KVM_TYPE_BF16) return kvm_bf2f(*(const uint16_t *)p);
     else return *(const float *)p;
 }
+// The same in two steps, so that loads can be issued ahead of every conversion.
+template <int T>
+__device__ __forceinline__ uint32_t view_raw(const uint8_t *p) {
+    if constexpr (T == KVM_TYPE_F32) return *(const uint32_t *)p;
+    else return *(const uint16_t *)p;
+}
+template <int T>
+__device__ __forceinline__ float raw_value(uint32_t u) {
+    if constexpr (T == KVM_TYPE_F16) return kvm_h2f((uint16_t)u);
+    else if constexpr (T == KVM_TYPE_BF16) return kvm_bf2f((uint16_t)u);
+    else return __uint_as_float(u);
+}
 // Byte offset of embedding e within a token of the view.
 __device__ __forceinline__ size_t view_off(const view_args &v, uint32_t e) {
     return (size_t)(e / v.ne0) * v.nb1 + (size_t)(e % v.ne0) * v.nb0;
@@ -99,25 +111,26 @@ __global__ void __launch_bounds__(256) k_query_add_rows(qview_args a) {
     __shared__ __align__(16) uint8_t s_rows[2][RB * SEG];
     const uint32_t tid = threadIdx.x, e0 = blockIdx.x * 64u;
     const uint8_t *p = a.v.data + (size_t)a.t0 * a.v.nb2 + view_off(a.v, e0) + 16u * (tid % UPR);
-    kvm_u32x4 r[B];
-    auto load = [&](uint32_t row0) {
+    // register sets: buffer c + 1's rows in one, c + 2's in the other
+    kvm_u32x4 r[2][B];
+    auto load = [&](kvm_u32x4 (&q)[B], uint32_t row0) {
 #pragma unroll
         for (uint32_t j = 0; j < B; ++j) {
             const uint32_t row = row0 + (j * 256u + tid) / UPR;
-            r[j] = *(const kvm_u32x4 *)(p + (size_t)(row < a.n_rows ? row : a.n_rows - 1) * a.v.nb2);
+            q[j] = *(const kvm_u32x4 *)(p + (size_t)(row < a.n_rows ? row : a.n_rows - 1) * a.v.nb2);
         }
     };
-    auto store = [&](uint32_t b) {
+    auto store = [&](const kvm_u32x4 (&q)[B], uint32_t b) {
 #pragma unroll
-        for (uint32_t j = 0; j < B; ++j) *(kvm_u32x4 *)&s_rows[b][16u * (j * 256u + tid)] = r[j];
+        for (uint32_t j = 0; j < B; ++j) *(kvm_u32x4 *)&s_rows[b][16u * (j * 256u + tid)] = q[j];
     };
-    load(0);
+    load(r[0], 0);
+    load(r[1], RB);
     float s = tid < 64u ? a.q_sum[e0 + tid] : 0.0f;
-    store(0);
+    store(r[0], 0);
     __syncthreads();
-    for (uint32_t row0 = 0, b = 0; row0 < a.n_rows; row0 += RB, b ^= 1u) {
-        const bool more = row0 + RB < a.n_rows;
-        if (more) load(row0 + RB);
+    auto step = [&](uint32_t row0, uint32_t b, kvm_u32x4 (&later)[B], const kvm_u32x4 (&next)[B]) {
+        load(later, row0 + 2 * RB);
         if (tid < 64u) {
             const uint8_t *x = &s_rows[b][tid * ES];
             const uint32_t nr = a.n_rows - row0 < RB ? a.n_rows - row0 : RB;
@@ -146,8 +159,12 @@ __global__ void __launch_bounds__(256) k_query_add_rows(qview_args a) {
                 add(v[1], c + 32u);
             }
         }
-        if (more) store(b ^ 1u);
+        store(next, b ^ 1u);
         __syncthreads();
+    };
+    for (uint32_t row0 = 0; row0 < a.n_rows; row0 += 2 * RB) {
+        step(row0, 0, r[0], r[1]);
+        if (row0 + RB < a.n_rows) step(row0 + RB, 1, r[1], r[0]);
     }
     if (tid < 64u) a.q_sum[e0 + tid] = s;
     if (e0 == 0 && tid == 0) a.q_count[0] += a.n_kept;
@@ -372,11 +389,12 @@ __global__ void __launch_bounds__(256) k_meank_add(meank_add_args a) {
         const uint8_t *x0 = a.v.data + (size_t)(start - a.pos0 + a.tok0) * a.v.nb2 + view_off(a.v, e);
         if (off != 0) s = *p;
         for (uint32_t t0 = 0; t0 < take; t0 += B) {
-            float x[B];
+            uint32_t x[B];
 #pragma unroll
-            for (uint32_t i = 0; i < B; ++i) x[i] = view_value<T>(x0 + (size_t)(t0 + i < take ? t0 + i : take - 1) * a.v.nb2);
+            for (uint32_t i = 0; i < B; ++i) x[i] = view_raw<T>(x0 + (size_t)(t0 + i < take ? t0 + i : take - 1) * a.v.nb2);
+            __builtin_amdgcn_sched_barrier(0);       // all of them in flight
 #pragma unroll
-            for (uint32_t i = 0; i < B; ++i) s = t0 + i < take ? kvm_fadd(s, x[i]) : s;
+            for (uint32_t i = 0; i < B; ++i) s = t0 + i < take ? kvm_fadd(s, raw_value<T>(x[i])) : s;
         }
         *p = s;
     }
