@@ -9,542 +9,898 @@
 // and a multi-token query, ggml's GPU backends convert K and V to f16 and run
 // an f16 matrix-core kernel; this file does the same with CDNA4 MFMA.
 //
-// Launch 1, k_pf_stage: per (kv head, 64-cell tile) the q8_0 K / q4_0 V (or
-// f16 / f16) tile becomes f16 MFMA operand tiles in the workspace, and tile
-// 0..n of the window gets a (min pos, max pos, live cells) summary.
-//   K f16 tile: [sub 4][kstep D/32][lane 64][8 halves], lane 16g+m = key
-//               16*sub+m, dims 32*kstep+8g..+7 (the A operand of S^T = K Q^T).
-//   V f16 tile: [dim tile D/16][kstep 2][lane 64][8 halves], lane 16g+m = dim
-//               16*dt+m; half j = 4h+r is key 32*kstep + 16h + 4g + r.  That
-//               key order is the order in which S^T's accumulator holds the
-//               scores (key 4g+r of each 16-key sub tile), so P goes from the
-//               S^T accumulator into the B operand of O^T = V^T P^T without a
-//               cross-lane exchange.
-// Launch 2, k_pf_attn: one workgroup per (128 query rows, kv head, key split);
-// a row is (token, query head of the group), so the 6 query heads of a kv
-// head share every K/V tile.  8 waves x 16 rows (two waves per SIMD).  K/V tiles are copied from
-// global memory straight into LDS (double buffered, one barrier per tile); the
-// tiles of the workgroup's key range that some row can see are listed in LDS
-// once at the start.  Q stays in registers as f16 B
-// operands; O^T (16 rows x D per wave) lives in the accumulators.  Online softmax in the
-// log2 domain with a lazy running maximum (rescale only when a row max grows
-// by more than 2^8).  Tiles no row of the workgroup can see are skipped;
-// tiles every row sees in full skip the mask.
-// Launch 3 (key splits > 1), k_pf_combine: merges the split partials.
+// k_pf_attn: one workgroup of 8 waves per CU; a row is (token, query head of the
+// group), so the query heads of a kv head share every K/V tile.  Each wave has 32
+// rows: the 32x32x16 MFMA reads half the LDS bytes per flop of 16 rows a wave.  A
+// unit is 256 / KW rows of a kv head (KW = 2: two waves share 32 rows, one on each
+// half of a tile's keys, and meet at the end).  The units' keys are dealt to the
+// workgroups in equal shares (pf_shares), so the CUs have the same work whatever
+// the shape; k_pf_combine merges the units that several workgroups share.
+// S^T = K Q^T and O^T += V^T P^T.  Key order: score row i of a 32-key sub tile is
+// key i with bits 2 and 3 swapped (the lane that supplies K row i reads that key),
+// so that the accumulator holds for each lane the 8 consecutive keys that the P V
+// operand wants and P needs no cross-lane exchange.  Online softmax in the log2
+// domain with a lazy running maximum (rescale only when a row max grows by more
+// than 2^8).  Tiles no row of the unit can see are left out of its list; tiles
+// every row sees in full skip the mask.
+// Where the tiles come from (SRC, pf_choose):
+//   PF_F16    an f16 window's tiles, which are the MFMA operands already, copied
+//             global -> LDS, double buffered;
+//   PF_STAGED the same from a workspace into which k_pf_stage converted the
+//             quantised window: one conversion for all row tiles;
+//   PF_QUANT  the quantised tiles, copied as they are and converted in LDS by
+//             the attention itself, between its MFMAs (few row tiles).
+// f16 tiles: K as kvm_kh_idx; V units of 8 keys of a dim (as kvm_vh_idx), in LDS
+// and in the workspace in the order [32-key half][16-dim tile][8-key group][dim].
+// What bounds it: large chunks, the matrix cores at the clock that the power limit
+// leaves (2,048 tokens x 34,816 cells: 1.10 -> 1.15 PFLOP/s, a large f16 matrix
+// product reaches 1.33); small ones, the latencies of the start and the piece
+// traffic (37 tokens x 32,768 cells: 147 -> 65 us; 100 x 8,192: 54.3 -> 47;
+// 700 x 8,192 on an f16 cache of 2 heads x 128: 51.6 -> 42).
 #include "kvm_internal.h"
 
-#include <climits>
+#include <type_traits>
 
-#define KVM_PF_ROWS 128          // query rows per workgroup
-#define KVM_PF_MAX_SPLITS 8
 #define KVM_PF_LAZY 8.0f         // log2 growth of a row max tolerated before a rescale
-#define KVM_PF_LIST 8192         // most tiles one key split may hold
+#define KVM_PF_LIST 8192u        // tiles of a segment: the keys of a unit are listed at most this many tiles at a time
+
+// Nothing moves over it, the MFMA that wrote x included: the operand loads stay
+// where the ring issues them (a scheduling barrier alone keeps the loads, but the
+// MFMAs, which nothing orders, sink below all of them and every operand is live).
+#define PF_PIN(x)                                    \
+    do {                                             \
+        asm volatile("" : "+v"(x) : : "memory");     \
+        __builtin_amdgcn_sched_barrier(0);           \
+    } while (0)
+
+enum { PF_STAGED, PF_F16, PF_QUANT };
 
 typedef __attribute__((address_space(3))) void *kvm_lds_ptr;
+typedef float kvm_f32x16 __attribute__((ext_vector_type(16)));
+typedef float kvm_f32x2 __attribute__((ext_vector_type(2)));
 
 extern "C" int kvm_fa_prefill_chunked(kvm_state *st, const kvm_window *w, const void *q, int q_type,
                                       const int32_t *q_pos, uint32_t n_tokens, uint32_t n_head,
                                       float scale, float *out);
 
+// ---------------------------------------------------------------------------
+// Quantised tile -> f16 operands.  A byte under 0x64 is the f16 number 1024 +
+// byte, so four values take two v_perm and two packed subtractions (exact); the
+// packed product with the f16 scale rounds once, as (f16)((float)q * d) does.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ kvm_f16x2 pf_bits2(uint32_t u) {
+    kvm_f16x2 v;
+    __builtin_memcpy(&v, &u, 4);
+    return v;
+}
+__device__ __forceinline__ void pf_pairs(uint32_t bytes, kvm_f16x2 &a, kvm_f16x2 &b) {
+    a = pf_bits2(__builtin_amdgcn_perm(0x64646464u, bytes, 0x04010400u));
+    b = pf_bits2(__builtin_amdgcn_perm(0x64646464u, bytes, 0x04030402u));
+}
+// 8 int8 quants times one scale
+__device__ __forceinline__ kvm_f16x8 pf_q8(uint32_t w0, uint32_t w1, uint32_t dbits) {
+    const kvm_f16x2 off = {(_Float16)1152.0f, (_Float16)1152.0f}, d = pf_bits2(dbits * 0x10001u);
+    kvm_f16x2 r[4];
+    pf_pairs(w0 ^ 0x80808080u, r[0], r[1]);
+    pf_pairs(w1 ^ 0x80808080u, r[2], r[3]);
+    kvm_f16x8 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[i] = (r[i] - off) * d;
+        o[2 * i] = r[i][0];
+        o[2 * i + 1] = r[i][1];
+    }
+    return o;
+}
+// the 8 q4_0 nibbles of a V word (kvm_vq_nib_shift) times their keys' scales
+__device__ __forceinline__ kvm_f16x8 pf_q4(uint32_t w, kvm_u32x4 scales) {
+    const kvm_f16x2 off = {(_Float16)1032.0f, (_Float16)1032.0f};
+    kvm_f16x2 r[4];
+    pf_pairs(w & 0x0f0f0f0fu, r[0], r[1]);
+    pf_pairs((w >> 4) & 0x0f0f0f0fu, r[2], r[3]);
+    kvm_f16x8 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[i] = (r[i] - off) * pf_bits2(scales[i]);
+        o[2 * i] = r[i][0];
+        o[2 * i + 1] = r[i][1];
+    }
+    return o;
+}
+
+// x, from which the compiler cannot tell that a value formed of it does not
+// change in a loop: hoisted, lane addresses take the registers that the
+// accumulators need.
+__device__ __forceinline__ uint32_t opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return (uint32_t)x;
+}
+
 struct pf_stage_args {
-    const uint8_t *k, *v;        // window K / V tiles
+    const uint8_t *k, *v;        // window K / V tiles (q8_0 / q4_0)
     const int32_t *cell_pos;
-    _Float16 *kh, *vh;           // f16 operand tiles [H][n_tiles][64 * D]
+    uint8_t *kh, *vh;            // f16 operand tiles [H][n_tiles][64 * D]
     int32_t *info;               // [n_tiles][4]: min live pos, max live pos, live cells, 0
     uint32_t n_tiles;
-    int k_q8, v_q4;
 };
-
-__device__ inline float q8_val(uint32_t w, int byte) {
-    return (float)(int8_t)(uint8_t)(w >> (8 * byte));
-}
-__device__ inline float q4_val(uint32_t w, uint32_t j) {
-    return (float)((int)((w >> kvm_vq_nib_shift(j)) & 15u) - 8);
-}
 
 template <int D>
 __global__ void __launch_bounds__(256) k_pf_stage(pf_stage_args a) {
     constexpr int NB = D / 32;
     const uint32_t t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const uint64_t tile = (uint64_t)h * a.n_tiles + t;
-    _Float16 *kh = a.kh + tile * 64 * D;
-    _Float16 *vh = a.vh + tile * 64 * D;
-    if (a.k_q8) {
-        // unit = the 16 quant bytes of (sub s, block pair p, lane 16g+m): key
-        // 16s+m, blocks 2p and 2p+1, dims 8g..8g+7 of each
-        const uint8_t *kt = a.k + tile * kvm_ktile_bytes(KVM_TYPE_Q8_0, D);
-        for (uint32_t u = tid; u < 4u * (NB / 2) * 64u; u += 256) {
-            const uint32_t ln = u & 63u, sp = u >> 6, s = sp / (NB / 2), p = sp % (NB / 2), m = ln & 15u;
-            const kvm_u32x4 qw = *(const kvm_u32x4 *)(kt + (u << 4));
-            const float d0 = kvm_h2f(*(const uint16_t *)(kt + kvm_kd_off(D, 16 * s + m, 2 * p)));
-            const float d1 = kvm_h2f(*(const uint16_t *)(kt + kvm_kd_off(D, 16 * s + m, 2 * p + 1)));
-            kvm_f16x8 o0, o1;
+    uint8_t *kh = a.kh + tile * 128 * D, *vh = a.vh + tile * 128 * D;
+    // K unit = the 16 quant bytes of (sub s, block pair p, lane 16g+m): key
+    // 16s+m, blocks 2p and 2p+1, dims 8g..8g+7 of each
+    const uint8_t *kt = a.k + tile * kvm_ktile_bytes(KVM_TYPE_Q8_0, D);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                o0[j] = (_Float16)(q8_val(qw[j >> 2], j & 3) * d0);
-                o1[j] = (_Float16)(q8_val(qw[2 + (j >> 2)], j & 3) * d1);
-            }
-            *(kvm_f16x8 *)(kh + ((s * NB + 2 * p) * 64 + ln) * 8) = o0;
-            *(kvm_f16x8 *)(kh + ((s * NB + 2 * p + 1) * 64 + ln) * 8) = o1;
-        }
-    } else {
-        // the f16 window tile already has the operand layout
-        const kvm_u32x4 *src = (const kvm_u32x4 *)(a.k + tile * kvm_ktile_bytes(KVM_TYPE_F16, D));
-        for (uint32_t i = tid; i < 64u * D / 8; i += 256) ((kvm_u32x4 *)kh)[i] = src[i];
+    for (uint32_t u = tid; u < 4u * (NB / 2) * 64u; u += 256) {
+        const uint32_t ln = u & 63u, sp = u >> 6, s = sp / (NB / 2), p = sp % (NB / 2), m = ln & 15u;
+        const kvm_u32x4 qw = *(const kvm_u32x4 *)(kt + (u << 4));
+        const uint32_t d0 = *(const uint16_t *)(kt + kvm_kd_off(D, 16 * s + m, 2 * p));
+        const uint32_t d1 = *(const uint16_t *)(kt + kvm_kd_off(D, 16 * s + m, 2 * p + 1));
+        *(kvm_f16x8 *)(kh + ((s * NB + 2 * p) * 64 + ln) * 16) = pf_q8(qw[0], qw[1], d0);
+        *(kvm_f16x8 *)(kh + ((s * NB + 2 * p + 1) * 64 + ln) * 16) = pf_q8(qw[2], qw[3], d1);
     }
-    // V: unit = (dim tile dt, kstep ks, pair gp, dim m).  Its two source words
-    // hold keys 32ks + 8gp + j (h = 0) and 32ks + 16 + 8gp + j (h = 1), j < 8;
-    // keys j < 4 go to operand lane group 2gp, keys j >= 4 to group 2gp + 1.
+    // V unit = the two words (32-key halves) of (dim tile dt, group g, dim m)
+    const uint8_t *vt = a.v + tile * kvm_vtile_bytes(KVM_TYPE_Q4_0, D);
+#pragma unroll
     for (uint32_t u = tid; u < 4u * D; u += 256) {
-        const uint32_t m = u & 15u, gp = (u >> 4) & 1u, ks = (u >> 5) & 1u, dt = u >> 6;
-        const uint32_t d = 16 * dt + m;
-        float va[8], vb[8];
-        if (a.v_q4) {
-            const uint8_t *vt = a.v + tile * kvm_vtile_bytes(KVM_TYPE_Q4_0, D);
-            const uint32_t wa = *(const uint32_t *)(vt + kvm_vq_word(d, gp, ks));
-            const uint32_t wb = *(const uint32_t *)(vt + kvm_vq_word(d, 2 + gp, ks));
-            const uint16_t *sa = (const uint16_t *)(vt + kvm_vd_off(D, 32 * ks + 8 * gp, d >> 5));
-            const uint16_t *sb = (const uint16_t *)(vt + kvm_vd_off(D, 32 * ks + 16 + 8 * gp, d >> 5));
+        const kvm_u32x2 vw = *(const kvm_u32x2 *)(vt + 8 * u);
+        const uint8_t *sc = vt + D * 32u + ((u >> 7) * 128u + ((u >> 4) & 3u) * 16u);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                va[j] = q4_val(wa, j) * kvm_h2f(sa[j]);
-                vb[j] = q4_val(wb, j) * kvm_h2f(sb[j]);
-            }
-        } else {
-            const _Float16 *vt = (const _Float16 *)(a.v + tile * kvm_vtile_bytes(KVM_TYPE_F16, D));
-            const kvm_f16x8 ha = *(const kvm_f16x8 *)(vt + kvm_vh_idx(32 * ks + 8 * gp, d));
-            const kvm_f16x8 hb = *(const kvm_f16x8 *)(vt + kvm_vh_idx(32 * ks + 16 + 8 * gp, d));
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                va[j] = (float)ha[j];
-                vb[j] = (float)hb[j];
-            }
-        }
-        kvm_f16x8 lo, hi;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            lo[r] = (_Float16)va[r];
-            lo[4 + r] = (_Float16)vb[r];
-            hi[r] = (_Float16)va[4 + r];
-            hi[4 + r] = (_Float16)vb[4 + r];
-        }
-        *(kvm_f16x8 *)(vh + ((dt * 2 + ks) * 64 + 16 * (2 * gp) + m) * 8) = lo;
-        *(kvm_f16x8 *)(vh + ((dt * 2 + ks) * 64 + 16 * (2 * gp + 1) + m) * 8) = hi;
+        for (uint32_t ks = 0; ks < 2; ++ks)
+            *(kvm_f16x8 *)(vh + ks * 64u * D + 16 * u) = pf_q4(vw[ks], *(const kvm_u32x4 *)(sc + 64 * ks));
     }
     if (h == 0 && tid < 64) {
         const int32_t p = a.cell_pos[(uint64_t)t * 64 + tid];
-        int32_t mn = p >= 0 ? p : INT_MAX, mx = p >= 0 ? p : INT_MIN, n = p >= 0;
+        int32_t mn = p >= 0 ? p : INT32_MAX, mx = p >= 0 ? p : INT32_MIN, n = p >= 0;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             mn = min(mn, __shfl_xor(mn, o, 64));
             mx = max(mx, __shfl_xor(mx, o, 64));
             n += __shfl_xor(n, o, 64);
         }
-        if (tid == 0) {
-            int32_t *f = a.info + (uint64_t)t * 4;
-            f[0] = mn;
-            f[1] = mx;
-            f[2] = n;
-            f[3] = 0;
-        }
+        if (tid == 0) *(kvm_i32x4 *)(a.info + (uint64_t)t * 4) = kvm_i32x4{mn, mx, n, 0};
     }
 }
 
+// The keys of U units (unit u: segment u % n_seg of row tile (u / n_seg) %
+// n_row_tiles of kv head u / n_seg / n_row_tiles), each counted as P, are dealt
+// to P workgroups in order: workgroup p has [p U, (p + 1) U) of U P.  The part of
+// a unit that a workgroup has is a piece; pieces of a unit with more than one go
+// to slot 2 p (the workgroup's first unit) or 2 p + 1 (its last).
 struct pf_args {
-    const _Float16 *kh, *vh;
+    const uint8_t *k, *v;        // f16 operand tiles, f16 window tiles or quantised window tiles
     const int32_t *info, *cell_pos;
     const void *q;
     const int32_t *q_pos;
     float *out;                  // [token][n_head][D] fp32
-    float *ws_o;                 // split partials [split][H][rows_pad][D]
-    float *ws_ml;                // [split][H][rows_pad][2]: scaled max, sum
-    uint32_t n_tiles, H, G, n_head, n_rows, rows_pad, n_splits, n_row_tiles;
+    float *ws_o;                 // pieces [slot][32-row group][dim / 4 of a lane half][lane][4]
+    float *ws_ml;                // [slot][row][2]: scaled max, sum
+    uint32_t U, P;               // U P < 2^32
+    uint32_t n_tiles, n_seg, H, G, n_head, n_rows, n_row_tiles;
     float c;                     // kq_scale * log2(e)
     int q_bf16;
 };
 
-template <int D, int RT>
-__global__ void __launch_bounds__(64 * (8 / RT)) k_pf_attn(pf_args a) {
+template <int D, int KW, int SRC, bool BF16>
+__global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
     // LDS operand rings: K runs KR-1 k-steps ahead of its MFMAs, V VR-1
-    // operands ahead (the first ones in flight during the softmax), so the
-    // LDS latency hides behind matrix-core work instead of a wait per MFMA
-    constexpr int KR = 3, VR = 6;
-    constexpr int NW = 8 / RT;                            // waves; NW x RT x 16 = 128 rows
-    constexpr int KS = D / 32, DT = D / 16;
-    constexpr uint32_t TILE_H = 64u * D;                  // halves per K (or V) tile
-    __shared__ __align__(16) _Float16 s_kv[2][2 * TILE_H];   // [buffer][K tile | V tile]
-    __shared__ __align__(16) int32_t s_cp[2][64];           // the tiles' cell positions
+    // operands ahead (the first ones in flight during the softmax)
+    constexpr int KR = 3, VR = 3;
+    constexpr int RG = 8 / KW, ROWS = 32 * RG;            // row groups (of 32) of a unit
+    constexpr int KS = D / 16, DT = D / 32, NB = D / 32;
+    constexpr uint32_t TILE_B = 128u * D;                 // bytes of an f16 K (or V) tile
+    constexpr uint32_t KRAW = 64u * D + 64u * NB * 2u, VRAW = 32u * D + NB * 128u;    // quantised tiles
+    constexpr uint32_t KRAW_L = (KRAW + 1023u) & ~1023u, VRAW_L = (VRAW + 1023u) & ~1023u;
+    static_assert(SRC != PF_QUANT || KW == 2, "the converting form has one sub tile a wave");
+    constexpr uint32_t MEM = 4u * TILE_B;                 // two K/V buffers; RG * 32 rows of O when key groups merge
+    static_assert(SRC != PF_QUANT || 2u * TILE_B + 2u * (KRAW_L + VRAW_L) <= MEM, "LDS");
+    // Q in LDS: units of 16 bytes of a row, of these at a time, and where: beside
+    // the first tile's copies if it fits there
+    constexpr uint32_t Q_UNITS = D * (BF16 ? 2 : 4) / 16, Q_UC = Q_UNITS * ROWS * 16 <= MEM ? Q_UNITS : Q_UNITS / 2;
+    constexpr bool Q_EARLY = Q_UC * ROWS * 16 <= 2 * TILE_B;
+    constexpr uint32_t Q_OFS = Q_EARLY && SRC != PF_QUANT ? 2 * TILE_B : 0;
+    static_assert(Q_UC * ROWS * 16 <= MEM && (Q_UNITS == Q_UC || Q_UNITS == 2 * Q_UC), "Q passes");
+    __shared__ __align__(16) uint8_t s_mem[MEM];
+    __shared__ uint8_t s_flag[KVM_PF_LIST];               // per tile: bit 0 some cell visible to some row, bit 1 all to all
+    __shared__ __align__(16) int32_t s_cp[4][64];         // the tiles' cell positions
     __shared__ uint16_t s_list[KVM_PF_LIST];
-    __shared__ int32_t s_mm[2][NW];
-    __shared__ uint32_t s_wsum[NW];
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, m = l & 15;
+    __shared__ uint32_t s_mm[2][8];
+    __shared__ uint32_t s_cnt[KVM_PF_LIST / 64];
+    __shared__ float s_ml[KW == 2 ? 8 : 1][32][2];
+    const int tid = threadIdx.x, l = tid & 63, g2 = l >> 5, m2 = l & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = w / KW, kg = w % KW;
 
-    // Workgroup -> (row tile, kv head, split).  Consecutive hardware workgroup
-    // ids go round robin over the 8 XCDs; regroup them so one XCD runs
-    // consecutive row tiles of the same (head, split), which share their K/V
-    // tiles in that XCD's L2.
-    const uint32_t n_wg = gridDim.x;
-    uint32_t wg = blockIdx.x;
-    if ((n_wg & 7u) == 0) wg = (wg & 7u) * (n_wg >> 3) + (wg >> 3);
-    const uint32_t rt_i = wg % a.n_row_tiles, hs = wg / a.n_row_tiles;
-    const uint32_t h = hs % a.H, split = hs / a.H;
-    const uint32_t r0 = rt_i * KVM_PF_ROWS;
+    const uint32_t lds_mem = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_mem[0];
 
-    // ---- rows of this lane: r0 + 16 RT w + 16 rt + m
-    int32_t qpos[RT];
-    uint32_t rows[RT];
-    int32_t mn = INT_MAX, mx = INT_MIN;
+    // Consecutive hardware workgroup ids go round robin over the 8 XCDs; regroup
+    // them so one XCD runs consecutive shares, whose K/V tiles its L2 holds.
+    uint32_t p = blockIdx.x;
+    if ((a.P & 7u) == 0) p = (p & 7u) * (a.P >> 3) + (p >> 3);
+    const uint32_t sh0 = p * a.U, sh1 = sh0 + a.U;
+    const uint32_t u_first = sh0 / a.P, u_last = (sh1 - 1) / a.P;
+
+    for (uint32_t u = u_first; u <= u_last; ++u) {
+        const uint32_t u0 = u * a.P;
+        const uint32_t f_lo = max(sh0, u0) - u0, f_hi = min(sh1 - u0, a.P);
+        const uint32_t seg = u % a.n_seg, rest = u / a.n_seg;
+        const uint32_t rt_i = __builtin_amdgcn_readfirstlane(rest % a.n_row_tiles), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
+        const bool whole = f_lo == 0 && f_hi == a.P && a.n_seg == 1;
+
+        // ---- the loads of the prologue, all issued before any is used: the lane's
+        // row position, the tiles' cells (or summaries), the Q row
+        const uint32_t row = rt_i * ROWS + 32 * rg + m2;
+        const bool live_row = row < a.n_rows;
+        const uint32_t row_ld = live_row ? row : 0u, tok = row_ld / a.G;
+        const int32_t qp = a.q_pos[tok];
+        const uint32_t t_begin = seg * KVM_PF_LIST;
+        const uint32_t n_seg_t = a.n_tiles - t_begin < KVM_PF_LIST ? a.n_tiles - t_begin : KVM_PF_LIST;
+        // a wave looks at 4 tiles at a time, 4 cells a lane (PF_STAGED: a lane at one tile's summary)
+        constexpr uint32_t NL = SRC == PF_STAGED ? 2 : 18, TPL = SRC == PF_STAGED ? 64 : 4, TPB = NL * 8 * TPL;
+        const uint32_t t_lane = SRC == PF_STAGED ? (uint32_t)tid : (uint32_t)(4 * w + (l >> 4));
+        kvm_u32x4 cells[NL];
+        auto load_cells = [&](uint32_t t0) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        rows[rt] = r0 + 16 * RT * w + 16 * rt + m;
-        const bool live = rows[rt] < a.n_rows;
-        qpos[rt] = live ? a.q_pos[rows[rt] / a.G] : INT_MIN;
-        if (live) {
-            mn = min(mn, qpos[rt]);
-            mx = max(mx, qpos[rt]);
+            for (uint32_t i = 0; i < NL; ++i) {
+                const uint32_t t = t0 + 8 * TPL * i + t_lane;
+                const uint64_t tile = t_begin + (t < n_seg_t ? t : 0u);
+                cells[i] = SRC == PF_STAGED ? *(const kvm_u32x4 *)(a.info + tile * 4)
+                                            : *(const kvm_u32x4 *)(a.cell_pos + tile * 64 + 4 * (l & 15));
+            }
+        };
+        load_cells(0);
+        // (rows past the last are row 0's: their results are never stored)
+        // Q rows, coalesced into LDS (as operand loads, 32 rows of 32 bytes an
+        // instruction, they took 4 us): unit c of row r at slot c ^ r, so that a
+        // column's reads use every bank.  Q_UC units of 16 bytes of each row a pass.
+        const uint8_t *q_head = (const uint8_t *)a.q;
+        auto dma_q = [&](int pass) {
+            constexpr int N = ROWS * Q_UC / 64 / 8;       // 1 KB copies of a wave
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const uint32_t x = opaque((w * N + i) * 64 + l), r = x / Q_UC, c = (x ^ r) % Q_UC;
+                const uint32_t rr = rt_i * ROWS + r < a.n_rows ? rt_i * ROWS + r : 0u, t = rr / a.G;
+                const uint8_t *src = q_head + (((uint64_t)t * a.n_head + h * a.G + (rr - t * a.G)) * Q_UNITS + pass * Q_UC + c) * 16;
+                uint32_t m0_saved;
+                asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                             : "=&s"(m0_saved) : "v"(src), "s"(lds_mem + Q_OFS + (w * N + i) * 1024u) : "memory");
+            }
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        dma_q(0);
+
+        // ---- a cell is visible to the lane's row iff (unsigned)position < qlim
+        const uint32_t qlim = live_row && qp >= 0 ? (uint32_t)qp + 1u : 0u;
+        const uint32_t mn = kvm_wave_min_u32(live_row ? qlim : 0xffffffffu), mx = ~kvm_wave_min_u32(~qlim);
+        if (l == 0) {
+            s_mm[0][w] = mn;
+            s_mm[1][w] = mx;
         }
-    }
+        KVM_LDS_BARRIER();
+        uint32_t wg_min = s_mm[0][0], wg_max = s_mm[1][0];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        mn = min(mn, __shfl_xor(mn, o, 64));
-        mx = max(mx, __shfl_xor(mx, o, 64));
-    }
-    if (l == 0) {
-        s_mm[0][w] = mn;
-        s_mm[1][w] = mx;
-    }
+        for (int i = 1; i < 8; ++i) {
+            wg_min = min(wg_min, s_mm[0][i]);
+            wg_max = max(wg_max, s_mm[1][i]);
+        }
 
-    // ---- Q rows as f16 B operands: lane (g, m) holds Q[row m][32ks + 8g .. +7]
-    kvm_f16x8 qop[RT][KS];
+        // ---- the piece's tiles: the segment's tiles that some row here can see,
+        // in order, and of these the share [f_lo, f_hi) / P.  s_list holds tile -
+        // t_begin and bit 15: every cell live and visible to every row, so no mask.
+        for (uint32_t t0 = 0;;) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const bool live = rows[rt] < a.n_rows;
-        const uint32_t row = live ? rows[rt] : 0;
-        const uint64_t base = ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            kvm_f16x8 v;
-            if (a.q_bf16) {
-                const kvm_u32x4 raw = *(const kvm_u32x4 *)((const uint16_t *)a.q + base + 32 * ks);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v[2 * j] = (_Float16)__uint_as_float(raw[j] << 16);
-                    v[2 * j + 1] = (_Float16)__uint_as_float(raw[j] & 0xffff0000u);
+            for (uint32_t i = 0; i < NL; ++i) {
+                const uint32_t t = t0 + 8 * TPL * i + t_lane;
+                const kvm_u32x4 c = cells[i];
+                bool some, all;
+                if constexpr (SRC == PF_STAGED) {
+                    some = c[2] != 0 && c[0] < wg_max;
+                    all = c[2] == 64 && c[1] < wg_min;
+                } else {
+                    const uint32_t lo = min(min(c[0], c[1]), min(c[2], c[3])), hi = max(max(c[0], c[1]), max(c[2], c[3]));
+                    some = ((uint32_t)(__builtin_amdgcn_ballot_w64(lo < wg_max) >> (l & 48)) & 0xffffu) != 0;
+                    all = ((uint32_t)(__builtin_amdgcn_ballot_w64(hi < wg_min) >> (l & 48)) & 0xffffu) == 0xffffu;
                 }
-            } else {
-                const kvm_f32x4 x0 = *(const kvm_f32x4 *)((const float *)a.q + base + 32 * ks);
-                const kvm_f32x4 x1 = *(const kvm_f32x4 *)((const float *)a.q + base + 32 * ks + 4);
+                if (t < n_seg_t && (SRC == PF_STAGED || (l & 15) == 0)) s_flag[t] = (uint8_t)(some | all << 1);
+            }
+            t0 += TPB;
+            if (t0 >= n_seg_t) break;
+            load_cells(t0);
+        }
+        KVM_LDS_BARRIER();
+        uint32_t n_t;
+        {
+            const uint32_t n_it = (n_seg_t + 511) / 512;
+            auto flag = [&](uint32_t it) { return 512 * it + tid < n_seg_t ? (uint32_t)s_flag[512 * it + tid] : 0u; };
+            for (uint32_t it = 0; it < n_it; ++it) {
+                const uint64_t bal = __builtin_amdgcn_ballot_w64(flag(it) & 1u);
+                if (l == 0) s_cnt[8 * it + w] = __popcll(bal);
+            }
+            KVM_LDS_BARRIER();
+            // every wave scans the counts of all (at most 16 x 8 of them)
+            const uint32_t c0 = (uint32_t)l < 8 * n_it ? s_cnt[l] : 0u, c1 = (uint32_t)l + 64 < 8 * n_it ? s_cnt[l + 64] : 0u;
+            const uint32_t i0 = kvm_wave_incl_scan(c0), half = __builtin_amdgcn_readlane(i0, 63);
+            const uint32_t i1 = n_it > 8 ? kvm_wave_incl_scan(c1) : 0u, total = half + (n_it > 8 ? __builtin_amdgcn_readlane(i1, 63) : 0u);
+            const uint32_t lo = total * f_lo / a.P, hi = total * f_hi / a.P;     // P <= 2^16
+            n_t = hi - lo;
+            for (uint32_t it = 0; it < n_it; ++it) {
+                const uint32_t f = flag(it), x = 8 * it + w;
+                const uint64_t bal = __builtin_amdgcn_ballot_w64(f & 1u);
+                const uint32_t base = x < 64 ? __builtin_amdgcn_readlane(i0 - c0, x) : half + __builtin_amdgcn_readlane(i1 - c1, x - 64);
+                const uint32_t rank = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                if ((f & 1u) && rank >= lo && rank < hi) s_list[rank - lo] = (uint16_t)((512 * it + tid) | (f >> 1) << 15);
+            }
+            KVM_LDS_BARRIER();
+        }
+        auto entry = [&](uint32_t k) { return (uint32_t)s_list[k < n_t ? k : n_t - 1]; };
+
+        // Q rows as f16 B operands: lane (g2, m2) holds Q[row m2][16ks + 8 g2 .. +7]
+        kvm_f16x8 qop[KS];
+        auto take_q = [&](int pass) {
+            const uint32_t le = opaque(l), r = 32 * rg + (le & 31u), sw = r % Q_UC;
+            const uint8_t *qr = s_mem + Q_OFS + r * (Q_UC * 16);
+            constexpr int KP = KS * Q_UC / Q_UNITS;       // k-steps of a pass
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v[j] = (_Float16)x0[j];
-                    v[4 + j] = (_Float16)x1[j];
+            for (int i = 0; i < KP; ++i) {
+                const int ks = pass * KP + i;
+                kvm_u32x4 x[BF16 ? 1 : 2];
+#pragma unroll
+                for (int j = 0; j < (BF16 ? 1 : 2); ++j)
+                    x[j] = *(const kvm_u32x4 *)(qr + ((((BF16 ? 1 : 2) * (2 * i + (le >> 5)) + j) ^ sw) * 16));
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t y = x[BF16 ? 0 : j >> 2][BF16 ? j >> 1 : j & 3];
+                    const float v = __uint_as_float(!BF16 ? y : j & 1 ? y & 0xffff0000u : y << 16);
+                    qop[ks][j] = (_Float16)v;
                 }
             }
-            if (!live) v = kvm_f16x8{};
-            qop[rt][ks] = v;
-        }
-    }
-    __syncthreads();
-    int32_t wg_min = s_mm[0][0], wg_max = s_mm[1][0];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) {
-        wg_min = min(wg_min, s_mm[0][i]);
-        wg_max = max(wg_max, s_mm[1][i]);
-    }
-
-    // ---- this split's tiles.  A list in LDS holds the tiles some row here can
-    // see (tile - t_begin, bit 15 = every cell live and visible to every row,
-    // so no mask), built once by a block-wide scan.
-    const uint32_t tps = (a.n_tiles + a.n_splits - 1) / a.n_splits;
-    const uint32_t t_begin = split * tps < a.n_tiles ? split * tps : a.n_tiles;
-    const uint32_t t_end = t_begin + tps < a.n_tiles ? t_begin + tps : a.n_tiles;
-    uint32_t n_live = 0;
-    for (uint32_t t0 = t_begin; t0 < t_end; t0 += 64 * NW) {
-        const uint32_t t = t0 + tid;
-        uint32_t live = 0, full = 0;
-        if (t < t_end) {
-            const kvm_i32x4 f = *(const kvm_i32x4 *)(a.info + (uint64_t)t * 4);
-            live = f[2] != 0 && f[0] <= wg_max;
-            full = f[2] == 64 && f[1] <= wg_min;
-        }
-        const uint32_t incl = kvm_wave_incl_scan(live);
-        if (l == 63) s_wsum[w] = incl;
-        __syncthreads();
-        uint32_t before = n_live, total = 0;
-#pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            before += i < w ? s_wsum[i] : 0u;
-            total += s_wsum[i];
-        }
-        if (live) s_list[before + incl - 1] = (uint16_t)((t - t_begin) | (full << 15));
-        n_live += total;
-        __syncthreads();
-    }
-
-    // Tile copies go global -> LDS directly (global_load_lds_dwordx4: lane l
-    // writes 16 bytes at M0 + offset + 16 l), issued from asm so the compiler
-    // adds no wait for them; the loop waits for them itself before each
-    // barrier.  The asm restores M0, which the compiler reserves.  Wave w copies
-    // bytes [CW w, CW (w+1)) of the tile's K and of its V: CW / 1 KB copies per
-    // part under one M0 value, the immediate offset moving the global and the
-    // LDS address alike.  Wave 0 also copies the tile's 64 cell positions.
-    constexpr uint32_t CW = TILE_H * 2 / NW;             // bytes of one K (or V) tile per wave
-    static_assert(CW == 4096 || CW == 2048, "copy layout");
-    const uint32_t lds_kv = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_kv[0][0];
-    const uint32_t lds_cp = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_cp[0][0];
-    const uint32_t loff = 16u * l;                       // this lane's bytes in a 1 KB copy
-    const uint32_t wofs = __builtin_amdgcn_readfirstlane(CW * w);
-    const uint8_t *k_head = (const uint8_t *)(a.kh + (uint64_t)h * a.n_tiles * TILE_H) + wofs;
-    const uint8_t *v_head = (const uint8_t *)(a.vh + (uint64_t)h * a.n_tiles * TILE_H) + wofs;
-    auto dma_tile = [&](uint32_t t, int buf) {
-        t = __builtin_amdgcn_readfirstlane(t);
-        const uint8_t *kb = k_head + (uint64_t)t * (TILE_H * 2);
-        const uint8_t *vb = v_head + (uint64_t)t * (TILE_H * 2);
-        const uint32_t dk = lds_kv + (uint32_t)buf * (2 * TILE_H * 2) + wofs;
-        const uint32_t dv = dk + TILE_H * 2;
-        uint32_t m0_saved;
-        if constexpr (CW == 4096) {
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
-                         "global_load_lds_dwordx4 %1, %4\n\t"
-                         "global_load_lds_dwordx4 %1, %4 offset:1024\n\t"
-                         "global_load_lds_dwordx4 %1, %4 offset:2048\n\t"
-                         "global_load_lds_dwordx4 %1, %4 offset:3072\n\t"
-                         "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                         "global_load_lds_dwordx4 %1, %5\n\t"
-                         "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
-                         "global_load_lds_dwordx4 %1, %5 offset:2048\n\t"
-                         "global_load_lds_dwordx4 %1, %5 offset:3072\n\t"
-                         "s_mov_b32 m0, %0"
-                         : "=&s"(m0_saved) : "v"(loff), "s"(dk), "s"(dv), "s"(kb), "s"(vb) : "memory");
-        } else {
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
-                         "global_load_lds_dwordx4 %1, %4\n\t"
-                         "global_load_lds_dwordx4 %1, %4 offset:1024\n\t"
-                         "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                         "global_load_lds_dwordx4 %1, %5\n\t"
-                         "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
-                         "s_mov_b32 m0, %0"
-                         : "=&s"(m0_saved) : "v"(loff), "s"(dk), "s"(dv), "s"(kb), "s"(vb) : "memory");
-        }
-        if (w == 0) {
-            const int32_t *src = a.cell_pos + (uint64_t)t * 64;
-            const uint32_t dst = lds_cp + (uint32_t)buf * 256;
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %3\n\ts_mov_b32 m0, %0"
-                         : "=&s"(m0_saved) : "v"(4u * l), "s"(dst), "s"(src) : "memory");
-        }
-    };
-
-    kvm_f32x4 O[RT][DT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) O[rt][dt] = kvm_f32x4{0.f, 0.f, 0.f, 0.f};
-    float ms[RT], lp[RT];                   // running max of each row (times c), lane's share of its sum
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        ms[rt] = -INFINITY;
-        lp[rt] = 0.0f;
-    }
-    const float c = a.c;
-
-    // list entries k and k+1 are in registers at the top of tile k; entry k+2
-    // is read during tile k
-    uint32_t e_cur = n_live > 0 ? s_list[0] : 0u, e_nxt = n_live > 1 ? s_list[1] : e_cur;
-    if (n_live > 0) dma_tile(t_begin + (e_cur & 0x7fffu), 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    for (uint32_t k = 0; k < n_live; ++k) {
-        const int b = k & 1;
-        const uint32_t e = __builtin_amdgcn_readfirstlane(e_cur);
-        const uint32_t en = __builtin_amdgcn_readfirstlane(e_nxt);
-        e_cur = en;
-        e_nxt = s_list[k + 2 < n_live ? k + 2 : n_live - 1];
-        dma_tile(t_begin + (en & 0x7fffu), b ^ 1);        // next tile, in flight during this one
-        const bool masked = (e >> 15) == 0;
-        const _Float16 *sk = s_kv[b];
-        const _Float16 *sv = s_kv[b] + TILE_H;
-
-        // S^T = K Q^T: sub tile s holds keys 16s + 4g + r of row m
-        kvm_f32x4 S[4][RT];
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) S[s][rt] = kvm_f32x4{0.f, 0.f, 0.f, 0.f};
-        // K operands run KR-1 k-steps ahead of their MFMAs (a register ring)
-        kvm_f16x8 kr[KR][4];
-#pragma unroll
-        for (int p = 0; p < KR - 1; ++p)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) kr[p][s] = *(const kvm_f16x8 *)(sk + ((s * KS + p) * 64 + l) * 8);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if (ks + KR - 1 < KS) {
-#pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    kr[(ks + KR - 1) % KR][s] = *(const kvm_f16x8 *)(sk + ((s * KS + ks + KR - 1) * 64 + l) * 8);
+        };
+        // (the caller has waited for its own copies)
+        auto load_q = [&]() {
+            KVM_LDS_BARRIER();
+            take_q(0);
+            if constexpr (Q_UNITS != Q_UC) {
+                KVM_LDS_BARRIER();
+                dma_q(1);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                KVM_LDS_BARRIER();
+                take_q(1);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            KVM_LDS_BARRIER();
+        };
+        kvm_f32x16 O[DT];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
-                    S[s][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kr[ks % KR][s], qop[rt][ks], S[s][rt], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // the first V operands, in flight during the softmax
-        kvm_f16x8 vr[VR];
+            for (int r = 0; r < 16; ++r) O[dt][r] = 0.0f;
+        float ms = -INFINITY, lp = 0.0f;        // running max of the row (times c), lane's share of its sum
+        const float c = a.c;
+
+        // operand addresses of a lane: K row m2 is key m2 with bits 2 and 3 swapped
+        auto k_lane = [&](uint32_t x) {
+            const uint32_t key = (x & 0x13) | (x & 4) << 1 | (x & 8) >> 1;
+            return ((key >> 4) * NB * 64 + 16 * (x >> 5) + (key & 15)) * 16 + (KW == 2 ? kg * 2 * NB * 1024 : 0);
+        };
+        auto v_lane = [&](uint32_t x) { return ((x >> 4 & 1) * 64 + 16 * (x >> 5) + (x & 15)) * 16 + (KW == 2 ? kg * (TILE_B / 2) : 0); };
+
+        // S^T of one 32-key sub tile: K operand ks at sk + ..., KR - 1 ahead
+        auto scores = [&](const uint8_t *sk, auto &&between) {
+            kvm_f32x16 S;
 #pragma unroll
-        for (int i = 0; i < VR - 1; ++i) vr[i] = *(const kvm_f16x8 *)(sv + (((i % DT) * 2 + i / DT) * 64 + l) * 8);
-        if (masked) {
-            asm volatile("" ::: "memory");                // keep the mask on this (rare) path
+            for (int r = 0; r < 16; ++r) S[r] = 0.0f;
+            kvm_f16x8 kr[KR];
+            auto ld = [&](int ks) { return *(const kvm_f16x8 *)(sk + (ks >> 1) * 1024 + (ks & 1) * 512); };
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const kvm_i32x4 cp = *(const kvm_i32x4 *)&s_cp[b][16 * s + 4 * g];
+            for (int i = 0; i < KR - 1; ++i) kr[i] = ld(i);
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
+            for (int ks = 0; ks < KS; ++ks) {
+                if (ks + KR - 1 < KS) kr[(ks + KR - 1) % KR] = ld(ks + KR - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kr[ks % KR], qop[ks], S, 0, 0, 0);
+                between(ks);
+                PF_PIN(S);
+            }
+            return S;
+        };
+        // mask, running maximum; returns the maximum that P is formed against
+        auto settle = [&](kvm_f32x16 &S, bool masked, const int32_t *cp) {
+            if (masked) {
+                asm volatile("" ::: "memory");            // keep the mask on this (rare) path
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const kvm_u32x4 x = *(const kvm_u32x4 *)(cp + 16 * (i >> 1) + 8 * (opaque(l) >> 5) + 4 * (i & 1));
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        if (!(cp[r] >= 0 && cp[r] <= qpos[rt])) S[s][rt][r] = -INFINITY;
-            }
-        }
-        // online softmax per row
-        float tmax[RT];
-        bool up[RT], any = false;
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            float x = S[0][rt][0];
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) x = fmaxf(x, S[s][rt][r]);
-            x = kvm_max_xor32(kvm_max_xor16(x));
-            tmax[rt] = x;
-            up[rt] = fmaf(x, c, -ms[rt]) > KVM_PF_LAZY;   // false for a row with nothing visible yet
-            any = any || up[rt];
-        }
-        if (__builtin_amdgcn_ballot_w64(any) != 0) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const float mnew = up[rt] ? tmax[rt] * c : ms[rt];
-                const float alpha = up[rt] ? __builtin_amdgcn_exp2f(ms[rt] - mnew) : 1.0f;
-                ms[rt] = mnew;
-                lp[rt] *= alpha;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) O[rt][dt] *= alpha;
-            }
-        }
-        kvm_f16x8 pB[RT][2];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const float msr = ms[rt] == -INFINITY ? 0.0f : ms[rt];
-            float sum = 0.0f;
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    // the row sum takes p before its rounding to the fp16 operand:
-                    // within 2^-11 of it per element
-                    const float p = __builtin_amdgcn_exp2f(fmaf(S[s][rt][r], c, -msr));
-                    pB[rt][s >> 1][4 * (s & 1) + r] = (_Float16)p;
-                    sum += p;
+                        if (!(x[r] < qlim)) S[4 * i + r] = -INFINITY;
                 }
-            lp[rt] += sum;
-        }
-        // O^T += V^T P^T
-        // operand i = (kk, dt) = (i / DT, i % DT); the ring stays VR-1 ahead
+            }
+            float x = S[0];
 #pragma unroll
-        for (int i = 0; i < 2 * DT; ++i) {
-            const int kk = i / DT, dt = i % DT, n = i + VR - 1;
-            if (n < 2 * DT) vr[n % VR] = *(const kvm_f16x8 *)(sv + (((n % DT) * 2 + n / DT) * 64 + l) * 8);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int r = 1; r < 16; ++r) x = fmaxf(x, S[r]);
+            x = kvm_max_xor32(x);
+            const bool up = fmaf(x, c, -ms) > KVM_PF_LAZY;   // false for a row with nothing visible yet
+            if (__builtin_amdgcn_ballot_w64(up) != 0) {
+                const float mnew = up ? x * c : ms;
+                const float alpha = up ? __builtin_amdgcn_exp2f(ms - mnew) : 1.0f;
+                ms = mnew;
+                lp *= alpha;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-                O[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vr[i % VR], pB[rt][kk], O[rt][dt], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's copies
-        __syncthreads();
-    }
+                for (int dt = 0; dt < DT; ++dt) O[dt] *= alpha;
+            }
+            return ms == -INFINITY ? 0.0f : ms;
+        };
+        // O^T += V^T P^T: operand i = (key half i / DT, dim tile i % DT); the
+        // second half's probabilities are formed between the first half's MFMAs
+        auto ldv = [&](const uint8_t *sv, int i) { return *(const kvm_f16x8 *)(sv + (i % DT) * 2048 + (i / DT) * 512); };
+        auto accumulate = [&](const uint8_t *sv, const kvm_f32x16 &S, float msr, kvm_f16x8 (&vr)[VR], auto &&between) {
+            kvm_f16x8 pb[2];
+            float sum = 0.0f;
+            auto prob = [&](int r) {
+                // the row sum takes p before its rounding to the fp16 operand:
+                // within 2^-11 of it per element
+                const float x = __builtin_amdgcn_exp2f(fmaf(S[r], c, -msr));
+                pb[r >> 3][r & 7] = (_Float16)x;
+                sum += x;
+            };
+#pragma unroll
+            for (int r = 0; r < 8; ++r) prob(r);
+#pragma unroll
+            for (int i = 0; i < 2 * DT; ++i) {
+                if (i + VR - 1 < 2 * DT) vr[(i + VR - 1) % VR] = ldv(sv, i + VR - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                O[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vr[i % VR], pb[i / DT], O[i % DT], 0, 0, 0);
+                if (i < DT) {
+#pragma unroll
+                    for (int j = 0; j < 8 / DT; ++j) prob(8 + i * (8 / DT) + j);
+                }
+                between(i);
+                PF_PIN(O[i % DT]);
+            }
+            lp += sum;
+        };
+        auto nothing = [](int) {};
 
-    // ---- results
+        // Copies go global -> LDS directly (global_load_lds_dwordx4: lane l writes
+        // 16 bytes at M0 + offset + 16 l), issued from asm so the compiler adds no
+        // wait for them; the loops wait for them themselves before each barrier.
+        // The asm restores M0, which the compiler reserves.
+        const uint32_t lds_cp = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_cp[0][0];
+        auto dma_cp = [&](uint32_t t, uint32_t buf) {
+            const int32_t *src = a.cell_pos + (uint64_t)t * 64;
+            uint32_t m0_saved;
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %3\n\ts_mov_b32 m0, %0"
+                         : "=&s"(m0_saved) : "v"(4u * opaque(l)), "s"(lds_cp + buf * 256u), "s"(src) : "memory");
+        };
+
+        if (n_t != 0) {
+            if constexpr (SRC != PF_QUANT) {
+                // Wave w copies bytes [CW w, CW (w+1)) of the tile's K and of its V in
+                // CW / 1 KB copies under one M0 value (the immediate offset moves the
+                // global and the LDS address alike).  A window's f16 V tile holds the
+                // two key halves of a dim side by side, so its copies read every
+                // second unit of a dim tile.  Wave 0 also copies the cell positions.
+                constexpr uint32_t CW = TILE_B / 8;
+                static_assert(CW == 4096 || CW == 2048, "copy layout");
+                const uint32_t wofs = __builtin_amdgcn_readfirstlane(CW * w), loff = 16u * l;
+                const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * TILE_B + wofs;
+                const uint8_t *v_head = a.v + (uint64_t)h * a.n_tiles * TILE_B +
+                                        (SRC == PF_F16 ? (w >> 2) * 16u + (w & 3) * 2u * CW : wofs);
+                const uint32_t voff = SRC == PF_F16 ? 32u * l : loff;
+                constexpr uint32_t VS = SRC == PF_F16 ? 1024u : 0u;     // global bytes a V copy moves beyond the LDS's
+                auto dma_tile = [&](uint32_t t, uint32_t buf) {
+                    const uint8_t *kb = k_head + (uint64_t)t * TILE_B, *vb = v_head + (uint64_t)t * TILE_B;
+                    const uint32_t dk = lds_mem + buf * (2 * TILE_B) + wofs, dv = dk + TILE_B;
+                    uint32_t m0_saved;
+                    if constexpr (CW == 4096) {
+                        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+                                     "global_load_lds_dwordx4 %1, %5\n\t"
+                                     "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
+                                     "global_load_lds_dwordx4 %1, %5 offset:2048\n\t"
+                                     "global_load_lds_dwordx4 %1, %5 offset:3072\n\t"
+                                     "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
+                                     "global_load_lds_dwordx4 %2, %6\n\t"
+                                     "global_load_lds_dwordx4 %2, %7 offset:1024\n\t"
+                                     "global_load_lds_dwordx4 %2, %8 offset:2048\n\t"
+                                     "global_load_lds_dwordx4 %2, %9 offset:3072\n\t"
+                                     "s_mov_b32 m0, %0"
+                                     : "=&s"(m0_saved) : "v"(loff), "v"(voff), "s"(dk), "s"(dv), "s"(kb), "s"(vb),
+                                       "s"(vb + VS), "s"(vb + 2 * VS), "s"(vb + 3 * VS) : "memory");
+                    } else {
+                        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+                                     "global_load_lds_dwordx4 %1, %5\n\t"
+                                     "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
+                                     "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
+                                     "global_load_lds_dwordx4 %2, %6\n\t"
+                                     "global_load_lds_dwordx4 %2, %7 offset:1024\n\t"
+                                     "s_mov_b32 m0, %0"
+                                     : "=&s"(m0_saved) : "v"(loff), "v"(voff), "s"(dk), "s"(dv), "s"(kb), "s"(vb),
+                                       "s"(vb + VS) : "memory");
+                    }
+                    if (w == 0) dma_cp(t, buf);
+                };
+                // list entries k and k+1 are in registers at the top of tile k; entry
+                // k+2 is read during tile k
+                uint32_t e_cur = entry(0), e_nxt = entry(1);
+                const uint32_t t_0 = t_begin + (__builtin_amdgcn_readfirstlane(e_cur) & 0x7fffu);
+                if constexpr (Q_EARLY) dma_tile(t_0, 0);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                load_q();
+                if constexpr (!Q_EARLY) {
+                    dma_tile(t_0, 0);
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    KVM_LDS_BARRIER();
+                }
+                const uint32_t k_ofs = k_lane(l), v_ofs = v_lane(l);
+                for (uint32_t k = 0; k < n_t; ++k) {
+                    const uint32_t b = k & 1u;
+                    const uint32_t e = __builtin_amdgcn_readfirstlane(e_cur), en = __builtin_amdgcn_readfirstlane(e_nxt);
+                    e_cur = en;
+                    e_nxt = entry(k + 2);
+                    dma_tile(t_begin + (en & 0x7fffu), b ^ 1u);       // next tile, in flight during this one
+                    const bool masked = (e >> 15) == 0;
+                    const uint8_t *sk = s_mem + b * (2 * TILE_B) + k_ofs, *sv = s_mem + b * (2 * TILE_B) + TILE_B + v_ofs;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        float lr = lp[rt];
-        lr = kvm_add_xor32(kvm_add_xor16(lr));
-        const uint32_t row = rows[rt];
-        if (row >= a.n_rows) continue;
-        if (a.n_splits == 1) {
-            const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
-            float *o = a.out + ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + 4 * g;
+                    for (int sub = 0; sub < 2 / KW; ++sub) {
+                        kvm_f32x16 S = scores(sk + sub * 2 * NB * 1024, nothing);
+                        kvm_f16x8 vr[VR];
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) *(kvm_f32x4 *)(o + 16 * dt) = O[rt][dt] * inv;
-        } else {
-            const uint64_t pr = ((uint64_t)split * a.H + h) * a.rows_pad + row;
-            float *o = a.ws_o + pr * D + 4 * g;
+                        for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv + sub * (TILE_B / 2), i);
+                        const float msr = settle(S, masked, &s_cp[b][32 * (KW == 2 ? kg : sub)]);
+                        accumulate(sv + sub * (TILE_B / 2), S, msr, vr, nothing);
+                    }
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's copies
+                    __syncthreads();
+                }
+            } else {
+                // One f16 K buffer, one f16 V buffer and two buffers of quantised
+                // tiles.  Tile k in two phases, a barrier after each: scores and
+                // softmax, with V of tile k converted between the MFMAs; P V, with K of
+                // tile k + 1 converted between them.  The copies run two tiles ahead.
+                uint8_t *const s_k = s_mem, *const s_v = s_mem + TILE_B, *const s_kr = s_mem + 2 * TILE_B,
+                        *const s_vr = s_kr + 2 * KRAW_L;
+                const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * KRAW, *v_head = a.v + (uint64_t)h * a.n_tiles * VRAW;
+                auto dma_raw = [&](const uint8_t *src, uint32_t bytes, uint32_t dst, int n_kb) {
+                    for (int i = w; i < n_kb; i += 8) {
+                        const uint32_t o = 1024u * i + 16u * opaque(l);
+                        uint32_t m0_saved;
+                        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                                     "global_load_lds_dwordx4 %1, %3\n\ts_mov_b32 m0, %0"
+                                     : "=&s"(m0_saved) : "v"(o < bytes ? o : bytes - 16u), "s"(dst + 1024u * i), "s"(src) : "memory");
+                    }
+                };
+                auto dma_k = [&](uint32_t e, uint32_t k) {
+                    const uint32_t t = t_begin + (e & 0x7fffu);
+                    dma_raw(k_head + (uint64_t)t * KRAW, KRAW, lds_mem + 2 * TILE_B + (k & 1u) * KRAW_L, KRAW_L / 1024);
+                    if (w == 7) dma_cp(t, k & 3u);
+                };
+                auto dma_v = [&](uint32_t e, uint32_t k) {
+                    const uint32_t t = t_begin + (e & 0x7fffu);
+                    dma_raw(v_head + (uint64_t)t * VRAW, VRAW, lds_mem + 2 * TILE_B + 2 * KRAW_L + (k & 1u) * VRAW_L, VRAW_L / 1024);
+                };
+                // this wave's copies of one K and one V tile: all but the last so many
+                // are waited for before a phase ends
+                const int n_kv = (int)(KRAW_L / 1024 + 7 - w) / 8 + (w == 7) + (int)(VRAW_L / 1024 + 7 - w) / 8;
+                auto wait_copies = [&]() {
+                    if (n_kv <= 1) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
+                    else if (n_kv == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+                    else if (n_kv == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+                    else if (n_kv == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                    else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+                };
+                // K: thread (w, l) converts the quants of (sub, block pair) CK w .., lane
+                // l, one unit a chunk; V: dim tiles CV w .., both key halves
+                constexpr int CK = NB / 4, CV = D / 128;
+                kvm_u32x4 ck;
+                uint32_t cd[2];
+                auto k_read = [&](const uint8_t *raw, int i) {
+                    const uint32_t ln = opaque(l), sp = CK * w + i, s = sp / (NB / 2), pr = sp % (NB / 2), m = ln & 15;
+                    ck = *(const kvm_u32x4 *)(raw + (sp * 64 + ln) * 16);
+                    cd[0] = *(const uint16_t *)(raw + kvm_kd_off(D, 16 * s + m, 2 * pr));
+                    cd[1] = *(const uint16_t *)(raw + kvm_kd_off(D, 16 * s + m, 2 * pr + 1));
+                };
+                auto k_write = [&](int i, int j) {
+                    const uint32_t sp = CK * w + i, s = sp / (NB / 2), pr = sp % (NB / 2);
+                    *(kvm_f16x8 *)(s_k + ((s * NB + 2 * pr + j) * 64 + opaque(l)) * 16) = pf_q8(ck[2 * j], ck[2 * j + 1], cd[j]);
+                };
+                kvm_u32x2 cv[CV];
+                kvm_u32x4 cs;
+                auto v_read = [&](const uint8_t *raw, int ks) {
+                    const uint32_t ln = opaque(l);
+                    if (ks == 0) {
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) *(kvm_f32x4 *)(o + 16 * dt) = O[rt][dt];
-            if (g == 0) {
-                a.ws_ml[pr * 2] = ms[rt];
-                a.ws_ml[pr * 2 + 1] = lr;
+                        for (int i = 0; i < CV; ++i) cv[i] = *(const kvm_u32x2 *)(raw + ((CV * w + i) * 64 + ln) * 8);
+                    }
+                    cs = *(const kvm_u32x4 *)(raw + 32 * D + (((CV * w) >> 1) * 8 + ks * 4 + (ln >> 4)) * 16);
+                };
+                auto v_write = [&](int i, int ks) {
+                    *(kvm_f16x8 *)(s_v + ks * (TILE_B / 2) + ((CV * w + i) * 64 + opaque(l)) * 16) = pf_q4(cv[i][ks], cs);
+                };
+                // steps of a conversion between the MFMAs (16 at D 256, 8 at 128)
+                auto conv_v = [&](const uint8_t *raw, int i) {
+                    constexpr int Q = KS / (2 * CV + 1);          // MFMAs between two writes
+                    if (i == 0) v_read(raw, 0);
+#pragma unroll
+                    for (int n = 0; n < 2 * CV; ++n)
+                        if (i == Q * (n + 1)) v_write(n % CV, n / CV);
+                    if (i == Q * CV) v_read(raw, 1);
+                };
+                auto conv_k = [&](const uint8_t *raw, int i) {
+                    constexpr int Q = KS / CK;                    // MFMAs of a chunk
+                    const int n = i / Q, o = i % Q;
+                    if (o == 0) k_read(raw, n);
+                    if (o == Q / 2) k_write(n, 0);
+                    if (o == Q / 2 + 2) k_write(n, 1);
+                };
+
+                if constexpr (!Q_EARLY) {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    load_q();
+                }
+                // list entries of tiles k .. k + 2, and k + 3's on its way
+                auto ent = [&](uint32_t k) { return (uint32_t)__builtin_amdgcn_readfirstlane(entry(k)); };
+                uint32_t e0 = ent(0), e1 = ent(1), e2 = ent(2), e_far = entry(3);
+                dma_k(e0, 0);
+                dma_v(e0, 0);
+                dma_k(e1, 1);
+                dma_v(e1, 1);
+                wait_copies();                            // Q's too: they are older
+                if constexpr (Q_EARLY) load_q();
+                else KVM_LDS_BARRIER();
+#pragma unroll
+                for (int i = 0; i < CK; ++i) {
+                    k_read(s_kr, i);
+                    k_write(i, 0);
+                    k_write(i, 1);
+                }
+                KVM_LDS_BARRIER();
+                for (uint32_t k = 0; k < n_t; ++k) {
+                    const uint32_t b = k & 1u;
+                    const bool masked = (e0 >> 15) == 0;
+                    dma_k(e2, k + 2);
+                    const uint8_t *vraw = s_vr + b * VRAW_L, *kraw = s_kr + (b ^ 1u) * KRAW_L;
+                    kvm_f32x16 S = scores(s_k + k_lane(opaque(l)), [&](int i) { conv_v(vraw, i); });
+                    const float msr = settle(S, masked, &s_cp[k & 3u][32 * kg]);
+                    wait_copies();
+                    KVM_LDS_BARRIER();
+                    dma_v(e2, k + 2);
+                    const uint8_t *sv = s_v + v_lane(opaque(l));
+                    kvm_f16x8 vr[VR];
+#pragma unroll
+                    for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv, i);
+                    accumulate(sv, S, msr, vr, [&](int i) { conv_k(kraw, i); });
+                    e0 = e1;
+                    e1 = e2;
+                    e2 = __builtin_amdgcn_readfirstlane(e_far);
+                    e_far = entry(k + 4);
+                    wait_copies();
+                    KVM_LDS_BARRIER();
+                }
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the copies past the last tile
+                __syncthreads();
             }
         }
+
+        if (n_t == 0) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // Q's copies
+            KVM_LDS_BARRIER();
+        }
+
+        // ---- results: O's quads i0 .. i0 + N - 1 (quad i: dims 8 i + 4 g2 .. + 3 of the lane's row)
+        float lr = kvm_add_xor32(lp);
+        auto quad = [&](int i) {
+            return kvm_f32x4{O[i >> 2][4 * (i & 3)], O[i >> 2][4 * (i & 3) + 1], O[i >> 2][4 * (i & 3) + 2], O[i >> 2][4 * (i & 3) + 3]};
+        };
+        // (the lane and its row are formed again here: kept through the loop they
+        // take registers that O needs)
+        const uint32_t le = opaque(l), me = le & 31u, ge = le >> 5, row_e = rt_i * ROWS + 32 * rg + me;
+        auto finish = [&](auto i0_, auto n_, float w0, const float *other, float w1, bool ml) {
+            constexpr int I0 = decltype(i0_)::value, N = decltype(n_)::value;
+            const uint64_t slot = 2 * (uint64_t)p + (u != u_first);
+            const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
+            float *o = whole ? a.out + ((uint64_t)(row_e / a.G) * a.n_head + h * a.G + row_e % a.G) * D + 4 * ge
+                             : a.ws_o + (slot * ROWS + 32 * rg) * D + 4 * le;
+            const uint32_t os = whole ? 8u : 256u;
+            if (whole ? row_e < a.n_rows : rt_i * ROWS + 32 * rg < a.n_rows) {
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    kvm_f32x4 x = quad(I0 + i);
+                    if constexpr (KW == 2) x = x * w0 + *(const kvm_f32x4 *)(other + 256 * i) * w1;
+                    if (whole) x *= inv;
+                    *(kvm_f32x4 *)(o + os * (I0 + i)) = x;
+                }
+                if (ml && !whole && ge == 0) {
+                    float *o_ml = a.ws_ml + (slot * ROWS + 32 * rg + me) * 2;
+                    o_ml[0] = ms;
+                    o_ml[1] = lr;
+                }
+            }
+        };
+        constexpr std::integral_constant<int, 0> first;
+        if constexpr (KW == 1) {
+            finish(first, std::integral_constant<int, DT * 4>{}, 1.0f, nullptr, 0.0f, true);
+        } else {
+            // the key groups of 32 rows merge through LDS: each hands the other one
+            // half of its dims
+            constexpr std::integral_constant<int, DT * 2> half;
+            float *const s_o = (float *)s_mem + 4 * le;
+            auto give = [&](auto i0_) {
+#pragma unroll
+                for (int i = 0; i < DT * 2; ++i) *(kvm_f32x4 *)(s_o + (w * DT * 2 + i) * 256) = quad(decltype(i0_)::value + i);
+            };
+            if (kg == 0) give(half);
+            else give(first);
+            if (ge == 0) {
+                s_ml[w][me][0] = ms;
+                s_ml[w][me][1] = lr;
+            }
+            KVM_LDS_BARRIER();
+            const float m1 = s_ml[w ^ 1][me][0], l1 = s_ml[w ^ 1][me][1], M = fmaxf(ms, m1);
+            const float w0 = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
+            const float w1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
+            lr = lr * w0 + l1 * w1;
+            ms = M;
+            const float *other = s_o + (w ^ 1) * DT * 2 * 256;
+            if (kg == 0) finish(first, half, w0, other, w1, true);
+            else finish(half, half, w0, other, w1, false);
+        }
+        if (u != u_last) __syncthreads();       // s_mem, s_mm and s_ml are reused by the next piece
     }
 }
 
-// Merge the key splits of each (kv head, row): one thread per 4 dims.
-template <int D>
+// Merge the pieces of a unit's 32-row group: a lane has 4 dims of a row.  WS waves
+// share the pieces, each with NP pieces' loads in flight, and meet in LDS: what
+// bounds a unit of many pieces is the round trips of its loads (32 pieces of 128
+// rows x 256 dims: 8.1 us with one wave, four trips).
+template <int D, int KW, int WS, int NP>
 __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
-    constexpr int TPR = D / 4;                            // threads per row
-    const uint32_t row = blockIdx.x * (256 / TPR) + threadIdx.x / TPR, h = blockIdx.y;
-    if (row >= a.n_rows) return;
-    const uint32_t d4 = (threadIdx.x % TPR) * 4;
-    float M = -INFINITY;
-    for (uint32_t s = 0; s < a.n_splits; ++s)
-        M = fmaxf(M, a.ws_ml[(((uint64_t)s * a.H + h) * a.rows_pad + row) * 2]);
+    constexpr uint32_t RG = 8 / KW, ROWS = 32 * RG, IB = 4 / WS;
+    const uint32_t l = threadIdx.x & 63u, wv = threadIdx.x >> 6, ws = wv % WS, i = blockIdx.x * IB + wv / WS;
+    const uint32_t rg = blockIdx.y, m2 = l & 31u, rt_i = blockIdx.z % a.n_row_tiles, h = blockIdx.z / a.n_row_tiles;
+    const uint32_t row = rt_i * ROWS + 32 * rg + m2;
+    // the unit's pieces: workgroups q0 .. q1 of each of its segments
+    const uint32_t u0 = blockIdx.z * a.n_seg, u1 = u0 + a.n_seg;
+    float M = -INFINITY, L = 0.0f;
     kvm_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    float L = 0.0f;
-    if (M != -INFINITY) {
-        for (uint32_t s = 0; s < a.n_splits; ++s) {
-            const uint64_t pr = ((uint64_t)s * a.H + h) * a.rows_pad + row;
-            const float ms = a.ws_ml[pr * 2];
-            const float wgt = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-            L += a.ws_ml[pr * 2 + 1] * wgt;
-            acc += *(const kvm_f32x4 *)(a.ws_o + pr * D + d4) * wgt;
+    if (rt_i * ROWS + 32 * rg >= a.n_rows) return;
+    for (uint32_t u = u0; u < u1; ++u) {
+        const uint32_t q0 = u * a.P / a.U, q1 = ((u + 1) * a.P - 1) / a.U;
+        if (q0 == q1 && a.n_seg == 1) return;             // whole: the attention wrote it
+        // q0's piece is its last unit's unless it is also its first (u P = q0 U)
+        const uint32_t s0 = 2 * q0 + (q0 * a.U / a.P != u);
+        for (uint32_t q = q0; q <= q1; q += NP * WS) {
+            kvm_f32x4 x[NP];
+            float m[NP], s[NP];
+#pragma unroll
+            for (uint32_t j = 0; j < NP; ++j) {
+                const uint32_t qj = q + WS * j + ws, pj = min(qj, q1);
+                const uint64_t slot = pj == q0 ? s0 : 2 * pj;
+                x[j] = *(const kvm_f32x4 *)(a.ws_o + (slot * ROWS + 32 * rg) * D + 256 * i + 4 * l);
+                const kvm_f32x2 ml = *(const kvm_f32x2 *)(a.ws_ml + (slot * ROWS + 32 * rg + m2) * 2);
+                m[j] = qj <= q1 ? ml[0] : -INFINITY;
+                s[j] = ml[1];
+            }
+            float mb = M;
+#pragma unroll
+            for (uint32_t j = 0; j < NP; ++j) mb = fmaxf(mb, m[j]);
+            const float keep = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - mb);
+            L *= keep;
+            acc *= keep;
+#pragma unroll
+            for (uint32_t j = 0; j < NP; ++j) {
+                const float wgt = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mb);
+                L += m[j] == -INFINITY ? 0.0f : s[j] * wgt;
+                acc += x[j] * wgt;
+            }
+            M = mb;
         }
     }
+    if constexpr (WS > 1) {
+        __shared__ __align__(16) float s_x[WS][64][4];
+        __shared__ float s_m[WS][64], s_l[WS][64];
+        *(kvm_f32x4 *)s_x[ws][l] = acc;
+        s_m[ws][l] = M;
+        s_l[ws][l] = L;
+        __syncthreads();
+        if (ws != 0) return;
+        float mb = M;
+#pragma unroll
+        for (int j = 1; j < WS; ++j) mb = fmaxf(mb, s_m[j][l]);
+        L = 0.0f;
+        acc = kvm_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < WS; ++j) {
+            const float wgt = s_m[j][l] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s_m[j][l] - mb);
+            L += s_l[j][l] * wgt;
+            acc += *(const kvm_f32x4 *)s_x[j][l] * wgt;
+        }
+    }
+    if (row >= a.n_rows) return;
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-    *(kvm_f32x4 *)(a.out + ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + d4) = acc * inv;
+    *(kvm_f32x4 *)(a.out + ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + 8 * i + 4 * (l >> 5)) = acc * inv;
 }
 
-// Key splits: the fewest that keep the whole device busy, for one resident
-// workgroup per CU (the double-buffered K/V tiles take 128 KB of LDS at D 256).
-// KVM_PF_SPLITS in the environment fixes the count.
-static uint32_t pf_choose_splits(uint32_t n_units, uint32_t n_tiles, int n_cu) {
-    if (const char *e = getenv("KVM_PF_SPLITS")) {
-        const int v = atoi(e);
-        if (v >= 1 && v <= KVM_PF_MAX_SPLITS) return (uint32_t)v < n_tiles ? (uint32_t)v : n_tiles;
-    }
-    uint32_t best = 1;
-    double best_t = 1e30;
-    for (uint32_t s = 1; s <= KVM_PF_MAX_SPLITS && s <= n_tiles; ++s) {
-        const uint32_t rounds = (n_units * s + n_cu - 1) / n_cu;
-        const double t = (double)rounds / s + (s > 1 ? 0.02 : 0.0);   // combine pass
-        if (t < best_t - 1e-9) {
-            best_t = t;
-            best = s;
-        }
-    }
-    return best;
+template <int D, int KW, int SRC>
+static void pf_attn(const pf_args &a, hipStream_t stream) {
+    if (a.q_bf16) hipLaunchKernelGGL((k_pf_attn<D, KW, SRC, true>), dim3(a.P), dim3(512), 0, stream, a);
+    else hipLaunchKernelGGL((k_pf_attn<D, KW, SRC, false>), dim3(a.P), dim3(512), 0, stream, a);
+    if (a.n_seg == 1 && a.U % a.P == 0) return;           // every unit whole
+    const dim3 g1(D / 32, 8 / KW, a.n_row_tiles * a.H), g4(D / 8, 8 / KW, a.n_row_tiles * a.H), t(256);
+    // most pieces of a unit (of one of its segments)
+    const uint32_t n = a.P % a.U == 0 ? a.P / a.U : a.P / a.U + 2;
+    if (n <= 2) hipLaunchKernelGGL((k_pf_combine<D, KW, 1, 2>), g1, t, 0, stream, a);
+    else if (n <= 4) hipLaunchKernelGGL((k_pf_combine<D, KW, 1, 4>), g1, t, 0, stream, a);
+    else if (n <= 8) hipLaunchKernelGGL((k_pf_combine<D, KW, 1, 8>), g1, t, 0, stream, a);
+    else if (n <= 16) hipLaunchKernelGGL((k_pf_combine<D, KW, 4, 4>), g4, t, 0, stream, a);
+    else hipLaunchKernelGGL((k_pf_combine<D, KW, 4, 8>), g4, t, 0, stream, a);
 }
 
 template <int D>
-static void pf_launch(const pf_args &a, const pf_stage_args &sa, hipStream_t stream) {
+static void pf_launch(const pf_args &a, const pf_stage_args &sa, int src, int kw, hipStream_t stream) {
+    if (src == PF_QUANT) return pf_attn<D, 2, PF_QUANT>(a, stream);
+    if (src == PF_F16) return kw == 1 ? pf_attn<D, 1, PF_F16>(a, stream) : pf_attn<D, 2, PF_F16>(a, stream);
     hipLaunchKernelGGL(k_pf_stage<D>, dim3(sa.n_tiles, a.H), dim3(256), 0, stream, sa);
-    // 8 waves of 16 rows: two waves per SIMD, so one wave's softmax overlaps
-    // the other's matrix-core work
-    hipLaunchKernelGGL((k_pf_attn<D, 1>), dim3(a.n_row_tiles * a.H * a.n_splits), dim3(512), 0, stream, a);
-    if (a.n_splits > 1)
-        hipLaunchKernelGGL(k_pf_combine<D>, dim3(kvm_cdiv(a.n_rows, 256 / (D / 4)), a.H), dim3(256), 0, stream, a);
+    return kw == 1 ? pf_attn<D, 1, PF_STAGED>(a, stream) : pf_attn<D, 2, PF_STAGED>(a, stream);
+}
+
+// ---- the launch's shape, from measured costs (us; D 256, half of it at D 128)
+// A 64-cell tile of a unit.
+static double pf_tile_us(uint32_t D, int kw, int src) {
+    return (kw == 1 ? 3.3 : src == PF_QUANT ? 2.3 : 1.55) * D / 256;
+}
+
+// Workgroups that U units of n_tiles tiles are dealt to, at most one per CU (LDS).
+// The same number s for every unit, so that none has two pieces (a second piece
+// costs its workgroup another start and end, PF_START us: 100 tokens over 32
+// tiles, 20 units, took 39.9 us on 256 workgroups, 29.3 on 220), unless so many
+// CUs would idle that the second piece is cheaper.  Each piece is written and read
+// once more, `piece` us of all (500 tokens over 16 tiles of 128 dims, 32 units:
+// 30.2 us in 256 pieces, 22.8 in 128).
+#define PF_START 8.0
+static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double t, double piece, uint32_t n_cu, double *cost) {
+    double best = PF_START + t * n_tiles * U / n_cu + piece * (U < n_cu ? n_cu + U : 2.0 * n_cu);
+    uint32_t P = n_cu;
+    for (uint64_t s = 1; s * U <= n_cu && s <= n_tiles; ++s) {
+        const double c = t * kvm_cdiv(n_tiles, s) + (s > 1 ? piece * (s * U) : 0.0);
+        if (c < best) {
+            best = c;
+            P = (uint32_t)(s * U);
+        }
+    }
+    if (cost) *cost = best;
+    return P;
+}
+// A piece's partial output, written and read at the rate that such launches reach.
+static double pf_piece_us(uint32_t D, uint64_t n_rows, uint32_t row_tiles) {
+    return (double)n_rows / row_tiles * D * 8 / 3.2e6;
+}
+
+// Row groups that share a tile, and where a quantised window is converted.
+// - 256 rows a workgroup (kw 1) once a workgroup has PF_LONG tiles of work: half
+//   the LDS writes and tile copies per row (1,500 tokens over 512 tiles of 8
+//   heads, 128 dims: 803 us against 911), but twice the piece bytes (700 tokens
+//   over 144 tiles of 2 heads: 50.4 against 45.8).
+// - converted by the attention (PF_QUANT) while its slower tiles cost less than
+//   the conversion's own launch (37 tokens over 544 tiles: 63 us against 88; 300
+//   over 128: 100 against 92).
+#define PF_LONG 64.0
+struct pf_shape {
+    int src, kw;
+};
+static pf_shape pf_choose(uint32_t D, uint32_t H, uint64_t n_rows, uint32_t n_tiles, uint32_t n_seg, bool quant,
+                          uint32_t n_cu) {
+    const uint64_t U = (uint64_t)kvm_cdiv(n_rows, 128) * H * n_seg;
+    const uint32_t seg_t = kvm_cdiv(n_tiles, n_seg);
+    const int kw = (double)U * seg_t / n_cu >= PF_LONG ? 1 : 2;
+    if (!quant) return {PF_F16, kw};
+    double own, staged;
+    const double piece = pf_piece_us(D, n_rows, kvm_cdiv(n_rows, 128));
+    pf_shares(U, seg_t, pf_tile_us(D, 2, PF_QUANT), piece, n_cu, &own);
+    pf_shares(U, seg_t, pf_tile_us(D, 2, PF_STAGED), piece, n_cu, &staged);
+    staged += 3.0 + 0.0162 * D / 256 * H * n_tiles;
+    return own <= staged ? pf_shape{PF_QUANT, 2} : pf_shape{PF_STAGED, kw};
 }
 
 extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q, int q_type,
@@ -563,54 +919,74 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     const uint32_t D = w->head_dim, H = w->n_head_kv, n_tiles = w->n_cells / KVM_TILE_CELLS;
     const uint64_t n_rows = (uint64_t)n_tokens * G;
     if (n_rows > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
-    int n_cu = 256;
-    if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, st->device) != hipSuccess || n_cu <= 0) n_cu = 256;
+    const bool quant = kvm_k_quant(w->k_type);
+
+    const uint32_t n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
+    const pf_shape sh = pf_choose(D, H, n_rows, n_tiles, n_seg, quant, st->n_cu);
+    int src = sh.src, kw = sh.kw;
 
     pf_args a{};
     a.n_tiles = n_tiles;
+    a.n_seg = n_seg;
     a.H = H;
     a.G = G;
     a.n_head = n_head;
     a.n_rows = (uint32_t)n_rows;
-    a.n_row_tiles = (uint32_t)kvm_cdiv(n_rows, KVM_PF_ROWS);
-    a.rows_pad = a.n_row_tiles * KVM_PF_ROWS;
-    a.n_splits = pf_choose_splits(a.n_row_tiles * H, n_tiles, n_cu);
-    while (kvm_cdiv(n_tiles, a.n_splits) > KVM_PF_LIST) ++a.n_splits;   // a split's tile list fits LDS
+    const uint32_t rows = 256u / kw;
+    a.n_row_tiles = (uint32_t)kvm_cdiv(n_rows, rows);
+    const uint64_t units = (uint64_t)a.n_row_tiles * H * a.n_seg;
+    if (units > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
+    a.U = (uint32_t)units;
+    uint64_t P = pf_shares(units, kvm_cdiv(n_tiles, n_seg), pf_tile_us(D, kw, src),
+                           pf_piece_us(D, n_rows, a.n_row_tiles), st->n_cu, nullptr);
+    // KVM_PF_SPLITS in the environment fixes the pieces per unit
+    if (const char *e = getenv("KVM_PF_SPLITS")) {
+        const int v = atoi(e);
+        if (v >= 1 && v <= 8) P = units * v < 65536u ? units * v : 65536u;
+    }
+    if (P * units > 0xffffffffu) P = 0xffffffffu / units;
+    a.P = (uint32_t)P;
     a.c = scale * 1.4426950408889634f;
     a.q_bf16 = q_type == KVM_TYPE_BF16;
     a.q = q;
     a.q_pos = q_pos;
     a.out = out;
     a.cell_pos = w->cell_pos;
+    a.k = (const uint8_t *)w->k;
+    a.v = (const uint8_t *)w->v;
 
-    // workspace: f16 K and V operand tiles, tile summaries, split partials
-    const size_t kv_bytes = (size_t)H * n_tiles * 64 * D * 2;
-    const size_t info_bytes = (size_t)n_tiles * 16;
-    const size_t part_o = a.n_splits > 1 ? (size_t)a.n_splits * H * a.rows_pad * D * 4 : 0;
-    const size_t part_ml = a.n_splits > 1 ? (size_t)a.n_splits * H * a.rows_pad * 2 * 4 : 0;
+    // workspace: the pieces, and for PF_STAGED the f16 K and V operand tiles and
+    // the tile summaries
     auto up256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t total = 2 * up256(kv_bytes) + up256(info_bytes) + up256(part_o) + up256(part_ml);
-    uint8_t *ws = (uint8_t *)kvm_workspace(st, total);
-    if (!ws) return kvm_fail(st, KVM_ENOMEM, "fa_prefill: workspace of %zu bytes", total);
+    const size_t kv_bytes = src == PF_STAGED ? up256((size_t)H * n_tiles * 64 * D * 2) : 0;
+    const size_t info_bytes = src == PF_STAGED ? up256((size_t)n_tiles * 16) : 0;
+    const bool pieces = a.n_seg > 1 || a.U % a.P != 0;
+    const size_t part_o = pieces ? (size_t)2 * a.P * rows * D * 4 : 0, part_ml = pieces ? (size_t)2 * a.P * rows * 8 : 0;
+    const size_t total = 2 * kv_bytes + info_bytes + part_o + part_ml;
+    uint8_t *ws = nullptr;
+    if (total) {
+        ws = (uint8_t *)kvm_workspace(st, total);
+        if (!ws) return kvm_fail(st, KVM_ENOMEM, "fa_prefill: workspace of %zu bytes", total);
+    }
     pf_stage_args sa{};
-    sa.k = (const uint8_t *)w->k;
-    sa.v = (const uint8_t *)w->v;
-    sa.cell_pos = w->cell_pos;
-    sa.kh = (_Float16 *)ws;
-    sa.vh = (_Float16 *)(ws + up256(kv_bytes));
-    sa.info = (int32_t *)(ws + 2 * up256(kv_bytes));
-    sa.n_tiles = n_tiles;
-    sa.k_q8 = kvm_k_quant(w->k_type);
-    sa.v_q4 = w->v_type == KVM_TYPE_Q4_0;
-    a.kh = sa.kh;
-    a.vh = sa.vh;
-    a.info = sa.info;
-    a.ws_o = (float *)(ws + 2 * up256(kv_bytes) + up256(info_bytes));
-    a.ws_ml = (float *)(ws + 2 * up256(kv_bytes) + up256(info_bytes) + up256(part_o));
+    if (src == PF_STAGED) {
+        sa.k = a.k;
+        sa.v = a.v;
+        sa.cell_pos = w->cell_pos;
+        sa.kh = ws;
+        sa.vh = ws + kv_bytes;
+        sa.info = (int32_t *)(ws + 2 * kv_bytes);
+        sa.n_tiles = n_tiles;
+        a.k = sa.kh;
+        a.v = sa.vh;
+        a.info = sa.info;
+    }
+    a.ws_o = (float *)(ws + 2 * kv_bytes + info_bytes);
+    a.ws_ml = (float *)(ws + 2 * kv_bytes + info_bytes + part_o);
 
     KVM_HIP(st, hipSetDevice(st->device));
-    if (D == 256) pf_launch<256>(a, sa, st->stream);
-    else pf_launch<128>(a, sa, st->stream);
+    if (D == 256) pf_launch<256>(a, sa, src, kw, st->stream);
+    else pf_launch<128>(a, sa, src, kw, st->stream);
     KVM_LAUNCH_CHECK(st, "fa_prefill");
     return KVM_OK;
 }

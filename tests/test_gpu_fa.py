@@ -292,3 +292,37 @@ def test_fa_decode_rejects_wide_batches(kvm_state):
     q = dev(np.zeros((6, 24, 256), np.float32))
     with pytest.raises(L.KvmError):
         api.fa_decode(kvm_state, w, q, dev(np.zeros(6, np.int32)), 24, 0.0625)
+
+
+PREFILL_EDGES = [
+    # n_cells, H, G, D, tokens, kt, vt, live cells (None = all), splits, q dtype
+    (128, 1, 11, 128, 3, L.T_Q8_0, L.T_Q4_0, None, None, "f32"),      # 33 rows over two tiles
+    (256, 2, 11, 256, 3, L.T_Q4_0, L.T_Q4_0, 130, None, "bf16"),      # a tile with two live cells
+    (1024, 1, 3, 256, 43, L.T_F16, L.T_F16, None, None, "f32"),       # 129 rows: a second, nearly empty row tile
+    (2048, 2, 8, 128, 32, L.T_F16, L.T_F16, 1100, None, "bf16"),      # 256 rows, half the window empty
+    (38400, 1, 6, 128, 10, L.T_Q8_0, L.T_Q4_0, 37000, None, "bf16"),  # more tiles than one look at the cells
+    (1024, 4, 6, 256, 200, L.T_Q8_0, L.T_Q4_0, None, None, "f32"),    # window converted ahead
+    (768, 2, 6, 256, 100, L.T_Q8_0, L.T_Q4_0, None, 8, "bf16"),       # more pieces of a unit than its rows see tiles
+    (4096, 8, 4, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16"),  # 256-row units, more of them than CUs
+    (4096, 8, 4, 256, 1100, L.T_F16, L.T_F16, 3900, None, "f32"),     # the same, Q in two passes
+]
+
+
+@pytest.mark.parametrize("case", range(len(PREFILL_EDGES)))
+def test_fa_prefill_edges(kvm_state, case, monkeypatch):
+    """Row and key remainders, every source of the tiles and both unit sizes, at
+    sampled tokens; the first token sees nothing."""
+    n, H, G, D, T, kt, vt, live, splits, qdt = PREFILL_EDGES[case]
+    if splits is not None:
+        monkeypatch.setenv("KVM_PF_SPLITS", str(splits))
+    rng = np.random.default_rng(300 + case)
+    w, kr, vr, cp = _window(kvm_state, rng, n, H, D, kt, vt, live=live)
+    last = n if live is None else live
+    pos = np.arange(last - T, last, dtype=np.int32)
+    pos[0] = -1
+    q = torch.from_numpy(rng.standard_normal((T, H * G, D)).astype(np.float32))
+    q = q.to(torch.bfloat16) if qdt == "bf16" else q
+    out = host(api.fa_prefill(kvm_state, w, q.cuda(), dev(pos), H * G, D ** -0.5))
+    assert np.isfinite(out).all() and np.all(out[0] == 0)
+    toks = np.unique(np.r_[1, 2, T // 2, T - 2, T - 1])
+    _prefill_check(out[toks], q.float().numpy()[toks], kr, vr, cp, pos[toks], H, G, D, kt, vt, D ** -0.5)
