@@ -3,6 +3,7 @@
 #include "kvm_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 // ---------------------------------------------------------------------------
 // geometry
@@ -77,12 +78,6 @@ struct win_geo {
     uint32_t bt, n_slots;
 };
 
-// An import into cell `cell` voids its slot's shadow (the shadow holds only
-// what a stage-in wrote); called by the thread of the cell's first row block.
-__device__ inline void void_shadow(const win_geo &g, uint32_t cell) {
-    if (g.shadow_rows && cell / g.bt < g.n_slots) g.shadow_rows[cell / g.bt] = 0u;
-}
-
 static win_geo geo_of(const kvm_window *w) {
     win_geo g;
     g.k = (uint8_t *)w->k;
@@ -98,135 +93,229 @@ static win_geo geo_of(const kvm_window *w) {
     return g;
 }
 
-// one thread per (cell, head, 32-dim block) of q8_0 K rows
-__global__ void k_import_k_q8(win_geo g, uint32_t cell0, uint32_t n, const uint8_t *rows) {
-    const uint32_t NB = g.D / 32;
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n * g.H * NB) return;
-    const uint32_t b = i % NB, h = (i / NB) % g.H, t = (uint32_t)(i / ((uint64_t)NB * g.H));
-    const uint32_t cell = cell0 + t, tile = cell / 64, c = cell % 64;
-    const uint8_t *src = rows + ((uint64_t)t * g.H + h) * NB * 34 + (uint64_t)b * 34;
-    uint8_t *dst = g.k + ((uint64_t)h * g.n_tiles + tile) * g.ktile;
-#pragma unroll
-    for (uint32_t gg = 0; gg < 4; ++gg) {
-        uint8_t *q = dst + kvm_kq_off(g.D, c, 32 * b + 8 * gg);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) q[j] = src[2 + 8 * gg + j];
-    }
-    uint8_t *sd = dst + kvm_kd_off(g.D, c, b);
-    sd[0] = src[0];
-    sd[1] = src[1];
-    if (b == 0 && h == 0) void_shadow(g, cell);
+// ---- One launch per import: workgroups [0, nb_k) take the K rows, [nb_k, nb_k +
+// nb_v) the V rows, the rest the positions and the touched slots' counts (a
+// separate launch for each cost more in launches than in bytes: 2,048 cells of
+// 4 x 256 values 20.2 us of kernels in four launches, byte by byte; 4 cells 13).
+// A thread reads a block's 16 or 32 quant bytes in 16-byte loads and writes whole
+// 8- or 16-byte pieces of the tile layout.  The rows may have any alignment.
+struct import_args {
+    win_geo g;
+    const uint8_t *k_rows, *v_rows;
+    const int32_t *pos;
+    int32_t *cell_pos;
+    uint32_t *pending;           // null, or the unharvested-row counts
+    uint32_t cell0, n, nb_k, nb_v;
+};
+
+template <typename T>
+__device__ __forceinline__ T load_any(const uint8_t *p) {
+    T x;
+    __builtin_memcpy(&x, p, sizeof(T));
+    return x;
 }
 
-// q4_0 K rows into the q8_0 tile format: quant j = nibble - 8 (low nibbles
-// are dims 0-15 of the block, high nibbles 16-31), the fp16 scale as it is
-__global__ void k_import_k_q4(win_geo g, uint32_t cell0, uint32_t n, const uint8_t *rows) {
-    const uint32_t NB = g.D / 32;
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n * g.H * NB) return;
-    const uint32_t b = i % NB, h = (i / NB) % g.H, t = (uint32_t)(i / ((uint64_t)NB * g.H));
-    const uint32_t cell = cell0 + t, tile = cell / 64, c = cell % 64;
-    const uint8_t *src = rows + ((uint64_t)t * g.H + h) * NB * 18 + (uint64_t)b * 18;
-    uint8_t *dst = g.k + ((uint64_t)h * g.n_tiles + tile) * g.ktile;
+// K: thread (16-cell run, head, block pair | cell of the run, block of the pair):
+// 32 threads write 256 contiguous bytes of each 8-dim group.
+template <int D, int KT>
+__device__ __forceinline__ void import_k(const import_args &a, uint64_t i) {
+    constexpr uint32_t NB = D / 32, BB = KT == KVM_TYPE_Q8_0 ? 34 : 18;
+    const win_geo &g = a.g;
+    if constexpr (KT == KVM_TYPE_F16) {
+        // thread (cell, head, 8 dims): one 16-byte unit
+        const uint32_t u = i % (D / 8), h = (uint32_t)(i / (D / 8)) % g.H;
+        const uint64_t t = i / ((uint64_t)(D / 8) * g.H);
+        if (t >= a.n) return;
+        const uint32_t cell = a.cell0 + (uint32_t)t;
+        uint16_t *dst = (uint16_t *)(g.k + ((uint64_t)h * g.n_tiles + cell / 64) * g.ktile);
+        *(kvm_u32x4 *)(dst + kvm_kh_idx(D, cell % 64, 8 * u)) = load_any<kvm_u32x4>(a.k_rows + ((t * g.H + h) * D + 8 * u) * 2);
+    } else {
+        const uint32_t bb = i & 1u, tm = (i >> 1) & 15u, pr = (i >> 5) % (NB / 2);
+        const uint64_t r = (i >> 5) / (NB / 2);
+        const uint32_t h = (uint32_t)(r % g.H);
+        const uint64_t t = r / g.H * 16 + tm;
+        if (t >= a.n) return;
+        const uint32_t cell = a.cell0 + (uint32_t)t, c = cell % 64, b = 2 * pr + bb;
+        const uint8_t *src = a.k_rows + ((t * g.H + h) * NB + b) * BB;
+        uint8_t *dst = g.k + ((uint64_t)h * g.n_tiles + cell / 64) * g.ktile;
+        const uint16_t d = load_any<uint16_t>(src);
+        kvm_u32x4 q[2];
+        q[0] = load_any<kvm_u32x4>(src + 2);
+        if constexpr (KT == KVM_TYPE_Q8_0) {
+            q[1] = load_any<kvm_u32x4>(src + 18);
+        } else {
+            // the q8_0 tile holds nibble - 8: low nibbles are dims 0-15, high ones 16-31
+            const kvm_u32x4 w = q[0];
 #pragma unroll
-    for (uint32_t gg = 0; gg < 4; ++gg) {
-        uint8_t *q = dst + kvm_kq_off(g.D, c, 32 * b + 8 * gg);
+            for (int j = 0; j < 4; ++j) {
+                q[0][j] = (((w[j] & 0x0f0f0f0fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
+                q[1][j] = ((((w[j] >> 4) & 0x0f0f0f0fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
+            }
+        }
 #pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-            const uint32_t e = 8 * gg + j, nib = e < 16 ? src[2 + e] & 15u : (uint32_t)src[2 + e - 16] >> 4;
-            q[j] = (uint8_t)(int8_t)((int)nib - 8);
+        for (int gg = 0; gg < 4; ++gg)
+            *(kvm_u32x2 *)(dst + kvm_kq_off(D, c, 32 * b + 8 * gg)) = kvm_u32x2{q[gg >> 1][2 * (gg & 1)], q[gg >> 1][2 * (gg & 1) + 1]};
+        *(uint16_t *)(dst + kvm_kd_off(D, c, b)) = d;
+    }
+}
+
+// out[k] = byte k of each x, in order: a 4 x 4 byte transpose
+__device__ __forceinline__ void transpose4(const uint32_t (&x)[4], uint32_t (&out)[4]) {
+    const uint32_t a0 = __builtin_amdgcn_perm(x[1], x[0], 0x05010400u), a1 = __builtin_amdgcn_perm(x[1], x[0], 0x07030602u);
+    const uint32_t b0 = __builtin_amdgcn_perm(x[3], x[2], 0x05010400u), b1 = __builtin_amdgcn_perm(x[3], x[2], 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(b0, a0, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(b1, a1, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+}
+
+// V, q4_0: thread (tile, head, block, 8-cell group gg of both 32-cell halves, four
+// source bytes): 16 cells' bytes become the words of 8 dims.  Words are written by
+// one thread; cells outside the import keep their nibbles.
+template <int D>
+__device__ __forceinline__ void import_v_q4(const import_args &a, uint64_t i) {
+    constexpr uint32_t NB = D / 32;
+    const win_geo &g = a.g;
+    const uint32_t e4 = i & 3u, gg = (i >> 2) & 3u, b = (uint32_t)(i >> 4) % NB;
+    const uint64_t r = (i >> 4) / NB;
+    const uint32_t h = (uint32_t)(r % g.H);
+    const uint64_t tile = a.cell0 / 64 + r / g.H;
+    const uint64_t end = (uint64_t)a.cell0 + a.n;
+    if (tile * 64 >= end) return;
+    uint32_t w[2][8], valid = 0;
+    uint16_t sc[4];
+    auto src = [&](uint64_t cell) {
+        const uint64_t t = cell < a.cell0 ? 0u : cell < end ? cell - a.cell0 : a.n - 1u;
+        return a.v_rows + ((t * g.H + h) * NB + b) * 18;
+    };
+    auto in = [&](uint64_t cell) { return cell >= a.cell0 && cell < end; };
+    // (the scales of four of the cells: half e4 / 2, cells 4 (e4 % 2) ..)
+    const uint64_t c_s = tile * 64 + 32 * (e4 >> 1) + 8 * gg + 4 * (e4 & 1u);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint64_t cell = tile * 64 + 32 * ks + 8 * gg + j;
+            w[ks][j] = load_any<uint32_t>(src(cell) + 2 + 4 * e4);
+            valid |= (uint32_t)in(cell) << (8 * ks + j);
+        }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sc[j] = load_any<uint16_t>(src(c_s + j));
+    uint8_t *vt = g.v + ((uint64_t)h * g.n_tiles + tile) * g.vtile;
+    if (valid) {
+        uint32_t word[2][2][4];                           // [nibble half][ks][dim]
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            uint32_t lo[4], hi[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                lo[j] = (w[ks][j] & 0x0f0f0f0fu) | (w[ks][j + 4] & 0x0f0f0f0fu) << 4;
+                hi[j] = ((w[ks][j] >> 4) & 0x0f0f0f0fu) | (w[ks][j + 4] & 0xf0f0f0f0u);
+            }
+            transpose4(lo, word[0][ks]);
+            transpose4(hi, word[1][ks]);
+        }
+#pragma unroll
+        for (int nh = 0; nh < 2; ++nh) {
+            uint32_t *dst = (uint32_t *)(vt + kvm_vq_word(32 * b + 16 * nh + 4 * e4, gg, 0));   // [dim][ks]
+            if (valid != 0xffffu) {
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    uint32_t m = 0;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (valid >> (8 * ks + j) & 1u) m |= 15u << kvm_vq_nib_shift(j);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) word[nh][ks][k] = (dst[2 * k + ks] & ~m) | (word[nh][ks][k] & m);
+                }
+            }
+            *(kvm_u32x4 *)dst = kvm_u32x4{word[nh][0][0], word[nh][1][0], word[nh][0][1], word[nh][1][1]};
+            *(kvm_u32x4 *)(dst + 4) = kvm_u32x4{word[nh][0][2], word[nh][1][2], word[nh][0][3], word[nh][1][3]};
         }
     }
-    uint8_t *sd = dst + kvm_kd_off(g.D, c, b);
-    sd[0] = src[0];
-    sd[1] = src[1];
-    if (b == 0 && h == 0) void_shadow(g, cell);
-}
-
-// f16 K rows: one thread per (cell, head, dim)
-__global__ void k_import_k_f16(win_geo g, uint32_t cell0, uint32_t n, const uint16_t *rows) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n * g.H * g.D) return;
-    const uint32_t d = i % g.D, h = (i / g.D) % g.H, t = (uint32_t)(i / ((uint64_t)g.D * g.H));
-    const uint32_t cell = cell0 + t, tile = cell / 64, c = cell % 64;
-    uint16_t *dst = (uint16_t *)(g.k + ((uint64_t)h * g.n_tiles + tile) * g.ktile);
-    dst[kvm_kh_idx(g.D, c, d)] = rows[((uint64_t)t * g.H + h) * g.D + d];
-}
-
-// q4_0 V nibbles: one thread per destination 32-bit word (8 keys of one dim),
-// so the cells sharing a byte are written by one thread; cells outside
-// [cell0, cell0+n) keep their nibble.
-__global__ void k_import_v_q4(win_geo g, uint32_t cell0, uint32_t n, const uint8_t *rows) {
-    const uint32_t NB = g.D / 32;
-    const uint32_t t0 = cell0 / 64, t1 = (cell0 + n + 63) / 64;
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)(t1 - t0) * g.H * g.D * 8) return;
-    const uint32_t wi = i % (g.D * 8), h = (i / (8ull * g.D)) % g.H;
-    const uint32_t tile = t0 + (uint32_t)(i / (8ull * g.D * g.H));
-    const uint32_t X = wi >> 1, ks = wi & 1u;
-    const uint32_t d = (X >> 6) * 16 + (X & 15u), gg = (X & 63u) >> 4;
-    uint32_t *dst = (uint32_t *)(g.v + ((uint64_t)h * g.n_tiles + tile) * g.vtile + kvm_vq_word(d, gg, ks));
-    uint32_t word = *dst;
-    const uint32_t b = d / 32, e = d % 32;
+    uint16_t *sd = (uint16_t *)(vt + kvm_vd_off(D, (uint32_t)(c_s % 64), b));
+    if (in(c_s) && in(c_s + 3)) {
+        *(kvm_u32x2 *)sd = kvm_u32x2{sc[0] | (uint32_t)sc[1] << 16, sc[2] | (uint32_t)sc[3] << 16};
+    } else {
 #pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) {
-        const uint32_t cell = tile * 64 + 32 * ks + 8 * gg + j;
-        if (cell < cell0 || cell >= cell0 + n) continue;
-        const uint8_t *blk = rows + ((uint64_t)(cell - cell0) * g.H + h) * NB * 18 + (uint64_t)b * 18;
-        const uint32_t nib = e < 16 ? (blk[2 + e] & 15u) : (uint32_t)(blk[2 + e - 16] >> 4);
-        word = (word & ~(15u << kvm_vq_nib_shift(j))) | (nib << kvm_vq_nib_shift(j));
+        for (int j = 0; j < 4; ++j)
+            if (in(c_s + j)) sd[j] = sc[j];
     }
-    *dst = word;
 }
 
-__global__ void k_import_v_q4_scales(win_geo g, uint32_t cell0, uint32_t n, const uint8_t *rows) {
-    const uint32_t NB = g.D / 32;
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n * g.H * NB) return;
-    const uint32_t b = i % NB, h = (i / NB) % g.H, t = (uint32_t)(i / ((uint64_t)NB * g.H));
-    const uint32_t cell = cell0 + t, tile = cell / 64, c = cell % 64;
-    const uint8_t *blk = rows + ((uint64_t)t * g.H + h) * NB * 18 + (uint64_t)b * 18;
-    uint8_t *dst = g.v + ((uint64_t)h * g.n_tiles + tile) * g.vtile + kvm_vd_off(g.D, c, b);
-    dst[0] = blk[0];
-    dst[1] = blk[1];
-    if (b == 0 && h == 0) void_shadow(g, cell);
-}
-
-__global__ void k_import_v_f16(win_geo g, uint32_t cell0, uint32_t n, const uint16_t *rows) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n * g.H * g.D) return;
-    const uint32_t d = i % g.D, h = (i / g.D) % g.H, t = (uint32_t)(i / ((uint64_t)g.D * g.H));
-    const uint32_t cell = cell0 + t, tile = cell / 64, c = cell % 64;
+// V, f16: thread (tile, head, 32-cell half, 8-cell group, 8 dims): 8 x 8 values
+// change from a cell's dims to a dim's cells.
+template <int D>
+__device__ __forceinline__ void import_v_f16(const import_args &a, uint64_t i) {
+    const win_geo &g = a.g;
+    const uint32_t u = i % (D / 8), gk = (uint32_t)(i / (D / 8)) & 7u;
+    const uint64_t r = i / (D / 8) / 8;
+    const uint32_t h = (uint32_t)(r % g.H);
+    const uint64_t tile = a.cell0 / 64 + r / g.H, c0 = tile * 64 + 8 * gk, end = (uint64_t)a.cell0 + a.n;
+    if (c0 + 8 <= a.cell0 || c0 >= end) return;
+    kvm_u32x4 x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint64_t cell = c0 + j, t = cell < a.cell0 ? 0u : cell < end ? cell - a.cell0 : a.n - 1u;
+        x[j] = load_any<kvm_u32x4>(a.v_rows + ((t * g.H + h) * D + 8 * u) * 2);
+    }
     uint16_t *dst = (uint16_t *)(g.v + ((uint64_t)h * g.n_tiles + tile) * g.vtile);
-    dst[kvm_vh_idx(c, d)] = rows[((uint64_t)t * g.H + h) * g.D + d];
+    const bool full = c0 >= a.cell0 && c0 + 8 <= end;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        uint16_t *o = dst + kvm_vh_idx((uint32_t)(c0 % 64), 8 * u + d);
+        if (full) {
+            kvm_u32x4 y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                y[j] = __builtin_amdgcn_perm(x[2 * j + 1][d >> 1], x[2 * j][d >> 1], d & 1 ? 0x07060302u : 0x05040100u);
+            *(kvm_u32x4 *)o = y;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (c0 + j >= a.cell0 && c0 + j < end) o[j] = (uint16_t)(x[j][d >> 1] >> (16 * (d & 1)));
+        }
+    }
 }
 
-__global__ void k_copy_i32(int32_t *dst, const int32_t *src, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
+template <int D, int KT>
+__global__ void __launch_bounds__(256) k_import_rows(import_args a) {
+    const uint32_t blk = blockIdx.x, tid = threadIdx.x;
+    if (blk < a.nb_k) {
+        import_k<D, KT>(a, (uint64_t)blk * 256 + tid);
+    } else if (blk < a.nb_k + a.nb_v) {
+        const uint64_t i = (uint64_t)(blk - a.nb_k) * 256 + tid;
+        if constexpr (KT == KVM_TYPE_F16) import_v_f16<D>(a, i);
+        else import_v_q4<D>(a, i);
+    } else {
+        const uint32_t i = (blk - a.nb_k - a.nb_v) * 256 + tid;
+        if (a.pos && i < a.n) a.cell_pos[a.cell0 + i] = a.pos[i];
+        // slots: an import voids a slot's shadow (which holds only what a stage-in
+        // wrote) and raises its unharvested-row count to the end of its rows there
+        const uint32_t bt = a.g.bt, slot = a.cell0 / bt + i, end = a.cell0 + a.n;
+        if ((a.k_rows || a.v_rows) && slot < a.g.n_slots && slot * bt < end) {
+            if (KT != KVM_TYPE_F16 && a.g.shadow_rows) a.g.shadow_rows[slot] = 0u;
+            if (a.pending) {
+                const uint32_t rows = ((slot + 1) * bt < end ? (slot + 1) * bt : end) - slot * bt, cur = a.pending[slot];
+                a.pending[slot] = rows > cur ? rows : cur;
+            }
+        }
+    }
 }
 
-// The unharvested-row count of every slot that cells [cell0, cell0 + n) touch:
-// raised by the rows an import writes there (add), lowered by the rows a
-// harvest takes into the host history (sub, not below zero).  One thread per
-// slot.
-// Per touched slot: the end (rows from the slot's first cell) of the rows
-// imported since the last harvest that reached them.  An import raises it to
-// the end of its rows in the slot (a re-import of the same cells, e.g. after
-// rejected draft tokens, adds nothing); a harvest whose cells reach that end
-// clears it; a copy of the slot from the host clears it.
-enum pending_op { PENDING_IMPORT = 0, PENDING_HARVEST = 1, PENDING_CLEAR = 2 };
+// The unharvested-row counts of the slots that cells [cell0, cell0 + n) touch, one
+// thread per slot: the end (rows from the slot's first cell) of the rows imported
+// since the last harvest that reached them.  An import raises it to the end of its
+// rows in the slot (k_import_rows; a re-import of the same cells, e.g. after
+// rejected draft tokens, adds nothing); a harvest whose cells reach that end clears
+// it; a copy of the slot from the host clears it.
+enum pending_op { PENDING_HARVEST, PENDING_CLEAR };
 __global__ void k_pending_rows(uint32_t *pending, uint32_t bt, uint32_t n_slots, uint32_t cell0, uint32_t n,
                                int op) {
     const uint32_t slot = cell0 / bt + blockIdx.x * blockDim.x + threadIdx.x;
     if (slot >= n_slots || slot * bt >= cell0 + n) return;
     const uint32_t hi = (slot + 1) * bt < cell0 + n ? (slot + 1) * bt : cell0 + n;
-    const uint32_t end = hi - slot * bt, cur = pending[slot];
-    if (op == PENDING_IMPORT)
-        pending[slot] = end > cur ? end : cur;
-    else if (op == PENDING_CLEAR || end >= cur)
-        pending[slot] = 0u;
+    if (op == PENDING_CLEAR || hi - slot * bt >= pending[slot]) pending[slot] = 0u;
 }
 
 static void pending_rows(kvm_state *st, const kvm_window *w, uint32_t cell0, uint32_t n, pending_op op) {
@@ -245,42 +334,32 @@ extern "C" int kvm_window_import_rows(kvm_state *st, const kvm_window *w, uint32
     if ((uint64_t)cell0 + n > w->n_cells) return kvm_fail(st, KVM_ERANGE, "import_rows: cells past window");
     if (n == 0) return KVM_OK;
     KVM_HIP(st, hipSetDevice(st->device));
-    const win_geo g = geo_of(w);
-    const uint32_t NB = g.D / 32;
-    if (k_rows) {
-        if (w->k_type == KVM_TYPE_Q8_0) {
-            const uint64_t nt = (uint64_t)n * g.H * NB;
-            hipLaunchKernelGGL(k_import_k_q8, dim3(kvm_cdiv(nt, 256)), dim3(256), 0, st->stream, g, cell0, n,
-                               (const uint8_t *)k_rows);
-        } else if (w->k_type == KVM_TYPE_Q4_0) {
-            const uint64_t nt = (uint64_t)n * g.H * NB;
-            hipLaunchKernelGGL(k_import_k_q4, dim3(kvm_cdiv(nt, 256)), dim3(256), 0, st->stream, g, cell0, n,
-                               (const uint8_t *)k_rows);
-        } else {
-            const uint64_t nt = (uint64_t)n * g.H * g.D;
-            hipLaunchKernelGGL(k_import_k_f16, dim3(kvm_cdiv(nt, 256)), dim3(256), 0, st->stream, g, cell0, n,
-                               (const uint16_t *)k_rows);
-        }
-    }
-    if (v_rows) {
-        if (w->v_type == KVM_TYPE_Q4_0) {
-            const uint32_t t0 = cell0 / 64, t1 = (cell0 + n + 63) / 64;
-            const uint64_t nb = (uint64_t)(t1 - t0) * g.H * g.D * 8;
-            hipLaunchKernelGGL(k_import_v_q4, dim3(kvm_cdiv(nb, 256)), dim3(256), 0, st->stream, g, cell0, n,
-                               (const uint8_t *)v_rows);
-            const uint64_t ns = (uint64_t)n * g.H * NB;
-            hipLaunchKernelGGL(k_import_v_q4_scales, dim3(kvm_cdiv(ns, 256)), dim3(256), 0, st->stream, g,
-                               cell0, n, (const uint8_t *)v_rows);
-        } else {
-            const uint64_t nt = (uint64_t)n * g.H * g.D;
-            hipLaunchKernelGGL(k_import_v_f16, dim3(kvm_cdiv(nt, 256)), dim3(256), 0, st->stream, g, cell0, n,
-                               (const uint16_t *)v_rows);
-        }
-    }
-    if (pos)
-        hipLaunchKernelGGL(k_copy_i32, dim3(kvm_cdiv(n, 256)), dim3(256), 0, st->stream,
-                           w->cell_pos + cell0, pos, n);
-    if (w->pending_rows && (k_rows || v_rows)) pending_rows(st, w, cell0, n, PENDING_IMPORT);
+    import_args a{};
+    a.g = geo_of(w);
+    a.k_rows = (const uint8_t *)k_rows;
+    a.v_rows = (const uint8_t *)v_rows;
+    a.pos = pos;
+    a.cell_pos = w->cell_pos;
+    a.pending = w->pending_rows;
+    a.cell0 = cell0;
+    a.n = n;
+    const bool quant = kvm_k_quant(w->k_type);
+    const uint32_t H = a.g.H, D = a.g.D, tiles = (cell0 + n + 63) / 64 - cell0 / 64;
+    if (k_rows) a.nb_k = kvm_cdiv(quant ? (uint64_t)kvm_cdiv(n, 16) * 16 * H * (D / 32) : (uint64_t)n * H * (D / 8), 256);
+    if (v_rows) a.nb_v = kvm_cdiv((uint64_t)tiles * H * (quant ? D / 2 : D), 256);
+    const bool slots = (k_rows || v_rows) && (a.pending || a.g.shadow_rows);
+    const dim3 grid(a.nb_k + a.nb_v + (pos ? kvm_cdiv(n, 256) : slots ? kvm_cdiv(n / a.g.bt + 2, 256) : 0u));
+    if (grid.x == 0) return KVM_OK;
+    auto go = [&](auto d, auto kt) {
+        hipLaunchKernelGGL((k_import_rows<decltype(d)::value, decltype(kt)::value>), grid, dim3(256), 0, st->stream, a);
+    };
+    auto go_d = [&](auto d) {
+        if (w->k_type == KVM_TYPE_Q8_0) go(d, std::integral_constant<int, KVM_TYPE_Q8_0>{});
+        else if (w->k_type == KVM_TYPE_Q4_0) go(d, std::integral_constant<int, KVM_TYPE_Q4_0>{});
+        else go(d, std::integral_constant<int, KVM_TYPE_F16>{});
+    };
+    if (D == 256) go_d(std::integral_constant<int, 256>{});
+    else go_d(std::integral_constant<int, 128>{});
     KVM_LAUNCH_CHECK(st, "import_rows");
     return KVM_OK;
 }

@@ -92,3 +92,39 @@ def test_d2d_batched_alignments_and_sizes(kvm_state):
     for so, do, n in ops:
         want[do:do + n] = ah[so:so + n]
     assert np.array_equal(bh, want)
+
+
+@pytest.mark.parametrize("kt,vt,d,H", [(L.T_Q8_0, L.T_Q4_0, 256, 4), (L.T_Q4_0, L.T_Q4_0, 128, 1),
+                                       (L.T_F16, L.T_F16, 256, 2), (L.T_F16, L.T_F16, 128, 3)])
+@pytest.mark.parametrize("cell0,n", [(0, 1), (63, 1), (61, 5), (15, 17), (64, 64), (1, 191), (100, 156)])
+def test_window_import_ranges(kvm_state, kt, vt, d, H, cell0, n):
+    """Imports that start and end anywhere in a tile, from rows at an odd address:
+    the cells written hold the rows, the others keep theirs; positions, K alone
+    and V alone likewise."""
+    rng = np.random.default_rng(1000 * cell0 + n + d)
+    n_cells = 256
+    w = api.KVWindow(kvm_state, n_cells, H, d, 128, kt, vt)
+    kr, vr = rand_rows(rng, n_cells, H, d, kt, vt)
+    w.import_rows(0, dev(kr), dev(vr), dev(np.arange(n_cells, dtype=np.int32)))
+    k2, v2 = rand_rows(rng, n, H, d, kt, vt)
+
+    def odd(rows):
+        buf = torch.zeros(rows.size + 1, dtype=torch.uint8, device="cuda")
+        buf[1:] = torch.from_numpy(np.ascontiguousarray(rows).view(np.uint8).reshape(-1)).cuda()
+        return buf[1:].view(rows.shape[0], -1)
+
+    ref_k, ref_v, ref_p = kr.copy(), vr.copy(), np.arange(n_cells, dtype=np.int32)
+    for part in ("k", "v", "pos"):
+        pos = np.arange(5000, 5000 + n, dtype=np.int32)
+        if part == "pos":
+            w.import_rows(cell0, odd(k2), odd(v2), dev(pos))
+            ref_p[cell0:cell0 + n] = pos
+        else:
+            w.import_rows(cell0, odd(k2) if part == "k" else None, odd(v2) if part == "v" else None)
+            if part == "k":
+                ref_k[cell0:cell0 + n] = k2
+            else:
+                ref_v[cell0:cell0 + n] = v2
+        ek, ev = w.export_rows(0, n_cells)
+        assert np.array_equal(host(ek), ref_k) and np.array_equal(host(ev), ref_v), part
+        assert np.array_equal(host(w.cell_pos), ref_p), part
