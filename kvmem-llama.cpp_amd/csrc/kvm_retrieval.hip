@@ -97,57 +97,79 @@ __global__ void __launch_bounds__(64) k_query_add(qview_args a) {
 }
 
 // Many rows of a view whose heads are contiguous and 16-byte aligned
-// (query_rows_ok): a workgroup takes 64 embeddings, and wave 0's lanes add one
-// each, in row order.  What bounds it is that chain (2,048 dependent adds), so
-// the rows come through LDS, two 32 KB buffers filled by all four waves with
-// 16-byte loads: the chain of one buffer runs while the next one's loads are in
-// flight.  2,048 bf16 rows of 24 heads x 256 dims: 25.6 us, against 678 for one
-// thread per embedding with a load in flight at a time.
+// (query_rows_ok): a workgroup takes 32 embeddings, and wave 0's lanes add one
+// each, in row order.  What bounds it is that chain (2,048 dependent adds of ~5
+// cycles), so wave 0 does nothing else: waves 1 - 4 load the rows two buffers
+// ahead, convert them and lay them in LDS four rows of an embedding together, and
+// the chain reads 32 rows with 8 loads while it adds the 32 before.  2,048 bf16
+// rows of 24 heads x 256 dims: 23.4 us with the conversions and a load per value
+// in the chain, 18.2 here (678 for one thread per embedding with a load in
+// flight at a time).  The row quads' columns are rotated (by xor) so that the
+// stores of a wave spread over the banks.
 template <int T>
-__global__ void __launch_bounds__(256) k_query_add_rows(qview_args a) {
-    constexpr uint32_t ES = T == KVM_TYPE_F32 ? 4u : 2u, SEG = 64u * ES;   // bytes of one row's 64 values
-    constexpr uint32_t RB = 32768u / SEG, UPR = SEG / 16u, B = 8;          // rows of a buffer, 16-byte units of a row
-    static_assert(RB * UPR == 256u * B && RB % 32u == 0, "buffer split");
-    __shared__ __align__(16) uint8_t s_rows[2][RB * SEG];
-    const uint32_t tid = threadIdx.x, e0 = blockIdx.x * 64u;
-    const uint8_t *p = a.v.data + (size_t)a.t0 * a.v.nb2 + view_off(a.v, e0) + 16u * (tid % UPR);
-    // register sets: buffer c + 1's rows in one, c + 2's in the other
-    kvm_u32x4 r[2][B];
-    auto load = [&](kvm_u32x4 (&q)[B], uint32_t row0) {
+__global__ void __launch_bounds__(320) k_query_add_rows(qview_args a) {
+    constexpr uint32_t ES = T == KVM_TYPE_F32 ? 4u : 2u, VPU = 16u / ES, UPR = 32u / VPU;   // values of a 16-byte unit, units of a row
+    constexpr uint32_t QUADS = 256u / UPR, RB = 4u * QUADS;               // row quads and rows of a buffer
+    static_assert(QUADS % 8u == 0, "chain steps of 8 quads");
+    __shared__ __align__(16) kvm_f32x4 s_rows[2][QUADS * 32];
+    const uint32_t tid = threadIdx.x, e0 = blockIdx.x * 32u, n_buf = (a.n_rows + RB - 1) / RB;
+    if (tid >= 64u) {
+        const uint32_t t = tid - 64u, o = t % UPR, rq = t / UPR;
+        const uint8_t *p = a.v.data + (size_t)a.t0 * a.v.nb2 + view_off(a.v, e0) + 16u * o;
+        kvm_u32x4 r[2][4];
+        auto load = [&](kvm_u32x4 (&q)[4], uint32_t buf) {
 #pragma unroll
-        for (uint32_t j = 0; j < B; ++j) {
-            const uint32_t row = row0 + (j * 256u + tid) / UPR;
-            q[j] = *(const kvm_u32x4 *)(p + (size_t)(row < a.n_rows ? row : a.n_rows - 1) * a.v.nb2);
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t row = buf * RB + 4u * rq + j;
+                q[j] = *(const kvm_u32x4 *)(p + (size_t)(row < a.n_rows ? row : a.n_rows - 1) * a.v.nb2);
+            }
+        };
+        auto store = [&](const kvm_u32x4 (&q)[4], uint32_t b) {
+#pragma unroll
+            for (uint32_t k = 0; k < VPU; ++k) {
+                kvm_f32x4 x;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    x[j] = raw_value<T>(T == KVM_TYPE_F32 ? q[j][k] : (q[j][k >> 1] >> (16u * (k & 1u))) & 0xffffu);
+                s_rows[b][rq * 32u + ((VPU * o + k) ^ (rq & 7u))] = x;
+            }
+        };
+        load(r[0], 0);
+        load(r[1], 1);
+        store(r[0], 0);
+        load(r[0], 2);
+        __syncthreads();
+        for (uint32_t i = 0; i < n_buf; i += 2) {
+            store(r[1], 1);
+            load(r[1], i + 3);
+            __syncthreads();
+            if (i + 1 >= n_buf) break;
+            store(r[0], 0);
+            load(r[0], i + 4);
+            __syncthreads();
         }
-    };
-    auto store = [&](const kvm_u32x4 (&q)[B], uint32_t b) {
+    } else {
+        const uint32_t e = tid & 31u;                     // (the upper lanes repeat the lower ones)
+        float s = a.q_sum[e0 + e];
+        uint32_t keep = a.keep[0];
+        __syncthreads();
+        for (uint32_t i = 0; i < n_buf; ++i) {
+            const kvm_f32x4 *x = s_rows[i & 1u];
+            const uint32_t nr = a.n_rows - i * RB < RB ? a.n_rows - i * RB : RB;
+            kvm_f32x4 v[2][8];
+            auto read = [&](kvm_f32x4 (&q)[8], uint32_t c) {        // rows c .. c + 31 of the buffer
 #pragma unroll
-        for (uint32_t j = 0; j < B; ++j) *(kvm_u32x4 *)&s_rows[b][16u * (j * 256u + tid)] = q[j];
-    };
-    load(r[0], 0);
-    load(r[1], RB);
-    float s = tid < 64u ? a.q_sum[e0 + tid] : 0.0f;
-    store(r[0], 0);
-    __syncthreads();
-    auto step = [&](uint32_t row0, uint32_t b, kvm_u32x4 (&later)[B], const kvm_u32x4 (&next)[B]) {
-        load(later, row0 + 2 * RB);
-        if (tid < 64u) {
-            const uint8_t *x = &s_rows[b][tid * ES];
-            const uint32_t nr = a.n_rows - row0 < RB ? a.n_rows - row0 : RB;
-            // the LDS reads of the next 32 rows run under the adds of these 32
-            float v[2][32];
-            auto read = [&](float (&o)[32], uint32_t c) {
-#pragma unroll
-                for (uint32_t i = 0; i < 32; ++i) o[i] = view_value<T>(x + (c + i) * SEG);
+                for (uint32_t j = 0; j < 8; ++j) q[j] = x[(c / 4u + j) * 32u + (e ^ j)];
             };
-            auto add = [&](const float (&o)[32], uint32_t c) {
-                const uint32_t k = a.keep[(row0 + c) >> 5];     // bits past n_rows are 0
+            auto add = [&](const kvm_f32x4 (&q)[8], uint32_t c) {
+                const uint32_t k = keep, w = (i * RB + c) / 32u + 1u;
+                keep = a.keep[w < KVM_QVIEW_ROWS / 32 ? w : 0u];    // bits past n_rows are 0
                 if (k == 0xffffffffu) {
 #pragma unroll
-                    for (uint32_t i = 0; i < 32; ++i) s = kvm_fadd(s, o[i]);
+                    for (uint32_t j = 0; j < 32; ++j) s = kvm_fadd(s, q[j >> 2][j & 3]);
                 } else {
 #pragma unroll
-                    for (uint32_t i = 0; i < 32; ++i) s = (k >> i) & 1u ? kvm_fadd(s, o[i]) : s;
+                    for (uint32_t j = 0; j < 32; ++j) s = (k >> j) & 1u ? kvm_fadd(s, q[j >> 2][j & 3]) : s;
                 }
             };
             read(v[0], 0);
@@ -158,16 +180,11 @@ __global__ void __launch_bounds__(256) k_query_add_rows(qview_args a) {
                 read(v[0], c + 64u < RB ? c + 64u : 0u);
                 add(v[1], c + 32u);
             }
+            __syncthreads();
         }
-        store(next, b ^ 1u);
-        __syncthreads();
-    };
-    for (uint32_t row0 = 0; row0 < a.n_rows; row0 += 2 * RB) {
-        step(row0, 0, r[0], r[1]);
-        if (row0 + RB < a.n_rows) step(row0 + RB, 1, r[1], r[0]);
+        if (tid < 32u) a.q_sum[e0 + e] = s;
+        if (e0 == 0 && tid == 0) a.q_count[0] += a.n_kept;
     }
-    if (tid < 64u) a.q_sum[e0 + tid] = s;
-    if (e0 == 0 && tid == 0) a.q_count[0] += a.n_kept;
 }
 
 // Zeroes up to four runs of 32-bit words in one launch.
@@ -311,7 +328,7 @@ extern "C" int kvm_query_add_view(kvm_state *st, const kvm_query_acc *acc, uint3
         auto go = [&](auto t) {
             constexpr int T = decltype(t)::value;
             if (rows_ok && a.n_rows > KVM_QROWS_MIN)
-                hipLaunchKernelGGL(k_query_add_rows<T>, dim3(n_embd / 64), dim3(256), 0, st->stream, a);
+                hipLaunchKernelGGL(k_query_add_rows<T>, dim3(n_embd / 32), dim3(320), 0, st->stream, a);
             else
                 hipLaunchKernelGGL(k_query_add<T>, dim3(kvm_cdiv(n_embd, 64)), dim3(64), 0, st->stream, a);
         };
