@@ -378,6 +378,8 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
             for (int r = 0; r < 16; ++r) O[dt][r] = 0.0f;
         float ms = -INFINITY, lp = 0.0f;        // running max of the row (times c), lane's share of its sum
         const float c = a.c;
+        // a wave of padding rows only copies and converts
+        const bool active = rt_i * ROWS + 32u * rg < a.n_rows;
 
         // operand addresses of a lane: K row m2 is key m2 with bits 2 and 3 swapped
         auto k_lane = [&](uint32_t x) {
@@ -542,14 +544,16 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
                     dma_tile(t_begin + (en & 0x7fffu), b ^ 1u);       // next tile, in flight during this one
                     const bool masked = (e >> 15) == 0;
                     const uint8_t *sk = s_mem + b * (2 * TILE_B) + k_ofs, *sv = s_mem + b * (2 * TILE_B) + TILE_B + v_ofs;
+                    if (active) {
 #pragma unroll
-                    for (int sub = 0; sub < 2 / KW; ++sub) {
-                        kvm_f32x16 S = scores(sk + sub * 2 * NB * 1024, nothing);
-                        kvm_f16x8 vr[VR];
+                        for (int sub = 0; sub < 2 / KW; ++sub) {
+                            kvm_f32x16 S = scores(sk + sub * 2 * NB * 1024, nothing);
+                            kvm_f16x8 vr[VR];
 #pragma unroll
-                        for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv + sub * (TILE_B / 2), i);
-                        const float msr = settle(S, masked, &s_cp[b][32 * (KW == 2 ? kg : sub)]);
-                        accumulate(sv + sub * (TILE_B / 2), S, msr, vr, nothing);
+                            for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv + sub * (TILE_B / 2), i);
+                            const float msr = settle(S, masked, &s_cp[b][32 * (KW == 2 ? kg : sub)]);
+                            accumulate(sv + sub * (TILE_B / 2), S, msr, vr, nothing);
+                        }
                     }
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's copies
                     __syncthreads();
@@ -661,16 +665,26 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
                     const bool masked = (e0 >> 15) == 0;
                     dma_k(e2, k + 2);
                     const uint8_t *vraw = s_vr + b * VRAW_L, *kraw = s_kr + (b ^ 1u) * KRAW_L;
-                    kvm_f32x16 S = scores(s_k + k_lane(opaque(l)), [&](int i) { conv_v(vraw, i); });
-                    const float msr = settle(S, masked, &s_cp[k & 3u][32 * kg]);
-                    wait_copies();
-                    KVM_LDS_BARRIER();
-                    dma_v(e2, k + 2);
-                    const uint8_t *sv = s_v + v_lane(opaque(l));
-                    kvm_f16x8 vr[VR];
+                    if (active) {
+                        kvm_f32x16 S = scores(s_k + k_lane(opaque(l)), [&](int i) { conv_v(vraw, i); });
+                        const float msr = settle(S, masked, &s_cp[k & 3u][32 * kg]);
+                        wait_copies();
+                        KVM_LDS_BARRIER();
+                        dma_v(e2, k + 2);
+                        const uint8_t *sv = s_v + v_lane(opaque(l));
+                        kvm_f16x8 vr[VR];
 #pragma unroll
-                    for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv, i);
-                    accumulate(sv, S, msr, vr, [&](int i) { conv_k(kraw, i); });
+                        for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv, i);
+                        accumulate(sv, S, msr, vr, [&](int i) { conv_k(kraw, i); });
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < KS; ++i) conv_v(vraw, i);
+                        wait_copies();
+                        KVM_LDS_BARRIER();
+                        dma_v(e2, k + 2);
+#pragma unroll
+                        for (int i = 0; i < KS; ++i) conv_k(kraw, i);
+                    }
                     e0 = e1;
                     e1 = e2;
                     e2 = __builtin_amdgcn_readfirstlane(e_far);
