@@ -9,13 +9,13 @@
 // and a multi-token query, ggml's GPU backends convert K and V to f16 and run
 // an f16 matrix-core kernel; this file does the same with CDNA4 MFMA.
 //
-// k_pf_attn: one workgroup of 8 waves per CU; a row is (token, query head of the
-// group), so the query heads of a kv head share every K/V tile.  Each wave has 32
-// rows: the 32x32x16 MFMA reads half the LDS bytes per flop of 16 rows a wave.  A
-// unit is 256 / KW rows of a kv head (KW = 2: two waves share 32 rows, one on each
-// half of a tile's keys, and meet at the end).  The units' keys are dealt to the
-// workgroups in equal shares (pf_shares), so the CUs have the same work whatever
-// the shape; k_pf_combine merges the units that several workgroups share.
+// One workgroup of 8 waves per CU; a row is (token, query head of the group), so the
+// query heads of a kv head share every K/V tile.  A wave has 32 rows: the 32x32x16
+// MFMA reads half the LDS bytes per flop of 16 rows a wave.  A unit is 256 rows of a
+// kv head (k_pf_attn: eight such waves) or 128 (k_pf_attn_split: four, and four that
+// bring the tiles).  The units' keys are dealt to the workgroups in equal shares
+// (pf_shares), so the CUs have the same work whatever the shape; k_pf_combine merges
+// the units that several workgroups share.
 // S^T = K Q^T and O^T += V^T P^T.  Key order: score row i of a 32-key sub tile is
 // key i with bits 2 and 3 swapped (the lane that supplies K row i reads that key),
 // so that the accumulator holds for each lane the 8 consecutive keys that the P V
@@ -23,20 +23,19 @@
 // domain with a lazy running maximum (rescale only when a row max grows by more
 // than 2^8).  Tiles no row of the unit can see are left out of its list; tiles
 // every row sees in full skip the mask.
-// Where the tiles come from (SRC, pf_choose):
+// Where the tiles come from (SRC):
 //   PF_F16    an f16 window's tiles, which are the MFMA operands already, copied
 //             global -> LDS, double buffered;
 //   PF_STAGED the same from a workspace into which k_pf_stage converted the
-//             quantised window: one conversion for all row tiles;
-//   PF_QUANT  the quantised tiles, copied as they are and converted in LDS by
-//             the attention itself, between its MFMAs (few row tiles).
+//             quantised window: one conversion for all row tiles (256-row units);
+//   PF_QUANT  the quantised tiles, converted by the attention's own waves (128).
 // f16 tiles: K as kvm_kh_idx; V units of 8 keys of a dim (as kvm_vh_idx), in LDS
 // and in the workspace in the order [32-key half][16-dim tile][8-key group][dim].
 // What bounds it: large chunks, the matrix cores at the clock that the power limit
 // leaves (2,048 tokens x 34,816 cells: 1.10 -> 1.15 PFLOP/s, a large f16 matrix
-// product reaches 1.33); small ones, the latencies of the start and the piece
-// traffic (37 tokens x 32,768 cells: 147 -> 65 us; 100 x 8,192: 54.3 -> 47;
-// 700 x 8,192 on an f16 cache of 2 heads x 128: 51.6 -> 42).
+// product reaches 1.33); small ones, the attention waves' chain, the latencies of the
+// start and the piece traffic (37 tokens x 32,768 cells: 147 -> 54 us; 100 x 8,192:
+// 54.3 -> 40; 700 x 8,192 on an f16 cache of 2 heads x 128: 51.6 -> 41).
 #include "kvm_internal.h"
 
 #include <type_traits>
@@ -184,35 +183,145 @@ struct pf_args {
     int q_bf16;
 };
 
-template <int D, int KW, int SRC, bool BF16>
+// Q rows of a unit into LDS, coalesced (as operand loads, 32 rows of 32 bytes an
+// instruction, they took 4 us): unit c of 16 bytes of row r at slot c ^ r, so that a
+// column's reads use every bank; Q_UC units of each row a pass.  Rows past the last
+// are row 0's: their results are never stored.
+template <int D, int ROWS, uint32_t Q_UC, bool BF16>
+__device__ __forceinline__ void pf_copy_q(const pf_args &a, uint32_t rt_i, uint32_t h, int pass, uint32_t lds, int w, int l) {
+    constexpr uint32_t Q_UNITS = D * (BF16 ? 2 : 4) / 16;
+    constexpr int N = ROWS * Q_UC / 64 / 8;               // 1 KB copies of a wave
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t x = opaque((w * N + i) * 64 + l), r = x / Q_UC, c = (x ^ r) % Q_UC;
+        const uint32_t rr = rt_i * ROWS + r < a.n_rows ? rt_i * ROWS + r : 0u, t = rr / a.G;
+        const uint8_t *src = (const uint8_t *)a.q + (((uint64_t)t * a.n_head + h * a.G + (rr - t * a.G)) * Q_UNITS + pass * Q_UC + c) * 16;
+        uint32_t m0_saved;
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                     : "=&s"(m0_saved) : "v"(src), "s"(lds + (w * N + i) * 1024u) : "memory");
+    }
+}
+
+// The start of a unit's piece: the lane's visibility limit, and the piece's tiles in
+// fr.list: the segment's tiles that some row of the workgroup can see, in order, and
+// of these the share [f_lo, f_hi) / P (returned: how many).
+struct pf_front {
+    uint8_t flag[KVM_PF_LIST];       // per tile: bit 0 some cell visible to some row, bit 1 all to all
+    uint16_t list[KVM_PF_LIST];      // tile - t_begin, bit 15: every cell live and visible to every row, so no mask
+    uint32_t mm[2][8], cnt[KVM_PF_LIST / 64];
+};
+template <bool STAGED, typename COPY_Q>
+__device__ __forceinline__ uint32_t pf_tiles(const pf_args &a, uint32_t row, uint32_t t_begin, uint32_t f_lo, uint32_t f_hi,
+                                             pf_front &fr, uint32_t &qlim, COPY_Q &&copy_q) {
+    const int tid = (int)opaque((int)threadIdx.x), l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+            // ---- the loads of the prologue, all issued before any is used: the lane's
+            // row position, the tiles' cells (or summaries), the Q row
+            const bool live_row = row < a.n_rows;
+            const int32_t qp = a.q_pos[(live_row ? row : 0u) / a.G];
+            const uint32_t n_seg_t = a.n_tiles - t_begin < KVM_PF_LIST ? a.n_tiles - t_begin : KVM_PF_LIST;
+            // a wave looks at 4 tiles at a time, 4 cells a lane (PF_STAGED: a lane at one tile's summary)
+            constexpr uint32_t NL = STAGED ? 2 : 18, TPL = STAGED ? 64 : 4, TPB = NL * 8 * TPL;
+            const uint32_t t_lane = STAGED ? (uint32_t)tid : (uint32_t)(4 * w + (l >> 4));
+            kvm_u32x4 cells[NL];
+            auto load_cells = [&](uint32_t t0) {
+#pragma unroll
+                for (uint32_t i = 0; i < NL; ++i) {
+                    const uint32_t t = t0 + 8 * TPL * i + t_lane;
+                    const uint64_t tile = t_begin + (t < n_seg_t ? t : 0u);
+                    cells[i] = STAGED ? *(const kvm_u32x4 *)(a.info + tile * 4)
+                                                : *(const kvm_u32x4 *)(a.cell_pos + tile * 64 + 4 * (l & 15));
+                }
+            };
+            load_cells(0);
+            copy_q();
+
+
+            // ---- a cell is visible to the lane's row iff (unsigned)position < qlim
+            qlim = live_row && qp >= 0 ? (uint32_t)qp + 1u : 0u;
+            const uint32_t mn = kvm_wave_min_u32(live_row ? qlim : 0xffffffffu), mx = ~kvm_wave_min_u32(~qlim);
+            if (l == 0) {
+                fr.mm[0][w] = mn;
+                fr.mm[1][w] = mx;
+            }
+            KVM_LDS_BARRIER();
+            uint32_t wg_min = fr.mm[0][0], wg_max = fr.mm[1][0];
+#pragma unroll
+            for (int i = 1; i < 8; ++i) {
+                wg_min = min(wg_min, fr.mm[0][i]);
+                wg_max = max(wg_max, fr.mm[1][i]);
+            }
+
+            // ---- the piece's tiles: the segment's tiles that some row here can see,
+            // in order, and of these the share [f_lo, f_hi) / P.  fr.list holds tile -
+            // t_begin and bit 15: every cell live and visible to every row, so no mask.
+            for (uint32_t t0 = 0;;) {
+#pragma unroll
+                for (uint32_t i = 0; i < NL; ++i) {
+                    const uint32_t t = t0 + 8 * TPL * i + t_lane;
+                    const kvm_u32x4 c = cells[i];
+                    bool some, all;
+                    if constexpr (STAGED) {
+                        some = c[2] != 0 && c[0] < wg_max;
+                        all = c[2] == 64 && c[1] < wg_min;
+                    } else {
+                        const uint32_t lo = min(min(c[0], c[1]), min(c[2], c[3])), hi = max(max(c[0], c[1]), max(c[2], c[3]));
+                        some = ((uint32_t)(__builtin_amdgcn_ballot_w64(lo < wg_max) >> (l & 48)) & 0xffffu) != 0;
+                        all = ((uint32_t)(__builtin_amdgcn_ballot_w64(hi < wg_min) >> (l & 48)) & 0xffffu) == 0xffffu;
+                    }
+                    if (t < n_seg_t && (STAGED || (l & 15) == 0)) fr.flag[t] = (uint8_t)(some | all << 1);
+                }
+                t0 += TPB;
+                if (t0 >= n_seg_t) break;
+                load_cells(t0);
+            }
+            KVM_LDS_BARRIER();
+            uint32_t n_t;
+            {
+                const uint32_t n_it = (n_seg_t + 511) / 512;
+                auto flag = [&](uint32_t it) { return 512 * it + tid < n_seg_t ? (uint32_t)fr.flag[512 * it + tid] : 0u; };
+                for (uint32_t it = 0; it < n_it; ++it) {
+                    const uint64_t bal = __builtin_amdgcn_ballot_w64(flag(it) & 1u);
+                    if (l == 0) fr.cnt[8 * it + w] = __popcll(bal);
+                }
+                KVM_LDS_BARRIER();
+                // every wave scans the counts of all (at most 16 x 8 of them)
+                const uint32_t c0 = (uint32_t)l < 8 * n_it ? fr.cnt[l] : 0u, c1 = (uint32_t)l + 64 < 8 * n_it ? fr.cnt[l + 64] : 0u;
+                const uint32_t i0 = kvm_wave_incl_scan(c0), half = __builtin_amdgcn_readlane(i0, 63);
+                const uint32_t i1 = n_it > 8 ? kvm_wave_incl_scan(c1) : 0u, total = half + (n_it > 8 ? __builtin_amdgcn_readlane(i1, 63) : 0u);
+                const uint32_t lo = total * f_lo / a.P, hi = total * f_hi / a.P;     // P <= 2^16
+                n_t = hi - lo;
+                for (uint32_t it = 0; it < n_it; ++it) {
+                    const uint32_t f = flag(it), x = 8 * it + w;
+                    const uint64_t bal = __builtin_amdgcn_ballot_w64(f & 1u);
+                    const uint32_t base = x < 64 ? __builtin_amdgcn_readlane(i0 - c0, x) : half + __builtin_amdgcn_readlane(i1 - c1, x - 64);
+                    const uint32_t rank = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                    if ((f & 1u) && rank >= lo && rank < hi) fr.list[rank - lo] = (uint16_t)((512 * it + tid) | (f >> 1) << 15);
+                }
+                KVM_LDS_BARRIER();
+            }
+    return n_t;
+}
+
+template <int D, int SRC, bool BF16>
 __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
     // LDS operand rings: K runs KR-1 k-steps ahead of its MFMAs, V VR-1
     // operands ahead (the first ones in flight during the softmax)
     constexpr int KR = 3, VR = 3;
-    constexpr int RG = 8 / KW, ROWS = 32 * RG;            // row groups (of 32) of a unit
+    constexpr int ROWS = 256;
     constexpr int KS = D / 16, DT = D / 32, NB = D / 32;
     constexpr uint32_t TILE_B = 128u * D;                 // bytes of an f16 K (or V) tile
-    constexpr uint32_t KRAW = 64u * D + 64u * NB * 2u, VRAW = 32u * D + NB * 128u;    // quantised tiles
-    constexpr uint32_t KRAW_L = (KRAW + 1023u) & ~1023u, VRAW_L = (VRAW + 1023u) & ~1023u;
-    static_assert(SRC != PF_QUANT || KW == 2, "the converting form has one sub tile a wave");
-    constexpr uint32_t MEM = 4u * TILE_B;                 // two K/V buffers; RG * 32 rows of O when key groups merge
-    static_assert(SRC != PF_QUANT || 2u * TILE_B + 2u * (KRAW_L + VRAW_L) <= MEM, "LDS");
+    constexpr uint32_t MEM = 4u * TILE_B;                 // two K/V buffers
     // Q in LDS: units of 16 bytes of a row, of these at a time, and where: beside
     // the first tile's copies if it fits there
     constexpr uint32_t Q_UNITS = D * (BF16 ? 2 : 4) / 16, Q_UC = Q_UNITS * ROWS * 16 <= MEM ? Q_UNITS : Q_UNITS / 2;
     constexpr bool Q_EARLY = Q_UC * ROWS * 16 <= 2 * TILE_B;
-    constexpr uint32_t Q_OFS = Q_EARLY && SRC != PF_QUANT ? 2 * TILE_B : 0;
+    constexpr uint32_t Q_OFS = Q_EARLY ? 2 * TILE_B : 0;
     static_assert(Q_UC * ROWS * 16 <= MEM && (Q_UNITS == Q_UC || Q_UNITS == 2 * Q_UC), "Q passes");
     __shared__ __align__(16) uint8_t s_mem[MEM];
-    __shared__ uint8_t s_flag[KVM_PF_LIST];               // per tile: bit 0 some cell visible to some row, bit 1 all to all
-    __shared__ __align__(16) int32_t s_cp[4][64];         // the tiles' cell positions
-    __shared__ uint16_t s_list[KVM_PF_LIST];
-    __shared__ uint32_t s_mm[2][8];
-    __shared__ uint32_t s_cnt[KVM_PF_LIST / 64];
-    __shared__ float s_ml[KW == 2 ? 8 : 1][32][2];
-    const int tid = threadIdx.x, l = tid & 63, g2 = l >> 5, m2 = l & 31;
+    __shared__ pf_front s_front;
+    __shared__ __align__(16) int32_t s_cp[2][64];         // the tiles' cell positions
+    const int tid = threadIdx.x, l = tid & 63, m2 = l & 31;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rg = w / KW, kg = w % KW;
 
     const uint32_t lds_mem = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_mem[0];
 
@@ -230,117 +339,17 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
         const uint32_t rt_i = __builtin_amdgcn_readfirstlane(rest % a.n_row_tiles), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
         const bool whole = f_lo == 0 && f_hi == a.P && a.n_seg == 1;
 
-        // ---- the loads of the prologue, all issued before any is used: the lane's
-        // row position, the tiles' cells (or summaries), the Q row
-        const uint32_t row = rt_i * ROWS + 32 * rg + m2;
-        const bool live_row = row < a.n_rows;
-        const uint32_t row_ld = live_row ? row : 0u, tok = row_ld / a.G;
-        const int32_t qp = a.q_pos[tok];
+        const uint32_t row = rt_i * ROWS + 32 * w + m2;
         const uint32_t t_begin = seg * KVM_PF_LIST;
-        const uint32_t n_seg_t = a.n_tiles - t_begin < KVM_PF_LIST ? a.n_tiles - t_begin : KVM_PF_LIST;
-        // a wave looks at 4 tiles at a time, 4 cells a lane (PF_STAGED: a lane at one tile's summary)
-        constexpr uint32_t NL = SRC == PF_STAGED ? 2 : 18, TPL = SRC == PF_STAGED ? 64 : 4, TPB = NL * 8 * TPL;
-        const uint32_t t_lane = SRC == PF_STAGED ? (uint32_t)tid : (uint32_t)(4 * w + (l >> 4));
-        kvm_u32x4 cells[NL];
-        auto load_cells = [&](uint32_t t0) {
-#pragma unroll
-            for (uint32_t i = 0; i < NL; ++i) {
-                const uint32_t t = t0 + 8 * TPL * i + t_lane;
-                const uint64_t tile = t_begin + (t < n_seg_t ? t : 0u);
-                cells[i] = SRC == PF_STAGED ? *(const kvm_u32x4 *)(a.info + tile * 4)
-                                            : *(const kvm_u32x4 *)(a.cell_pos + tile * 64 + 4 * (l & 15));
-            }
-        };
-        load_cells(0);
-        // (rows past the last are row 0's: their results are never stored)
-        // Q rows, coalesced into LDS (as operand loads, 32 rows of 32 bytes an
-        // instruction, they took 4 us): unit c of row r at slot c ^ r, so that a
-        // column's reads use every bank.  Q_UC units of 16 bytes of each row a pass.
-        const uint8_t *q_head = (const uint8_t *)a.q;
-        auto dma_q = [&](int pass) {
-            constexpr int N = ROWS * Q_UC / 64 / 8;       // 1 KB copies of a wave
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const uint32_t x = opaque((w * N + i) * 64 + l), r = x / Q_UC, c = (x ^ r) % Q_UC;
-                const uint32_t rr = rt_i * ROWS + r < a.n_rows ? rt_i * ROWS + r : 0u, t = rr / a.G;
-                const uint8_t *src = q_head + (((uint64_t)t * a.n_head + h * a.G + (rr - t * a.G)) * Q_UNITS + pass * Q_UC + c) * 16;
-                uint32_t m0_saved;
-                asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                             : "=&s"(m0_saved) : "v"(src), "s"(lds_mem + Q_OFS + (w * N + i) * 1024u) : "memory");
-            }
-        };
-        __builtin_amdgcn_sched_barrier(0);
-        dma_q(0);
-
-        // ---- a cell is visible to the lane's row iff (unsigned)position < qlim
-        const uint32_t qlim = live_row && qp >= 0 ? (uint32_t)qp + 1u : 0u;
-        const uint32_t mn = kvm_wave_min_u32(live_row ? qlim : 0xffffffffu), mx = ~kvm_wave_min_u32(~qlim);
-        if (l == 0) {
-            s_mm[0][w] = mn;
-            s_mm[1][w] = mx;
-        }
-        KVM_LDS_BARRIER();
-        uint32_t wg_min = s_mm[0][0], wg_max = s_mm[1][0];
-#pragma unroll
-        for (int i = 1; i < 8; ++i) {
-            wg_min = min(wg_min, s_mm[0][i]);
-            wg_max = max(wg_max, s_mm[1][i]);
-        }
-
-        // ---- the piece's tiles: the segment's tiles that some row here can see,
-        // in order, and of these the share [f_lo, f_hi) / P.  s_list holds tile -
-        // t_begin and bit 15: every cell live and visible to every row, so no mask.
-        for (uint32_t t0 = 0;;) {
-#pragma unroll
-            for (uint32_t i = 0; i < NL; ++i) {
-                const uint32_t t = t0 + 8 * TPL * i + t_lane;
-                const kvm_u32x4 c = cells[i];
-                bool some, all;
-                if constexpr (SRC == PF_STAGED) {
-                    some = c[2] != 0 && c[0] < wg_max;
-                    all = c[2] == 64 && c[1] < wg_min;
-                } else {
-                    const uint32_t lo = min(min(c[0], c[1]), min(c[2], c[3])), hi = max(max(c[0], c[1]), max(c[2], c[3]));
-                    some = ((uint32_t)(__builtin_amdgcn_ballot_w64(lo < wg_max) >> (l & 48)) & 0xffffu) != 0;
-                    all = ((uint32_t)(__builtin_amdgcn_ballot_w64(hi < wg_min) >> (l & 48)) & 0xffffu) == 0xffffu;
-                }
-                if (t < n_seg_t && (SRC == PF_STAGED || (l & 15) == 0)) s_flag[t] = (uint8_t)(some | all << 1);
-            }
-            t0 += TPB;
-            if (t0 >= n_seg_t) break;
-            load_cells(t0);
-        }
-        KVM_LDS_BARRIER();
-        uint32_t n_t;
-        {
-            const uint32_t n_it = (n_seg_t + 511) / 512;
-            auto flag = [&](uint32_t it) { return 512 * it + tid < n_seg_t ? (uint32_t)s_flag[512 * it + tid] : 0u; };
-            for (uint32_t it = 0; it < n_it; ++it) {
-                const uint64_t bal = __builtin_amdgcn_ballot_w64(flag(it) & 1u);
-                if (l == 0) s_cnt[8 * it + w] = __popcll(bal);
-            }
-            KVM_LDS_BARRIER();
-            // every wave scans the counts of all (at most 16 x 8 of them)
-            const uint32_t c0 = (uint32_t)l < 8 * n_it ? s_cnt[l] : 0u, c1 = (uint32_t)l + 64 < 8 * n_it ? s_cnt[l + 64] : 0u;
-            const uint32_t i0 = kvm_wave_incl_scan(c0), half = __builtin_amdgcn_readlane(i0, 63);
-            const uint32_t i1 = n_it > 8 ? kvm_wave_incl_scan(c1) : 0u, total = half + (n_it > 8 ? __builtin_amdgcn_readlane(i1, 63) : 0u);
-            const uint32_t lo = total * f_lo / a.P, hi = total * f_hi / a.P;     // P <= 2^16
-            n_t = hi - lo;
-            for (uint32_t it = 0; it < n_it; ++it) {
-                const uint32_t f = flag(it), x = 8 * it + w;
-                const uint64_t bal = __builtin_amdgcn_ballot_w64(f & 1u);
-                const uint32_t base = x < 64 ? __builtin_amdgcn_readlane(i0 - c0, x) : half + __builtin_amdgcn_readlane(i1 - c1, x - 64);
-                const uint32_t rank = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                if ((f & 1u) && rank >= lo && rank < hi) s_list[rank - lo] = (uint16_t)((512 * it + tid) | (f >> 1) << 15);
-            }
-            KVM_LDS_BARRIER();
-        }
-        auto entry = [&](uint32_t k) { return (uint32_t)s_list[k < n_t ? k : n_t - 1]; };
+        uint32_t qlim;
+        auto dma_q = [&](int pass) { pf_copy_q<D, ROWS, Q_UC, BF16>(a, rt_i, h, pass, lds_mem + Q_OFS, w, l); };
+        const uint32_t n_t = pf_tiles<false>(a, row, t_begin, f_lo, f_hi, s_front, qlim, [&]() { dma_q(0); });
+        auto entry = [&](uint32_t k) { return (uint32_t)s_front.list[k < n_t ? k : n_t - 1]; };
 
         // Q rows as f16 B operands: lane (g2, m2) holds Q[row m2][16ks + 8 g2 .. +7]
         kvm_f16x8 qop[KS];
         auto take_q = [&](int pass) {
-            const uint32_t le = opaque(l), r = 32 * rg + (le & 31u), sw = r % Q_UC;
+            const uint32_t le = opaque(l), r = 32 * w + (le & 31u), sw = r % Q_UC;
             const uint8_t *qr = s_mem + Q_OFS + r * (Q_UC * 16);
             constexpr int KP = KS * Q_UC / Q_UNITS;       // k-steps of a pass
 #pragma unroll
@@ -378,18 +387,18 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
             for (int r = 0; r < 16; ++r) O[dt][r] = 0.0f;
         float ms = -INFINITY, lp = 0.0f;        // running max of the row (times c), lane's share of its sum
         const float c = a.c;
-        // a wave of padding rows only copies and converts
-        const bool active = rt_i * ROWS + 32u * rg < a.n_rows;
+        // a wave of padding rows only copies
+        const bool active = rt_i * ROWS + 32u * w < a.n_rows;
 
         // operand addresses of a lane: K row m2 is key m2 with bits 2 and 3 swapped
         auto k_lane = [&](uint32_t x) {
             const uint32_t key = (x & 0x13) | (x & 4) << 1 | (x & 8) >> 1;
-            return ((key >> 4) * NB * 64 + 16 * (x >> 5) + (key & 15)) * 16 + (KW == 2 ? kg * 2 * NB * 1024 : 0);
+            return ((key >> 4) * NB * 64 + 16 * (x >> 5) + (key & 15)) * 16;
         };
-        auto v_lane = [&](uint32_t x) { return ((x >> 4 & 1) * 64 + 16 * (x >> 5) + (x & 15)) * 16 + (KW == 2 ? kg * (TILE_B / 2) : 0); };
+        auto v_lane = [&](uint32_t x) { return ((x >> 4 & 1) * 64 + 16 * (x >> 5) + (x & 15)) * 16; };
 
         // S^T of one 32-key sub tile: K operand ks at sk + ..., KR - 1 ahead
-        auto scores = [&](const uint8_t *sk, auto &&between) {
+        auto scores = [&](const uint8_t *sk) {
             kvm_f32x16 S;
 #pragma unroll
             for (int r = 0; r < 16; ++r) S[r] = 0.0f;
@@ -402,7 +411,6 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
                 if (ks + KR - 1 < KS) kr[(ks + KR - 1) % KR] = ld(ks + KR - 1);
                 __builtin_amdgcn_sched_barrier(0);
                 S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kr[ks % KR], qop[ks], S, 0, 0, 0);
-                between(ks);
                 PF_PIN(S);
             }
             return S;
@@ -437,7 +445,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
         // O^T += V^T P^T: operand i = (key half i / DT, dim tile i % DT); the
         // second half's probabilities are formed between the first half's MFMAs
         auto ldv = [&](const uint8_t *sv, int i) { return *(const kvm_f16x8 *)(sv + (i % DT) * 2048 + (i / DT) * 512); };
-        auto accumulate = [&](const uint8_t *sv, const kvm_f32x16 &S, float msr, kvm_f16x8 (&vr)[VR], auto &&between) {
+        auto accumulate = [&](const uint8_t *sv, const kvm_f32x16 &S, float msr, kvm_f16x8 (&vr)[VR]) {
             kvm_f16x8 pb[2];
             float sum = 0.0f;
             auto prob = [&](int r) {
@@ -458,13 +466,10 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
 #pragma unroll
                     for (int j = 0; j < 8 / DT; ++j) prob(8 + i * (8 / DT) + j);
                 }
-                between(i);
                 PF_PIN(O[i % DT]);
             }
             lp += sum;
         };
-        auto nothing = [](int) {};
-
         // Copies go global -> LDS directly (global_load_lds_dwordx4: lane l writes
         // 16 bytes at M0 + offset + 16 l), issued from asm so the compiler adds no
         // wait for them; the loops wait for them themselves before each barrier.
@@ -478,221 +483,83 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
         };
 
         if (n_t != 0) {
-            if constexpr (SRC != PF_QUANT) {
-                // Wave w copies bytes [CW w, CW (w+1)) of the tile's K and of its V in
-                // CW / 1 KB copies under one M0 value (the immediate offset moves the
-                // global and the LDS address alike).  A window's f16 V tile holds the
-                // two key halves of a dim side by side, so its copies read every
-                // second unit of a dim tile.  Wave 0 also copies the cell positions.
-                constexpr uint32_t CW = TILE_B / 8;
-                static_assert(CW == 4096 || CW == 2048, "copy layout");
-                const uint32_t wofs = __builtin_amdgcn_readfirstlane(CW * w), loff = 16u * l;
-                const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * TILE_B + wofs;
-                const uint8_t *v_head = a.v + (uint64_t)h * a.n_tiles * TILE_B +
-                                        (SRC == PF_F16 ? (w >> 2) * 16u + (w & 3) * 2u * CW : wofs);
-                const uint32_t voff = SRC == PF_F16 ? 32u * l : loff;
-                constexpr uint32_t VS = SRC == PF_F16 ? 1024u : 0u;     // global bytes a V copy moves beyond the LDS's
-                auto dma_tile = [&](uint32_t t, uint32_t buf) {
-                    const uint8_t *kb = k_head + (uint64_t)t * TILE_B, *vb = v_head + (uint64_t)t * TILE_B;
-                    const uint32_t dk = lds_mem + buf * (2 * TILE_B) + wofs, dv = dk + TILE_B;
-                    uint32_t m0_saved;
-                    if constexpr (CW == 4096) {
-                        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                                     "global_load_lds_dwordx4 %1, %5\n\t"
-                                     "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
-                                     "global_load_lds_dwordx4 %1, %5 offset:2048\n\t"
-                                     "global_load_lds_dwordx4 %1, %5 offset:3072\n\t"
-                                     "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
-                                     "global_load_lds_dwordx4 %2, %6\n\t"
-                                     "global_load_lds_dwordx4 %2, %7 offset:1024\n\t"
-                                     "global_load_lds_dwordx4 %2, %8 offset:2048\n\t"
-                                     "global_load_lds_dwordx4 %2, %9 offset:3072\n\t"
-                                     "s_mov_b32 m0, %0"
-                                     : "=&s"(m0_saved) : "v"(loff), "v"(voff), "s"(dk), "s"(dv), "s"(kb), "s"(vb),
-                                       "s"(vb + VS), "s"(vb + 2 * VS), "s"(vb + 3 * VS) : "memory");
-                    } else {
-                        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                                     "global_load_lds_dwordx4 %1, %5\n\t"
-                                     "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
-                                     "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
-                                     "global_load_lds_dwordx4 %2, %6\n\t"
-                                     "global_load_lds_dwordx4 %2, %7 offset:1024\n\t"
-                                     "s_mov_b32 m0, %0"
-                                     : "=&s"(m0_saved) : "v"(loff), "v"(voff), "s"(dk), "s"(dv), "s"(kb), "s"(vb),
-                                       "s"(vb + VS) : "memory");
-                    }
-                    if (w == 0) dma_cp(t, buf);
-                };
-                // list entries k and k+1 are in registers at the top of tile k; entry
-                // k+2 is read during tile k
-                uint32_t e_cur = entry(0), e_nxt = entry(1);
-                const uint32_t t_0 = t_begin + (__builtin_amdgcn_readfirstlane(e_cur) & 0x7fffu);
-                if constexpr (Q_EARLY) dma_tile(t_0, 0);
+            // Wave w copies bytes [CW w, CW (w+1)) of the tile's K and of its V in
+            // CW / 1 KB copies under one M0 value (the immediate offset moves the
+            // global and the LDS address alike).  A window's f16 V tile holds the
+            // two key halves of a dim side by side, so its copies read every
+            // second unit of a dim tile.  Wave 0 also copies the cell positions.
+            constexpr uint32_t CW = TILE_B / 8;
+            static_assert(CW == 4096 || CW == 2048, "copy layout");
+            const uint32_t wofs = __builtin_amdgcn_readfirstlane(CW * w), loff = 16u * l;
+            const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * TILE_B + wofs;
+            const uint8_t *v_head = a.v + (uint64_t)h * a.n_tiles * TILE_B +
+                                    (SRC == PF_F16 ? (w >> 2) * 16u + (w & 3) * 2u * CW : wofs);
+            const uint32_t voff = SRC == PF_F16 ? 32u * l : loff;
+            constexpr uint32_t VS = SRC == PF_F16 ? 1024u : 0u;     // global bytes a V copy moves beyond the LDS's
+            auto dma_tile = [&](uint32_t t, uint32_t buf) {
+                const uint8_t *kb = k_head + (uint64_t)t * TILE_B, *vb = v_head + (uint64_t)t * TILE_B;
+                const uint32_t dk = lds_mem + buf * (2 * TILE_B) + wofs, dv = dk + TILE_B;
+                uint32_t m0_saved;
+                if constexpr (CW == 4096) {
+                    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+                                 "global_load_lds_dwordx4 %1, %5\n\t"
+                                 "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
+                                 "global_load_lds_dwordx4 %1, %5 offset:2048\n\t"
+                                 "global_load_lds_dwordx4 %1, %5 offset:3072\n\t"
+                                 "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
+                                 "global_load_lds_dwordx4 %2, %6\n\t"
+                                 "global_load_lds_dwordx4 %2, %7 offset:1024\n\t"
+                                 "global_load_lds_dwordx4 %2, %8 offset:2048\n\t"
+                                 "global_load_lds_dwordx4 %2, %9 offset:3072\n\t"
+                                 "s_mov_b32 m0, %0"
+                                 : "=&s"(m0_saved) : "v"(loff), "v"(voff), "s"(dk), "s"(dv), "s"(kb), "s"(vb),
+                                   "s"(vb + VS), "s"(vb + 2 * VS), "s"(vb + 3 * VS) : "memory");
+                } else {
+                    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+                                 "global_load_lds_dwordx4 %1, %5\n\t"
+                                 "global_load_lds_dwordx4 %1, %5 offset:1024\n\t"
+                                 "s_mov_b32 m0, %4\n\ts_nop 0\n\t"
+                                 "global_load_lds_dwordx4 %2, %6\n\t"
+                                 "global_load_lds_dwordx4 %2, %7 offset:1024\n\t"
+                                 "s_mov_b32 m0, %0"
+                                 : "=&s"(m0_saved) : "v"(loff), "v"(voff), "s"(dk), "s"(dv), "s"(kb), "s"(vb),
+                                   "s"(vb + VS) : "memory");
+                }
+                if (w == 0) dma_cp(t, buf);
+            };
+            // list entries k and k+1 are in registers at the top of tile k; entry
+            // k+2 is read during tile k
+            uint32_t e_cur = entry(0), e_nxt = entry(1);
+            const uint32_t t_0 = t_begin + (__builtin_amdgcn_readfirstlane(e_cur) & 0x7fffu);
+            if constexpr (Q_EARLY) dma_tile(t_0, 0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            load_q();
+            if constexpr (!Q_EARLY) {
+                dma_tile(t_0, 0);
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                load_q();
-                if constexpr (!Q_EARLY) {
-                    dma_tile(t_0, 0);
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    KVM_LDS_BARRIER();
-                }
-                const uint32_t k_ofs = k_lane(l), v_ofs = v_lane(l);
-                for (uint32_t k = 0; k < n_t; ++k) {
-                    const uint32_t b = k & 1u;
-                    const uint32_t e = __builtin_amdgcn_readfirstlane(e_cur), en = __builtin_amdgcn_readfirstlane(e_nxt);
-                    e_cur = en;
-                    e_nxt = entry(k + 2);
-                    dma_tile(t_begin + (en & 0x7fffu), b ^ 1u);       // next tile, in flight during this one
-                    const bool masked = (e >> 15) == 0;
-                    const uint8_t *sk = s_mem + b * (2 * TILE_B) + k_ofs, *sv = s_mem + b * (2 * TILE_B) + TILE_B + v_ofs;
-                    if (active) {
-#pragma unroll
-                        for (int sub = 0; sub < 2 / KW; ++sub) {
-                            kvm_f32x16 S = scores(sk + sub * 2 * NB * 1024, nothing);
-                            kvm_f16x8 vr[VR];
-#pragma unroll
-                            for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv + sub * (TILE_B / 2), i);
-                            const float msr = settle(S, masked, &s_cp[b][32 * (KW == 2 ? kg : sub)]);
-                            accumulate(sv + sub * (TILE_B / 2), S, msr, vr, nothing);
-                        }
-                    }
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's copies
-                    __syncthreads();
-                }
-            } else {
-                // One f16 K buffer, one f16 V buffer and two buffers of quantised
-                // tiles.  Tile k in two phases, a barrier after each: scores and
-                // softmax, with V of tile k converted between the MFMAs; P V, with K of
-                // tile k + 1 converted between them.  The copies run two tiles ahead.
-                uint8_t *const s_k = s_mem, *const s_v = s_mem + TILE_B, *const s_kr = s_mem + 2 * TILE_B,
-                        *const s_vr = s_kr + 2 * KRAW_L;
-                const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * KRAW, *v_head = a.v + (uint64_t)h * a.n_tiles * VRAW;
-                auto dma_raw = [&](const uint8_t *src, uint32_t bytes, uint32_t dst, int n_kb) {
-                    for (int i = w; i < n_kb; i += 8) {
-                        const uint32_t o = 1024u * i + 16u * opaque(l);
-                        uint32_t m0_saved;
-                        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
-                                     "global_load_lds_dwordx4 %1, %3\n\ts_mov_b32 m0, %0"
-                                     : "=&s"(m0_saved) : "v"(o < bytes ? o : bytes - 16u), "s"(dst + 1024u * i), "s"(src) : "memory");
-                    }
-                };
-                auto dma_k = [&](uint32_t e, uint32_t k) {
-                    const uint32_t t = t_begin + (e & 0x7fffu);
-                    dma_raw(k_head + (uint64_t)t * KRAW, KRAW, lds_mem + 2 * TILE_B + (k & 1u) * KRAW_L, KRAW_L / 1024);
-                    if (w == 7) dma_cp(t, k & 3u);
-                };
-                auto dma_v = [&](uint32_t e, uint32_t k) {
-                    const uint32_t t = t_begin + (e & 0x7fffu);
-                    dma_raw(v_head + (uint64_t)t * VRAW, VRAW, lds_mem + 2 * TILE_B + 2 * KRAW_L + (k & 1u) * VRAW_L, VRAW_L / 1024);
-                };
-                // this wave's copies of one K and one V tile: all but the last so many
-                // are waited for before a phase ends
-                const int n_kv = (int)(KRAW_L / 1024 + 7 - w) / 8 + (w == 7) + (int)(VRAW_L / 1024 + 7 - w) / 8;
-                auto wait_copies = [&]() {
-                    if (n_kv <= 1) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
-                    else if (n_kv == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-                    else if (n_kv == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-                    else if (n_kv == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-                    else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-                };
-                // K: thread (w, l) converts the quants of (sub, block pair) CK w .., lane
-                // l, one unit a chunk; V: dim tiles CV w .., both key halves
-                constexpr int CK = NB / 4, CV = D / 128;
-                kvm_u32x4 ck;
-                uint32_t cd[2];
-                auto k_read = [&](const uint8_t *raw, int i) {
-                    const uint32_t ln = opaque(l), sp = CK * w + i, s = sp / (NB / 2), pr = sp % (NB / 2), m = ln & 15;
-                    ck = *(const kvm_u32x4 *)(raw + (sp * 64 + ln) * 16);
-                    cd[0] = *(const uint16_t *)(raw + kvm_kd_off(D, 16 * s + m, 2 * pr));
-                    cd[1] = *(const uint16_t *)(raw + kvm_kd_off(D, 16 * s + m, 2 * pr + 1));
-                };
-                auto k_write = [&](int i, int j) {
-                    const uint32_t sp = CK * w + i, s = sp / (NB / 2), pr = sp % (NB / 2);
-                    *(kvm_f16x8 *)(s_k + ((s * NB + 2 * pr + j) * 64 + opaque(l)) * 16) = pf_q8(ck[2 * j], ck[2 * j + 1], cd[j]);
-                };
-                kvm_u32x2 cv[CV];
-                kvm_u32x4 cs;
-                auto v_read = [&](const uint8_t *raw, int ks) {
-                    const uint32_t ln = opaque(l);
-                    if (ks == 0) {
-#pragma unroll
-                        for (int i = 0; i < CV; ++i) cv[i] = *(const kvm_u32x2 *)(raw + ((CV * w + i) * 64 + ln) * 8);
-                    }
-                    cs = *(const kvm_u32x4 *)(raw + 32 * D + (((CV * w) >> 1) * 8 + ks * 4 + (ln >> 4)) * 16);
-                };
-                auto v_write = [&](int i, int ks) {
-                    *(kvm_f16x8 *)(s_v + ks * (TILE_B / 2) + ((CV * w + i) * 64 + opaque(l)) * 16) = pf_q4(cv[i][ks], cs);
-                };
-                // steps of a conversion between the MFMAs (16 at D 256, 8 at 128)
-                auto conv_v = [&](const uint8_t *raw, int i) {
-                    constexpr int Q = KS / (2 * CV + 1);          // MFMAs between two writes
-                    if (i == 0) v_read(raw, 0);
-#pragma unroll
-                    for (int n = 0; n < 2 * CV; ++n)
-                        if (i == Q * (n + 1)) v_write(n % CV, n / CV);
-                    if (i == Q * CV) v_read(raw, 1);
-                };
-                auto conv_k = [&](const uint8_t *raw, int i) {
-                    constexpr int Q = KS / CK;                    // MFMAs of a chunk
-                    const int n = i / Q, o = i % Q;
-                    if (o == 0) k_read(raw, n);
-                    if (o == Q / 2) k_write(n, 0);
-                    if (o == Q / 2 + 2) k_write(n, 1);
-                };
-
-                if constexpr (!Q_EARLY) {
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    load_q();
-                }
-                // list entries of tiles k .. k + 2, and k + 3's on its way
-                auto ent = [&](uint32_t k) { return (uint32_t)__builtin_amdgcn_readfirstlane(entry(k)); };
-                uint32_t e0 = ent(0), e1 = ent(1), e2 = ent(2), e_far = entry(3);
-                dma_k(e0, 0);
-                dma_v(e0, 0);
-                dma_k(e1, 1);
-                dma_v(e1, 1);
-                wait_copies();                            // Q's too: they are older
-                if constexpr (Q_EARLY) load_q();
-                else KVM_LDS_BARRIER();
-#pragma unroll
-                for (int i = 0; i < CK; ++i) {
-                    k_read(s_kr, i);
-                    k_write(i, 0);
-                    k_write(i, 1);
-                }
                 KVM_LDS_BARRIER();
-                for (uint32_t k = 0; k < n_t; ++k) {
-                    const uint32_t b = k & 1u;
-                    const bool masked = (e0 >> 15) == 0;
-                    dma_k(e2, k + 2);
-                    const uint8_t *vraw = s_vr + b * VRAW_L, *kraw = s_kr + (b ^ 1u) * KRAW_L;
-                    if (active) {
-                        kvm_f32x16 S = scores(s_k + k_lane(opaque(l)), [&](int i) { conv_v(vraw, i); });
-                        const float msr = settle(S, masked, &s_cp[k & 3u][32 * kg]);
-                        wait_copies();
-                        KVM_LDS_BARRIER();
-                        dma_v(e2, k + 2);
-                        const uint8_t *sv = s_v + v_lane(opaque(l));
+            }
+            const uint32_t k_ofs = k_lane(l), v_ofs = v_lane(l);
+            for (uint32_t k = 0; k < n_t; ++k) {
+                const uint32_t b = k & 1u;
+                const uint32_t e = __builtin_amdgcn_readfirstlane(e_cur), en = __builtin_amdgcn_readfirstlane(e_nxt);
+                e_cur = en;
+                e_nxt = entry(k + 2);
+                dma_tile(t_begin + (en & 0x7fffu), b ^ 1u);       // next tile, in flight during this one
+                const bool masked = (e >> 15) == 0;
+                const uint8_t *sk = s_mem + b * (2 * TILE_B) + k_ofs, *sv = s_mem + b * (2 * TILE_B) + TILE_B + v_ofs;
+                if (active) {
+#pragma unroll
+                    for (int sub = 0; sub < 2; ++sub) {
+                        kvm_f32x16 S = scores(sk + sub * 2 * NB * 1024);
                         kvm_f16x8 vr[VR];
 #pragma unroll
-                        for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv, i);
-                        accumulate(sv, S, msr, vr, [&](int i) { conv_k(kraw, i); });
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < KS; ++i) conv_v(vraw, i);
-                        wait_copies();
-                        KVM_LDS_BARRIER();
-                        dma_v(e2, k + 2);
-#pragma unroll
-                        for (int i = 0; i < KS; ++i) conv_k(kraw, i);
+                        for (int i = 0; i < VR - 1; ++i) vr[i] = ldv(sv + sub * (TILE_B / 2), i);
+                        const float msr = settle(S, masked, &s_cp[b][32 * sub]);
+                        accumulate(sv + sub * (TILE_B / 2), S, msr, vr);
                     }
-                    e0 = e1;
-                    e1 = e2;
-                    e2 = __builtin_amdgcn_readfirstlane(e_far);
-                    e_far = entry(k + 4);
-                    wait_copies();
-                    KVM_LDS_BARRIER();
                 }
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the copies past the last tile
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's copies
                 __syncthreads();
             }
         }
@@ -702,65 +569,388 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
             KVM_LDS_BARRIER();
         }
 
-        // ---- results: O's quads i0 .. i0 + N - 1 (quad i: dims 8 i + 4 g2 .. + 3 of the lane's row)
-        float lr = kvm_add_xor32(lp);
+        // ---- results: quad i of O: dims 8 i + 4 g2 .. + 3 of the lane's row.  (The lane
+        // and its row are formed again here: kept through the loop they take registers
+        // that O needs.)
+        const float lr = kvm_add_xor32(lp);
+        const uint32_t le = opaque(l), me = le & 31u, ge = le >> 5, row_e = rt_i * ROWS + 32 * w + me;
         auto quad = [&](int i) {
             return kvm_f32x4{O[i >> 2][4 * (i & 3)], O[i >> 2][4 * (i & 3) + 1], O[i >> 2][4 * (i & 3) + 2], O[i >> 2][4 * (i & 3) + 3]};
         };
-        // (the lane and its row are formed again here: kept through the loop they
-        // take registers that O needs)
-        const uint32_t le = opaque(l), me = le & 31u, ge = le >> 5, row_e = rt_i * ROWS + 32 * rg + me;
-        auto finish = [&](auto i0_, auto n_, float w0, const float *other, float w1, bool ml) {
-            constexpr int I0 = decltype(i0_)::value, N = decltype(n_)::value;
-            const uint64_t slot = 2 * (uint64_t)p + (u != u_first);
-            const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
-            float *o = whole ? a.out + ((uint64_t)(row_e / a.G) * a.n_head + h * a.G + row_e % a.G) * D + 4 * ge
-                             : a.ws_o + (slot * ROWS + 32 * rg) * D + 4 * le;
-            const uint32_t os = whole ? 8u : 256u;
-            if (whole ? row_e < a.n_rows : rt_i * ROWS + 32 * rg < a.n_rows) {
+        if (whole) {
+            if (row_e < a.n_rows) {
+                const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
+                float *o = a.out + ((uint64_t)(row_e / a.G) * a.n_head + h * a.G + row_e % a.G) * D + 4 * ge;
 #pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    kvm_f32x4 x = quad(I0 + i);
-                    if constexpr (KW == 2) x = x * w0 + *(const kvm_f32x4 *)(other + 256 * i) * w1;
-                    if (whole) x *= inv;
-                    *(kvm_f32x4 *)(o + os * (I0 + i)) = x;
+                for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = quad(i) * inv;
+            }
+        } else if (active) {
+            const uint64_t slot = 2 * (uint64_t)p + (u != u_first);
+            float *o = a.ws_o + (slot * ROWS + 32 * w) * D + 4 * le;
+#pragma unroll
+            for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 256 * i) = quad(i);
+            if (ge == 0) {
+                float *o_ml = a.ws_ml + (slot * ROWS + 32 * w + me) * 2;
+                o_ml[0] = ms;
+                o_ml[1] = lr;
+            }
+        }
+        if (u != u_last) __syncthreads();       // the LDS is the next piece's
+    }
+}
+
+// Units of 128 rows, two roles.  Waves 0 - 3, one a SIMD, have 32 rows each and take
+// every key of a tile; waves 4 - 7 bring tile k + 1 into one LDS buffer while tile k in
+// the other is worked on, one barrier a tile: an f16 window's by copies, a quantised
+// one's through registers, loaded two tiles ahead and written as f16 operands.  What bounds it is the attention waves'
+// chain (~3,900 cycles a tile of 256 dims, of which 2,048 on the matrix cores): the
+// softmax of a 32-key sub tile is taken between the MFMAs of the next scores or of
+// the P V before.  (Converting between the MFMAs of eight attention waves took 5,300:
+// their LDS writes, 64 bytes a cycle, held up the operand reads.  37 tokens x 32,768
+// cells 61.6 -> 54 us, 64 x 4,096 of 8 heads x 128 28 -> 22.5.)
+template <int D, int SRC, bool BF16>
+__global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
+    constexpr int ROWS = 128;
+    constexpr int KS = D / 16, DT = D / 32, NB = D / 32;  // k-steps of a score; MFMAs of a sub tile's P V: 2 DT = KS
+    constexpr uint32_t TILE_B = 128u * D;                 // bytes of an f16 K (or V) tile
+    constexpr uint32_t KRAW = 64u * D + 64u * NB * 2u, VRAW = 32u * D + NB * 128u;    // quantised tiles
+    constexpr uint32_t MEM = 4u * TILE_B;                 // two K/V buffers
+    constexpr uint32_t Q_UNITS = D * (BF16 ? 2 : 4) / 16, Q_UC = Q_UNITS;
+    constexpr bool Q_EARLY = Q_UNITS * ROWS * 16 <= 2 * TILE_B;      // Q fits beside the first tile
+    constexpr uint32_t Q_OFS = Q_EARLY ? 2 * TILE_B : 0;
+    static_assert(Q_UNITS * ROWS * 16 <= MEM, "Q in LDS");
+    // Operand rings: R1 where a softmax is under way (registers), R0 elsewhere.  At
+    // 256 dims there are none left to keep the softmax's steps where they are
+    // written, so the compiler gathers the exponentials.
+    constexpr std::integral_constant<int, 6> R0;
+    constexpr std::integral_constant<int, D == 256 ? 2 : 4> R1;
+    constexpr bool PINS = D == 128;
+    __shared__ __align__(16) uint8_t s_mem[MEM];
+    __shared__ pf_front s_front;
+    __shared__ __align__(16) int32_t s_cp[2][64];         // the tiles' cell positions
+    const int tid = threadIdx.x, l = tid & 63, g2 = l >> 5, m2 = l & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), rg = w & 3;
+    const bool consumer = w < 4;
+    const uint32_t lds_mem = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_mem[0];
+    uint32_t p = blockIdx.x;
+    if ((a.P & 7u) == 0) p = (p & 7u) * (a.P >> 3) + (p >> 3);       // as k_pf_attn
+    const uint32_t sh0 = p * a.U, sh1 = sh0 + a.U;
+    const uint32_t u_first = sh0 / a.P, u_last = (sh1 - 1) / a.P;
+
+    for (uint32_t u = u_first; u <= u_last; ++u) {
+        const uint32_t u0 = u * a.P;
+        const uint32_t f_lo = max(sh0, u0) - u0, f_hi = min(sh1 - u0, a.P);
+        const uint32_t seg = u % a.n_seg, rest = u / a.n_seg;
+        const uint32_t rt_i = __builtin_amdgcn_readfirstlane(rest % a.n_row_tiles), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
+        const bool whole = f_lo == 0 && f_hi == a.P && a.n_seg == 1;
+        const uint32_t row = rt_i * ROWS + 32 * rg + m2;
+        const uint32_t t_begin = seg * KVM_PF_LIST;
+        uint32_t qlim;
+        const uint32_t n_t = pf_tiles<false>(a, row, t_begin, f_lo, f_hi, s_front, qlim, [&]() {
+            pf_copy_q<D, ROWS, Q_UC, BF16>(a, rt_i, h, 0, lds_mem + Q_OFS, w, l);
+        });
+        // Both roles take the same barriers: one when Q is in LDS (two if the first
+        // tile has to wait for it to be read), one when the first tile is ready, and
+        // one a tile.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        KVM_LDS_BARRIER();
+        if (consumer) {
+            // ======== consumers: S^T = K Q^T, softmax, O^T += V^T P^T of 32 rows
+            const float c = a.c;
+            kvm_f32x16 O[DT];
+            float ms = -INFINITY, lp = 0.0f;        // running max of the row (times c), lane's share of its sum
+            // Q rows as f16 B operands: lane (g2, m2) holds Q[row m2][16ks + 8 g2 .. +7]
+            kvm_f16x8 qop[KS];
+            {
+                const uint32_t lq = opaque(l), r = 32 * rg + (lq & 31u), sw = r % Q_UNITS;
+                const uint8_t *qr = s_mem + Q_OFS + r * (Q_UNITS * 16);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    kvm_u32x4 x[BF16 ? 1 : 2];
+#pragma unroll
+                    for (int j = 0; j < (BF16 ? 1 : 2); ++j)
+                        x[j] = *(const kvm_u32x4 *)(qr + ((((BF16 ? 1 : 2) * (2 * ks + (lq >> 5)) + j) ^ sw) * 16));
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const uint32_t y = x[BF16 ? 0 : j >> 2][BF16 ? j >> 1 : j & 3];
+                        qop[ks][j] = (_Float16)__uint_as_float(!BF16 ? y : j & 1 ? y & 0xffff0000u : y << 16);
+                    }
                 }
-                if (ml && !whole && ge == 0) {
+            }
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) O[dt][r] = 0.0f;
+            // operand addresses of a lane: K row m2 is key m2 with bits 2 and 3 swapped
+            const uint32_t key = (m2 & 0x13) | (m2 & 4) << 1 | (m2 & 8) >> 1;
+            const uint32_t k_ofs = ((key >> 4) * NB * 64 + 16 * g2 + (key & 15)) * 16;
+            const uint32_t v_ofs = ((m2 >> 4) * 64 + 16 * g2 + (m2 & 15)) * 16;
+            if constexpr (!Q_EARLY) KVM_LDS_BARRIER();
+
+            // S^T of one 32-key sub tile: K operand ks at sk + ..., KR - 1 ahead;
+            // between(ks) follows MFMA ks
+            auto scores = [&](auto ring, const uint8_t *sk, auto &&between) {
+                constexpr int KR = decltype(ring)::value;
+                kvm_f32x16 S;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) S[r] = 0.0f;
+                kvm_f16x8 kr[KR];
+                auto ld = [&](int ks) { return *(const kvm_f16x8 *)(sk + (ks >> 1) * 1024 + (ks & 1) * 512); };
+#pragma unroll
+                for (int i = 0; i < KR - 1; ++i) kr[i] = ld(i);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    if (ks + KR - 1 < KS) kr[(ks + KR - 1) % KR] = ld(ks + KR - 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kr[ks % KR], qop[ks], S, 0, 0, 0);
+                    between(ks);
+                    PF_PIN(S);
+                }
+                return S;
+            };
+            // O^T += V^T P^T: operand i = (key half i / DT, dim tile i % DT)
+            auto accumulate = [&](auto ring, const uint8_t *sv, const kvm_f16x8 (&pb)[2], auto &&between) {
+                constexpr int VR = decltype(ring)::value;
+                kvm_f16x8 vr[VR];
+                auto ld = [&](int i) { return *(const kvm_f16x8 *)(sv + (i % DT) * 2048 + (i / DT) * 512); };
+#pragma unroll
+                for (int i = 0; i < VR - 1; ++i) vr[i] = ld(i);
+#pragma unroll
+                for (int i = 0; i < 2 * DT; ++i) {
+                    if (i + VR - 1 < 2 * DT) vr[(i + VR - 1) % VR] = ld(i + VR - 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    O[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vr[i % VR], pb[i / DT], O[i % DT], 0, 0, 0);
+                    between(i);
+                    PF_PIN(O[i % DT]);
+                }
+            };
+            auto mask = [&](kvm_f32x16 &S, const int32_t *cp) {
+                asm volatile("" ::: "memory");            // keep the mask on this (rare) path
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const kvm_u32x4 x = *(const kvm_u32x4 *)(cp + 16 * (i >> 1) + 8 * (opaque(l) >> 5) + 4 * (i & 1));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (!(x[r] < qlim)) S[4 * i + r] = -INFINITY;
+                }
+            };
+            // The softmax of a sub tile in KS steps, taken between another's MFMAs:
+            // the maximum (KS / 4 steps), the running maximum's move (one step), the
+            // probabilities (KS / 2 steps).
+            float x = 0.0f, msr = 0.0f, alpha = 1.0f, sum = 0.0f;
+            bool moved = false;
+            auto soft = [&](const kvm_f32x16 &S, kvm_f16x8 (&pb)[2], int i) {
+                constexpr int NM = KS / 4, EM = 16 / NM, EP = 16 / (KS / 2);
+                if (i < NM) {
+#pragma unroll
+                    for (int r = 0; r < EM; ++r) x = i == 0 && r == 0 ? S[0] : fmaxf(x, S[EM * i + r]);
+                    if constexpr (PINS) asm volatile("" : "+v"(x));
+                } else if (i == NM) {
+                    x = kvm_max_xor32(x);
+                    const bool up = fmaf(x, c, -ms) > KVM_PF_LAZY;   // false for a row with nothing visible yet
+                    moved = __builtin_amdgcn_ballot_w64(up) != 0;
+                    const float mnew = up ? x * c : ms;
+                    alpha = up ? __builtin_amdgcn_exp2f(ms - mnew) : 1.0f;
+                    ms = mnew;
+                    msr = ms == -INFINITY ? 0.0f : ms;
+                    sum = 0.0f;
+                } else if (i >= KS / 2) {
+#pragma unroll
+                    for (int j = 0; j < EP; ++j) {
+                        // the row sum takes p before its rounding to the fp16 operand:
+                        // within 2^-11 of it per element
+                        const int r = EP * (i - KS / 2) + j;
+                        const float y = __builtin_amdgcn_exp2f(fmaf(S[r], c, -msr));
+                        pb[r >> 3][r & 7] = (_Float16)y;
+                        sum += y;
+                        if constexpr (PINS) asm volatile("" : "+v"(sum));
+                    }
+                    if constexpr (PINS) asm volatile("" : "+v"(pb[(EP * (i - KS / 2)) >> 3]));
+                }
+            };
+            // what the moved maximum asks of the sums so far
+            auto settle = [&]() {
+                if (moved) {
+                    asm volatile("" ::: "memory");        // keep it on this (rare) path
+                    lp *= alpha;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) O[dt] *= alpha;
+                }
+                lp += sum;
+            };
+            auto nothing = [](int) {};
+
+            KVM_LDS_BARRIER();                            // the first tile is in LDS
+            const bool active = rt_i * ROWS + 32u * rg < a.n_rows;    // not a wave of padding rows
+            uint32_t e_nxt = n_t ? s_front.list[0] : 0u;
+            for (uint32_t k = 0; k < n_t; ++k) {
+                if (!active) {
+                    KVM_LDS_BARRIER();
+                    continue;
+                }
+                const bool masked = (__builtin_amdgcn_readfirstlane(e_nxt) >> 15) == 0;
+                e_nxt = s_front.list[k + 1 < n_t ? k + 1 : k];
+                const uint8_t *sk = s_mem + (k & 1u) * (2 * TILE_B) + k_ofs, *sv = s_mem + (k & 1u) * (2 * TILE_B) + TILE_B + v_ofs;
+                kvm_f16x8 pb[2];
+                kvm_f32x16 S0 = scores(R0, sk, nothing);
+                if (masked) mask(S0, &s_cp[k & 1u][0]);
+                kvm_f32x16 S1 = scores(R1, sk + 2 * NB * 1024, [&](int i) { soft(S0, pb, i); });
+                settle();
+                if (masked) mask(S1, &s_cp[k & 1u][32]);
+                kvm_f16x8 pb1[2];
+                accumulate(R1, sv, pb, [&](int i) { soft(S1, pb1, i); });
+                settle();
+                accumulate(R0, sv + TILE_B / 2, pb1, nothing);
+                KVM_LDS_BARRIER();
+            }
+            // ---- results: quad i of O: dims 8 i + 4 g2 .. + 3 of the lane's row
+            const float lr = kvm_add_xor32(lp);
+            const uint32_t le = opaque(l), me = le & 31u, ge = le >> 5, row_e = rt_i * ROWS + 32 * rg + me;
+            auto quad = [&](int i) {
+                return kvm_f32x4{O[i >> 2][4 * (i & 3)], O[i >> 2][4 * (i & 3) + 1], O[i >> 2][4 * (i & 3) + 2], O[i >> 2][4 * (i & 3) + 3]};
+            };
+            if (whole) {
+                if (row_e < a.n_rows) {
+                    const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
+                    float *o = a.out + ((uint64_t)(row_e / a.G) * a.n_head + h * a.G + row_e % a.G) * D + 4 * ge;
+#pragma unroll
+                    for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = quad(i) * inv;
+                }
+            } else if (rt_i * ROWS + 32 * rg < a.n_rows) {
+                const uint64_t slot = 2 * (uint64_t)p + (u != u_first);
+                float *o = a.ws_o + (slot * ROWS + 32 * rg) * D + 4 * le;
+#pragma unroll
+                for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 256 * i) = quad(i);
+                if (ge == 0) {
                     float *o_ml = a.ws_ml + (slot * ROWS + 32 * rg + me) * 2;
                     o_ml[0] = ms;
                     o_ml[1] = lr;
                 }
             }
-        };
-        constexpr std::integral_constant<int, 0> first;
-        if constexpr (KW == 1) {
-            finish(first, std::integral_constant<int, DT * 4>{}, 1.0f, nullptr, 0.0f, true);
         } else {
-            // the key groups of 32 rows merge through LDS: each hands the other one
-            // half of its dims
-            constexpr std::integral_constant<int, DT * 2> half;
-            float *const s_o = (float *)s_mem + 4 * le;
-            auto give = [&](auto i0_) {
+            // ======== producers: tile k + 1 into one buffer while the consumers work
+            // on tile k in the other
+            const int pw = w - 4;
+            auto tile = [&](uint32_t k) { return t_begin + (__builtin_amdgcn_readfirstlane((uint32_t)s_front.list[k < n_t ? k : n_t - 1]) & 0x7fffu); };
+            auto cells_to = [&](uint32_t t) { return a.cell_pos[(uint64_t)t * 64 + l]; };
+            if constexpr (SRC != PF_QUANT) {
+                // Copies go global -> LDS directly (global_load_lds_dwordx4: lane l
+                // writes 16 bytes at M0 + 16 l), issued from asm so the compiler adds
+                // no wait for them; the wait is before the barrier.  The asm restores
+                // M0, which the compiler reserves.  A window's f16 V tile holds the two
+                // key halves of a dim side by side, so its copies read every second
+                // unit of a dim tile.
+                constexpr int NC = (int)TILE_B / 4096;    // 1 KB copies of a wave, of K and of V
+                const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * TILE_B, *v_head = a.v + (uint64_t)h * a.n_tiles * TILE_B;
+                auto copy = [&](uint32_t voff, uint32_t dst, const uint8_t *src) {
+                    uint32_t m0_saved;
+                    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                                 "global_load_lds_dwordx4 %1, %3\n\ts_mov_b32 m0, %0"
+                                 : "=&s"(m0_saved) : "v"(voff), "s"(dst), "s"(src) : "memory");
+                };
+                auto copy_tile = [&](uint32_t t, uint32_t buf) {
+                    const uint32_t dst = lds_mem + buf * (2 * TILE_B);
+                    const uint8_t *kt = k_head + (uint64_t)t * TILE_B, *vt = v_head + (uint64_t)t * TILE_B;
 #pragma unroll
-                for (int i = 0; i < DT * 2; ++i) *(kvm_f32x4 *)(s_o + (w * DT * 2 + i) * 256) = quad(decltype(i0_)::value + i);
-            };
-            if (kg == 0) give(half);
-            else give(first);
-            if (ge == 0) {
-                s_ml[w][me][0] = ms;
-                s_ml[w][me][1] = lr;
+                    for (int i = 0; i < NC; ++i) copy(16u * opaque(l), dst + (pw * NC + i) * 1024u, kt + (pw * NC + i) * 1024u);
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        const uint32_t x = pw * NC + i;   // key half, dim tile
+                        const uint8_t *src = SRC == PF_F16 ? vt + (x % (D / 16)) * 2048u + (x / (D / 16)) * 16u : vt + x * 1024u;
+                        copy((SRC == PF_F16 ? 32u : 16u) * opaque(l), dst + TILE_B + x * 1024u, src);
+                    }
+                };
+                if constexpr (!Q_EARLY) KVM_LDS_BARRIER();
+                if (n_t != 0) {
+                    const uint32_t t = tile(0);
+                    copy_tile(t, 0);
+                    if (pw == 0) s_cp[0][l] = cells_to(t);
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
+                KVM_LDS_BARRIER();
+                for (uint32_t k = 0; k < n_t; ++k) {
+                    if (k + 1 < n_t) {
+                        const uint32_t t = tile(k + 1);
+                        copy_tile(t, (k + 1) & 1u);
+                        if (pw == 0) s_cp[(k + 1) & 1u][l] = cells_to(t);
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    }
+                    KVM_LDS_BARRIER();
+                }
+            } else {
+                // The quantised tile goes through registers (two sets: tiles k + 2 and
+                // k + 3 are in flight while tile k + 1 is converted).  Thread (pw, l): K
+                // units 4 j + pw (lane l of (sub, block pair)), V dim tiles VJ pw + j.
+                constexpr int KJ = D / 64, VJ = D / 64, VB = VJ / 2;
+                struct raw_tile {
+                    kvm_u32x4 k[KJ];
+                    uint32_t kd[KJ][2];
+                    kvm_u32x2 v[VJ];
+                    kvm_u32x4 vs[VB][2];
+                    int32_t cp;
+                };
+                raw_tile rt[2] = {};
+                const uint8_t *k_head = a.k + (uint64_t)h * a.n_tiles * KRAW, *v_head = a.v + (uint64_t)h * a.n_tiles * VRAW;
+                auto load = [&](raw_tile &r, uint32_t t) {
+                    const uint32_t ln = opaque(l);
+                    const uint8_t *kt = k_head + (uint64_t)t * KRAW, *vt = v_head + (uint64_t)t * VRAW;
+#pragma unroll
+                    for (int j = 0; j < KJ; ++j) {
+                        const uint32_t sp = 4 * j + pw, s = sp / (NB / 2), pr = sp % (NB / 2);
+                        r.k[j] = *(const kvm_u32x4 *)(kt + (sp * 64 + ln) * 16);
+                        r.kd[j][0] = *(const uint16_t *)(kt + kvm_kd_off(D, 16 * s + (ln & 15), 2 * pr));
+                        r.kd[j][1] = *(const uint16_t *)(kt + kvm_kd_off(D, 16 * s + (ln & 15), 2 * pr + 1));
+                    }
+#pragma unroll
+                    for (int j = 0; j < VJ; ++j) r.v[j] = *(const kvm_u32x2 *)(vt + ((VJ * pw + j) * 64 + ln) * 8);
+#pragma unroll
+                    for (int b = 0; b < VB; ++b)
+#pragma unroll
+                        for (int ks = 0; ks < 2; ++ks)
+                            r.vs[b][ks] = *(const kvm_u32x4 *)(vt + 32 * D + (((VB * pw + b) * 2 + ks) * 4 + (ln >> 4)) * 16);
+                    r.cp = cells_to(t);
+                };
+                auto convert = [&](const raw_tile &r, uint32_t buf) {
+                    uint8_t *dk = s_mem + buf * (2 * TILE_B) + 16 * opaque(l), *dv = dk + TILE_B;
+#pragma unroll
+                    for (int j = 0; j < KJ; ++j) {
+                        const uint32_t sp = 4 * j + pw, s = sp / (NB / 2), pr = sp % (NB / 2);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            *(kvm_f16x8 *)(dk + (s * NB + 2 * pr + i) * 1024) = pf_q8(r.k[j][2 * i], r.k[j][2 * i + 1], r.kd[j][i]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < VJ; ++j)
+#pragma unroll
+                        for (int ks = 0; ks < 2; ++ks)
+                            *(kvm_f16x8 *)(dv + ks * (TILE_B / 2) + (VJ * pw + j) * 1024) = pf_q4(r.v[j][ks], r.vs[j / 2][ks]);
+                    if (pw == 0) s_cp[buf][l] = r.cp;
+                };
+                if (n_t != 0) {
+                    load(rt[0], tile(0));
+                    load(rt[1], tile(1));
+                }
+                if constexpr (!Q_EARLY) KVM_LDS_BARRIER();
+                if (n_t != 0) {
+                    convert(rt[0], 0);
+                }
+                KVM_LDS_BARRIER();
+                if (2 < n_t) load(rt[0], tile(2));
+                auto step = [&](raw_tile &r, uint32_t k) {
+                    if (k + 1 < n_t) convert(r, (k + 1) & 1u);
+                    if (k + 3 < n_t) load(r, tile(k + 3));
+                    KVM_LDS_BARRIER();
+                };
+                uint32_t k = 0;
+                for (; k + 2 <= n_t; k += 2) {
+                    step(rt[1], k);
+                    step(rt[0], k + 1);
+                }
+                if (k < n_t) step(rt[1], k);
             }
-            KVM_LDS_BARRIER();
-            const float m1 = s_ml[w ^ 1][me][0], l1 = s_ml[w ^ 1][me][1], M = fmaxf(ms, m1);
-            const float w0 = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-            const float w1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
-            lr = lr * w0 + l1 * w1;
-            ms = M;
-            const float *other = s_o + (w ^ 1) * DT * 2 * 256;
-            if (kg == 0) finish(first, half, w0, other, w1, true);
-            else finish(half, half, w0, other, w1, false);
         }
-        if (u != u_last) __syncthreads();       // s_mem, s_mm and s_ml are reused by the next piece
+
+        if (u != u_last) __syncthreads();       // the LDS is the next piece's
     }
 }
 
@@ -768,9 +958,9 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
 // share the pieces, each with NP pieces' loads in flight, and meet in LDS: what
 // bounds a unit of many pieces is the round trips of its loads (32 pieces of 128
 // rows x 256 dims: 8.1 us with one wave, four trips).
-template <int D, int KW, int WS, int NP>
+template <int D, int ROWS, int WS, int NP>
 __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
-    constexpr uint32_t RG = 8 / KW, ROWS = 32 * RG, IB = 4 / WS;
+    constexpr uint32_t IB = 4 / WS;
     const uint32_t l = threadIdx.x & 63u, wv = threadIdx.x >> 6, ws = wv % WS, i = blockIdx.x * IB + wv / WS;
     const uint32_t rg = blockIdx.y, m2 = l & 31u, rt_i = blockIdx.z % a.n_row_tiles, h = blockIdx.z / a.n_row_tiles;
     const uint32_t row = rt_i * ROWS + 32 * rg + m2;
@@ -836,33 +1026,38 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     *(kvm_f32x4 *)(a.out + ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + 8 * i + 4 * (l >> 5)) = acc * inv;
 }
 
-template <int D, int KW, int SRC>
+template <int D, int ROWS, int SRC>
 static void pf_attn(const pf_args &a, hipStream_t stream) {
-    if (a.q_bf16) hipLaunchKernelGGL((k_pf_attn<D, KW, SRC, true>), dim3(a.P), dim3(512), 0, stream, a);
-    else hipLaunchKernelGGL((k_pf_attn<D, KW, SRC, false>), dim3(a.P), dim3(512), 0, stream, a);
+    auto go = [&](auto bf16) {
+        constexpr bool B = decltype(bf16)::value;
+        if constexpr (ROWS == 256) hipLaunchKernelGGL((k_pf_attn<D, SRC, B>), dim3(a.P), dim3(512), 0, stream, a);
+        else hipLaunchKernelGGL((k_pf_attn_split<D, SRC, B>), dim3(a.P), dim3(512), 0, stream, a);
+    };
+    if (a.q_bf16) go(std::true_type{});
+    else go(std::false_type{});
     if (a.n_seg == 1 && a.U % a.P == 0) return;           // every unit whole
-    const dim3 g1(D / 32, 8 / KW, a.n_row_tiles * a.H), g4(D / 8, 8 / KW, a.n_row_tiles * a.H), t(256);
+    const dim3 g1(D / 32, ROWS / 32, a.n_row_tiles * a.H), g4(D / 8, ROWS / 32, a.n_row_tiles * a.H), t(256);
     // most pieces of a unit (of one of its segments)
     const uint32_t n = a.P % a.U == 0 ? a.P / a.U : a.P / a.U + 2;
-    if (n <= 2) hipLaunchKernelGGL((k_pf_combine<D, KW, 1, 2>), g1, t, 0, stream, a);
-    else if (n <= 4) hipLaunchKernelGGL((k_pf_combine<D, KW, 1, 4>), g1, t, 0, stream, a);
-    else if (n <= 8) hipLaunchKernelGGL((k_pf_combine<D, KW, 1, 8>), g1, t, 0, stream, a);
-    else if (n <= 16) hipLaunchKernelGGL((k_pf_combine<D, KW, 4, 4>), g4, t, 0, stream, a);
-    else hipLaunchKernelGGL((k_pf_combine<D, KW, 4, 8>), g4, t, 0, stream, a);
+    if (n <= 2) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 1, 2>), g1, t, 0, stream, a);
+    else if (n <= 4) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 1, 4>), g1, t, 0, stream, a);
+    else if (n <= 8) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 1, 8>), g1, t, 0, stream, a);
+    else if (n <= 16) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 4, 4>), g4, t, 0, stream, a);
+    else hipLaunchKernelGGL((k_pf_combine<D, ROWS, 4, 8>), g4, t, 0, stream, a);
 }
 
 template <int D>
-static void pf_launch(const pf_args &a, const pf_stage_args &sa, int src, int kw, hipStream_t stream) {
-    if (src == PF_QUANT) return pf_attn<D, 2, PF_QUANT>(a, stream);
-    if (src == PF_F16) return kw == 1 ? pf_attn<D, 1, PF_F16>(a, stream) : pf_attn<D, 2, PF_F16>(a, stream);
+static void pf_launch(const pf_args &a, const pf_stage_args &sa, int src, uint32_t rows, hipStream_t stream) {
+    if (src == PF_QUANT) return pf_attn<D, 128, PF_QUANT>(a, stream);
+    if (src == PF_F16) return rows == 256 ? pf_attn<D, 256, PF_F16>(a, stream) : pf_attn<D, 128, PF_F16>(a, stream);
     hipLaunchKernelGGL(k_pf_stage<D>, dim3(sa.n_tiles, a.H), dim3(256), 0, stream, sa);
-    return kw == 1 ? pf_attn<D, 1, PF_STAGED>(a, stream) : pf_attn<D, 2, PF_STAGED>(a, stream);
+    pf_attn<D, 256, PF_STAGED>(a, stream);
 }
 
 // ---- the launch's shape, from measured costs (us; D 256, half of it at D 128)
 // A 64-cell tile of a unit.
-static double pf_tile_us(uint32_t D, int kw, int src) {
-    return (kw == 1 ? 3.3 : src == PF_QUANT ? 2.3 : 1.55) * D / 256;
+static double pf_tile_us(uint32_t D, int src, uint32_t rows) {
+    return (rows == 256 ? 3.3 : src == PF_QUANT ? 1.75 : 1.6) * D / 256;
 }
 
 // Workgroups that U units of n_tiles tiles are dealt to, at most one per CU (LDS).
@@ -873,7 +1068,7 @@ static double pf_tile_us(uint32_t D, int kw, int src) {
 // once more, `piece` us of all (500 tokens over 16 tiles of 128 dims, 32 units:
 // 30.2 us in 256 pieces, 22.8 in 128).
 #define PF_START 8.0
-static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double t, double piece, uint32_t n_cu, double *cost) {
+static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double t, double piece, uint32_t n_cu) {
     double best = PF_START + t * n_tiles * U / n_cu + piece * (U < n_cu ? n_cu + U : 2.0 * n_cu);
     uint32_t P = n_cu;
     for (uint64_t s = 1; s * U <= n_cu && s <= n_tiles; ++s) {
@@ -883,7 +1078,6 @@ static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double t, double piece, 
             P = (uint32_t)(s * U);
         }
     }
-    if (cost) *cost = best;
     return P;
 }
 // A piece's partial output, written and read at the rate that such launches reach.
@@ -891,31 +1085,13 @@ static double pf_piece_us(uint32_t D, uint64_t n_rows, uint32_t row_tiles) {
     return (double)n_rows / row_tiles * D * 8 / 3.2e6;
 }
 
-// Row groups that share a tile, and where a quantised window is converted.
-// - 256 rows a workgroup (kw 1) once a workgroup has PF_LONG tiles of work: half
-//   the LDS writes and tile copies per row (1,500 tokens over 512 tiles of 8
-//   heads, 128 dims: 803 us against 911), but twice the piece bytes (700 tokens
-//   over 144 tiles of 2 heads: 50.4 against 45.8).
-// - converted by the attention (PF_QUANT) while its slower tiles cost less than
-//   the conversion's own launch (37 tokens over 544 tiles: 63 us against 88; 300
-//   over 128: 100 against 92).
+// Rows of a unit, and with them the kernel: 256 (k_pf_attn; a quantised window is
+// converted ahead) once a workgroup would have PF_LONG tiles of 128 rows, 128
+// (k_pf_attn_split) below.  1,500 tokens x 512 tiles, 8 heads x 128: 770 us with
+// 256 rows, 944 with 128; 1,000 x 128, 4 x 256: 201 and 215; 300 x 128, 4 x 256: 87
+// and 78; 37 x 544, 4 x 256: 99 and 54; on an f16 window 1,000 x 256, 8 x 128: 255
+// and 271; 700 x 144, 2 x 128: 48 and 41.
 #define PF_LONG 64.0
-struct pf_shape {
-    int src, kw;
-};
-static pf_shape pf_choose(uint32_t D, uint32_t H, uint64_t n_rows, uint32_t n_tiles, uint32_t n_seg, bool quant,
-                          uint32_t n_cu) {
-    const uint64_t U = (uint64_t)kvm_cdiv(n_rows, 128) * H * n_seg;
-    const uint32_t seg_t = kvm_cdiv(n_tiles, n_seg);
-    const int kw = (double)U * seg_t / n_cu >= PF_LONG ? 1 : 2;
-    if (!quant) return {PF_F16, kw};
-    double own, staged;
-    const double piece = pf_piece_us(D, n_rows, kvm_cdiv(n_rows, 128));
-    pf_shares(U, seg_t, pf_tile_us(D, 2, PF_QUANT), piece, n_cu, &own);
-    pf_shares(U, seg_t, pf_tile_us(D, 2, PF_STAGED), piece, n_cu, &staged);
-    staged += 3.0 + 0.0162 * D / 256 * H * n_tiles;
-    return own <= staged ? pf_shape{PF_QUANT, 2} : pf_shape{PF_STAGED, kw};
-}
 
 extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q, int q_type,
                               const int32_t *q_pos, uint32_t n_tokens, uint32_t n_head, float scale,
@@ -936,8 +1112,9 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     const bool quant = kvm_k_quant(w->k_type);
 
     const uint32_t n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
-    const pf_shape sh = pf_choose(D, H, n_rows, n_tiles, n_seg, quant, st->n_cu);
-    int src = sh.src, kw = sh.kw;
+    const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / st->n_cu >= PF_LONG;
+    const uint32_t rows = long_work ? 256u : 128u;
+    const int src = !quant ? PF_F16 : long_work ? PF_STAGED : PF_QUANT;
 
     pf_args a{};
     a.n_tiles = n_tiles;
@@ -946,13 +1123,12 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     a.G = G;
     a.n_head = n_head;
     a.n_rows = (uint32_t)n_rows;
-    const uint32_t rows = 256u / kw;
     a.n_row_tiles = (uint32_t)kvm_cdiv(n_rows, rows);
     const uint64_t units = (uint64_t)a.n_row_tiles * H * a.n_seg;
     if (units > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
     a.U = (uint32_t)units;
-    uint64_t P = pf_shares(units, kvm_cdiv(n_tiles, n_seg), pf_tile_us(D, kw, src),
-                           pf_piece_us(D, n_rows, a.n_row_tiles), st->n_cu, nullptr);
+    uint64_t P = pf_shares(units, kvm_cdiv(n_tiles, n_seg), pf_tile_us(D, src, rows),
+                           pf_piece_us(D, n_rows, a.n_row_tiles), st->n_cu);
     // KVM_PF_SPLITS in the environment fixes the pieces per unit
     if (const char *e = getenv("KVM_PF_SPLITS")) {
         const int v = atoi(e);
@@ -999,8 +1175,8 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     a.ws_ml = (float *)(ws + 2 * kv_bytes + info_bytes + part_o);
 
     KVM_HIP(st, hipSetDevice(st->device));
-    if (D == 256) pf_launch<256>(a, sa, src, kw, st->stream);
-    else pf_launch<128>(a, sa, src, kw, st->stream);
+    if (D == 256) pf_launch<256>(a, sa, src, rows, st->stream);
+    else pf_launch<128>(a, sa, src, rows, st->stream);
     KVM_LAUNCH_CHECK(st, "fa_prefill");
     return KVM_OK;
 }
