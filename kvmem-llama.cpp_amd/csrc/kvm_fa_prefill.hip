@@ -117,9 +117,7 @@ __device__ __forceinline__ uint32_t opaque(int x) {
 
 struct pf_stage_args {
     const uint8_t *k, *v;        // window K / V tiles (q8_0 / q4_0)
-    const int32_t *cell_pos;
     uint8_t *kh, *vh;            // f16 operand tiles [H][n_tiles][64 * D]
-    int32_t *info;               // [n_tiles][4]: min live pos, max live pos, live cells, 0
     uint32_t n_tiles;
 };
 
@@ -151,17 +149,6 @@ __global__ void __launch_bounds__(256) k_pf_stage(pf_stage_args a) {
         for (uint32_t ks = 0; ks < 2; ++ks)
             *(kvm_f16x8 *)(vh + ks * 64u * D + 16 * u) = pf_q4(vw[ks], *(const kvm_u32x4 *)(sc + 64 * ks));
     }
-    if (h == 0 && tid < 64) {
-        const int32_t p = a.cell_pos[(uint64_t)t * 64 + tid];
-        int32_t mn = p >= 0 ? p : INT32_MAX, mx = p >= 0 ? p : INT32_MIN, n = p >= 0;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            mn = min(mn, __shfl_xor(mn, o, 64));
-            mx = max(mx, __shfl_xor(mx, o, 64));
-            n += __shfl_xor(n, o, 64);
-        }
-        if (tid == 0) *(kvm_i32x4 *)(a.info + (uint64_t)t * 4) = kvm_i32x4{mn, mx, n, 0};
-    }
 }
 
 // The keys of U units (unit u: segment u % n_seg of row tile (u / n_seg) %
@@ -171,7 +158,7 @@ __global__ void __launch_bounds__(256) k_pf_stage(pf_stage_args a) {
 // to slot 2 p (the workgroup's first unit) or 2 p + 1 (its last).
 struct pf_args {
     const uint8_t *k, *v;        // f16 operand tiles, f16 window tiles or quantised window tiles
-    const int32_t *info, *cell_pos;
+    const int32_t *cell_pos;
     const void *q;
     const int32_t *q_pos;
     float *out;                  // [token][n_head][D] fp32
@@ -210,95 +197,88 @@ struct pf_front {
     uint16_t list[KVM_PF_LIST];      // tile - t_begin, bit 15: every cell live and visible to every row, so no mask
     uint32_t mm[2][8], cnt[KVM_PF_LIST / 64];
 };
-template <bool STAGED, typename COPY_Q>
+template <typename COPY_Q>
 __device__ __forceinline__ uint32_t pf_tiles(const pf_args &a, uint32_t row, uint32_t t_begin, uint32_t f_lo, uint32_t f_hi,
                                              pf_front &fr, uint32_t &qlim, COPY_Q &&copy_q) {
     const int tid = (int)opaque((int)threadIdx.x), l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-            // ---- the loads of the prologue, all issued before any is used: the lane's
-            // row position, the tiles' cells (or summaries), the Q row
-            const bool live_row = row < a.n_rows;
-            const int32_t qp = a.q_pos[(live_row ? row : 0u) / a.G];
-            const uint32_t n_seg_t = a.n_tiles - t_begin < KVM_PF_LIST ? a.n_tiles - t_begin : KVM_PF_LIST;
-            // a wave looks at 4 tiles at a time, 4 cells a lane (PF_STAGED: a lane at one tile's summary)
-            constexpr uint32_t NL = STAGED ? 2 : 18, TPL = STAGED ? 64 : 4, TPB = NL * 8 * TPL;
-            const uint32_t t_lane = STAGED ? (uint32_t)tid : (uint32_t)(4 * w + (l >> 4));
-            kvm_u32x4 cells[NL];
-            auto load_cells = [&](uint32_t t0) {
+    // ---- the loads of the prologue, all issued before any is used: the lane's
+    // row position, the tiles' cells, the Q rows' copies
+    const bool live_row = row < a.n_rows;
+    const int32_t qp = a.q_pos[(live_row ? row : 0u) / a.G];
+    const uint32_t n_seg_t = a.n_tiles - t_begin < KVM_PF_LIST ? a.n_tiles - t_begin : KVM_PF_LIST;
+    // a wave looks at 4 tiles at a time, 4 cells a lane (36,864 cells at once)
+    constexpr uint32_t NL = 18, TPB = NL * 32;
+    const uint32_t t_lane = (uint32_t)(4 * w + (l >> 4));
+    kvm_u32x4 cells[NL];
+    auto load_cells = [&](uint32_t t0) {
 #pragma unroll
-                for (uint32_t i = 0; i < NL; ++i) {
-                    const uint32_t t = t0 + 8 * TPL * i + t_lane;
-                    const uint64_t tile = t_begin + (t < n_seg_t ? t : 0u);
-                    cells[i] = STAGED ? *(const kvm_u32x4 *)(a.info + tile * 4)
-                                                : *(const kvm_u32x4 *)(a.cell_pos + tile * 64 + 4 * (l & 15));
-                }
-            };
-            load_cells(0);
-            copy_q();
+        for (uint32_t i = 0; i < NL; ++i) {
+            const uint32_t t = t0 + 32 * i + t_lane;
+            const uint64_t tile = t_begin + (t < n_seg_t ? t : 0u);
+            cells[i] = *(const kvm_u32x4 *)(a.cell_pos + tile * 64 + 4 * (l & 15));
+        }
+    };
+    load_cells(0);
+    copy_q();
+    __builtin_amdgcn_sched_barrier(0);
 
-
-            // ---- a cell is visible to the lane's row iff (unsigned)position < qlim
-            qlim = live_row && qp >= 0 ? (uint32_t)qp + 1u : 0u;
-            const uint32_t mn = kvm_wave_min_u32(live_row ? qlim : 0xffffffffu), mx = ~kvm_wave_min_u32(~qlim);
-            if (l == 0) {
-                fr.mm[0][w] = mn;
-                fr.mm[1][w] = mx;
-            }
-            KVM_LDS_BARRIER();
-            uint32_t wg_min = fr.mm[0][0], wg_max = fr.mm[1][0];
+    // ---- a cell is visible to the lane's row iff (unsigned)position < qlim
+    qlim = live_row && qp >= 0 ? (uint32_t)qp + 1u : 0u;
+    const uint32_t mn = kvm_wave_min_u32(live_row ? qlim : 0xffffffffu), mx = ~kvm_wave_min_u32(~qlim);
+    if (l == 0) {
+        fr.mm[0][w] = mn;
+        fr.mm[1][w] = mx;
+    }
+    KVM_LDS_BARRIER();
+    uint32_t wg_min = fr.mm[0][0], wg_max = fr.mm[1][0];
 #pragma unroll
-            for (int i = 1; i < 8; ++i) {
-                wg_min = min(wg_min, fr.mm[0][i]);
-                wg_max = max(wg_max, fr.mm[1][i]);
-            }
+    for (int i = 1; i < 8; ++i) {
+        wg_min = min(wg_min, fr.mm[0][i]);
+        wg_max = max(wg_max, fr.mm[1][i]);
+    }
 
-            // ---- the piece's tiles: the segment's tiles that some row here can see,
-            // in order, and of these the share [f_lo, f_hi) / P.  fr.list holds tile -
-            // t_begin and bit 15: every cell live and visible to every row, so no mask.
-            for (uint32_t t0 = 0;;) {
+    // ---- the piece's tiles: the segment's tiles that some row here can see,
+    // in order, and of these the share [f_lo, f_hi) / P.  fr.list holds tile -
+    // t_begin and bit 15: every cell live and visible to every row, so no mask.
+    for (uint32_t t0 = 0;;) {
 #pragma unroll
-                for (uint32_t i = 0; i < NL; ++i) {
-                    const uint32_t t = t0 + 8 * TPL * i + t_lane;
-                    const kvm_u32x4 c = cells[i];
-                    bool some, all;
-                    if constexpr (STAGED) {
-                        some = c[2] != 0 && c[0] < wg_max;
-                        all = c[2] == 64 && c[1] < wg_min;
-                    } else {
-                        const uint32_t lo = min(min(c[0], c[1]), min(c[2], c[3])), hi = max(max(c[0], c[1]), max(c[2], c[3]));
-                        some = ((uint32_t)(__builtin_amdgcn_ballot_w64(lo < wg_max) >> (l & 48)) & 0xffffu) != 0;
-                        all = ((uint32_t)(__builtin_amdgcn_ballot_w64(hi < wg_min) >> (l & 48)) & 0xffffu) == 0xffffu;
-                    }
-                    if (t < n_seg_t && (STAGED || (l & 15) == 0)) fr.flag[t] = (uint8_t)(some | all << 1);
-                }
-                t0 += TPB;
-                if (t0 >= n_seg_t) break;
-                load_cells(t0);
-            }
-            KVM_LDS_BARRIER();
-            uint32_t n_t;
-            {
-                const uint32_t n_it = (n_seg_t + 511) / 512;
-                auto flag = [&](uint32_t it) { return 512 * it + tid < n_seg_t ? (uint32_t)fr.flag[512 * it + tid] : 0u; };
-                for (uint32_t it = 0; it < n_it; ++it) {
-                    const uint64_t bal = __builtin_amdgcn_ballot_w64(flag(it) & 1u);
-                    if (l == 0) fr.cnt[8 * it + w] = __popcll(bal);
-                }
-                KVM_LDS_BARRIER();
-                // every wave scans the counts of all (at most 16 x 8 of them)
-                const uint32_t c0 = (uint32_t)l < 8 * n_it ? fr.cnt[l] : 0u, c1 = (uint32_t)l + 64 < 8 * n_it ? fr.cnt[l + 64] : 0u;
-                const uint32_t i0 = kvm_wave_incl_scan(c0), half = __builtin_amdgcn_readlane(i0, 63);
-                const uint32_t i1 = n_it > 8 ? kvm_wave_incl_scan(c1) : 0u, total = half + (n_it > 8 ? __builtin_amdgcn_readlane(i1, 63) : 0u);
-                const uint32_t lo = total * f_lo / a.P, hi = total * f_hi / a.P;     // P <= 2^16
-                n_t = hi - lo;
-                for (uint32_t it = 0; it < n_it; ++it) {
-                    const uint32_t f = flag(it), x = 8 * it + w;
-                    const uint64_t bal = __builtin_amdgcn_ballot_w64(f & 1u);
-                    const uint32_t base = x < 64 ? __builtin_amdgcn_readlane(i0 - c0, x) : half + __builtin_amdgcn_readlane(i1 - c1, x - 64);
-                    const uint32_t rank = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                    if ((f & 1u) && rank >= lo && rank < hi) fr.list[rank - lo] = (uint16_t)((512 * it + tid) | (f >> 1) << 15);
-                }
-                KVM_LDS_BARRIER();
-            }
+        for (uint32_t i = 0; i < NL; ++i) {
+            const uint32_t t = t0 + 32 * i + t_lane;
+            const kvm_u32x4 c = cells[i];
+            const uint32_t lo = min(min(c[0], c[1]), min(c[2], c[3])), hi = max(max(c[0], c[1]), max(c[2], c[3]));
+            const uint32_t some = (uint32_t)(__builtin_amdgcn_ballot_w64(lo < wg_max) >> (l & 48)) & 0xffffu;
+            const uint32_t all = (uint32_t)(__builtin_amdgcn_ballot_w64(hi < wg_min) >> (l & 48)) & 0xffffu;
+            if (t < n_seg_t && (l & 15) == 0) fr.flag[t] = (uint8_t)((some != 0) | (all == 0xffffu) << 1);
+        }
+        t0 += TPB;
+        if (t0 >= n_seg_t) break;
+        load_cells(t0);
+    }
+    KVM_LDS_BARRIER();
+    uint32_t n_t;
+    {
+        const uint32_t n_it = (n_seg_t + 511) / 512;
+        auto flag = [&](uint32_t it) { return 512 * it + tid < n_seg_t ? (uint32_t)fr.flag[512 * it + tid] : 0u; };
+        for (uint32_t it = 0; it < n_it; ++it) {
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(flag(it) & 1u);
+            if (l == 0) fr.cnt[8 * it + w] = __popcll(bal);
+        }
+        KVM_LDS_BARRIER();
+        // every wave scans the counts of all (at most 16 x 8 of them)
+        const uint32_t c0 = (uint32_t)l < 8 * n_it ? fr.cnt[l] : 0u, c1 = (uint32_t)l + 64 < 8 * n_it ? fr.cnt[l + 64] : 0u;
+        const uint32_t i0 = kvm_wave_incl_scan(c0), half = __builtin_amdgcn_readlane(i0, 63);
+        const uint32_t i1 = n_it > 8 ? kvm_wave_incl_scan(c1) : 0u, total = half + (n_it > 8 ? __builtin_amdgcn_readlane(i1, 63) : 0u);
+        const uint32_t lo = total * f_lo / a.P, hi = total * f_hi / a.P;     // P <= 2^16
+        n_t = hi - lo;
+        for (uint32_t it = 0; it < n_it; ++it) {
+            const uint32_t f = flag(it), x = 8 * it + w;
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(f & 1u);
+            const uint32_t base = x < 64 ? __builtin_amdgcn_readlane(i0 - c0, x) : half + __builtin_amdgcn_readlane(i1 - c1, x - 64);
+            const uint32_t rank = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+            if ((f & 1u) && rank >= lo && rank < hi) fr.list[rank - lo] = (uint16_t)((512 * it + tid) | (f >> 1) << 15);
+        }
+        KVM_LDS_BARRIER();
+    }
     return n_t;
 }
 
@@ -343,7 +323,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
         const uint32_t t_begin = seg * KVM_PF_LIST;
         uint32_t qlim;
         auto dma_q = [&](int pass) { pf_copy_q<D, ROWS, Q_UC, BF16>(a, rt_i, h, pass, lds_mem + Q_OFS, w, l); };
-        const uint32_t n_t = pf_tiles<false>(a, row, t_begin, f_lo, f_hi, s_front, qlim, [&]() { dma_q(0); });
+        const uint32_t n_t = pf_tiles(a, row, t_begin, f_lo, f_hi, s_front, qlim, [&]() { dma_q(0); });
         auto entry = [&](uint32_t k) { return (uint32_t)s_front.list[k < n_t ? k : n_t - 1]; };
 
         // Q rows as f16 B operands: lane (g2, m2) holds Q[row m2][16ks + 8 g2 .. +7]
@@ -646,7 +626,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
         const uint32_t row = rt_i * ROWS + 32 * rg + m2;
         const uint32_t t_begin = seg * KVM_PF_LIST;
         uint32_t qlim;
-        const uint32_t n_t = pf_tiles<false>(a, row, t_begin, f_lo, f_hi, s_front, qlim, [&]() {
+        const uint32_t n_t = pf_tiles(a, row, t_begin, f_lo, f_hi, s_front, qlim, [&]() {
             pf_copy_q<D, ROWS, Q_UC, BF16>(a, rt_i, h, 0, lds_mem + Q_OFS, w, l);
         });
         // Both roles take the same barriers: one when Q is in LDS (two if the first
@@ -961,11 +941,11 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
 template <int D, int ROWS, int WS, int NP>
 __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     constexpr uint32_t IB = 4 / WS;
-    const uint32_t l = threadIdx.x & 63u, wv = threadIdx.x >> 6, ws = wv % WS, i = blockIdx.x * IB + wv / WS;
-    const uint32_t rg = blockIdx.y, m2 = l & 31u, rt_i = blockIdx.z % a.n_row_tiles, h = blockIdx.z / a.n_row_tiles;
+    const uint32_t l = threadIdx.x & 63u, wv = threadIdx.x >> 6, ws = wv % WS, i = blockIdx.z * IB + wv / WS;
+    const uint32_t rg = blockIdx.y, m2 = l & 31u, rt_i = blockIdx.x % a.n_row_tiles, h = blockIdx.x / a.n_row_tiles;
     const uint32_t row = rt_i * ROWS + 32 * rg + m2;
     // the unit's pieces: workgroups q0 .. q1 of each of its segments
-    const uint32_t u0 = blockIdx.z * a.n_seg, u1 = u0 + a.n_seg;
+    const uint32_t u0 = blockIdx.x * a.n_seg, u1 = u0 + a.n_seg;
     float M = -INFINITY, L = 0.0f;
     kvm_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     if (rt_i * ROWS + 32 * rg >= a.n_rows) return;
@@ -1026,6 +1006,16 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     *(kvm_f32x4 *)(a.out + ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + 8 * i + 4 * (l >> 5)) = acc * inv;
 }
 
+// The copies global -> LDS take 16-byte aligned sources: a buffer that is not is
+// copied to the workspace first.
+__global__ void __launch_bounds__(256) k_pf_align(const uint8_t *src, uint8_t *dst, uint64_t n16) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n16) return;
+    kvm_u32x4 x;
+    __builtin_memcpy(&x, src + 16 * i, 16);
+    *(kvm_u32x4 *)(dst + 16 * i) = x;
+}
+
 template <int D, int ROWS, int SRC>
 static void pf_attn(const pf_args &a, hipStream_t stream) {
     auto go = [&](auto bf16) {
@@ -1036,7 +1026,7 @@ static void pf_attn(const pf_args &a, hipStream_t stream) {
     if (a.q_bf16) go(std::true_type{});
     else go(std::false_type{});
     if (a.n_seg == 1 && a.U % a.P == 0) return;           // every unit whole
-    const dim3 g1(D / 32, ROWS / 32, a.n_row_tiles * a.H), g4(D / 8, ROWS / 32, a.n_row_tiles * a.H), t(256);
+    const dim3 g1(a.n_row_tiles * a.H, ROWS / 32, D / 32), g4(a.n_row_tiles * a.H, ROWS / 32, D / 8), t(256);
     // most pieces of a unit (of one of its segments)
     const uint32_t n = a.P % a.U == 0 ? a.P / a.U : a.P / a.U + 2;
     if (n <= 2) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 1, 2>), g1, t, 0, stream, a);
@@ -1110,7 +1100,6 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     const uint64_t n_rows = (uint64_t)n_tokens * G;
     if (n_rows > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
     const bool quant = kvm_k_quant(w->k_type);
-
     const uint32_t n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
     const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / st->n_cu >= PF_LONG;
     const uint32_t rows = long_work ? 256u : 128u;
@@ -1145,14 +1134,22 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     a.k = (const uint8_t *)w->k;
     a.v = (const uint8_t *)w->v;
 
-    // workspace: the pieces, and for PF_STAGED the f16 K and V operand tiles and
-    // the tile summaries
+    // workspace: the pieces, and for PF_STAGED the f16 K and V operand tiles
     auto up256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t kv_bytes = src == PF_STAGED ? up256((size_t)H * n_tiles * 64 * D * 2) : 0;
-    const size_t info_bytes = src == PF_STAGED ? up256((size_t)n_tiles * 16) : 0;
     const bool pieces = a.n_seg > 1 || a.U % a.P != 0;
     const size_t part_o = pieces ? (size_t)2 * a.P * rows * D * 4 : 0, part_ml = pieces ? (size_t)2 * a.P * rows * 8 : 0;
-    const size_t total = 2 * kv_bytes + info_bytes + part_o + part_ml;
+    // aligned copies (all sizes are multiples of 16)
+    struct { const uint8_t **p; size_t bytes; } src_buf[3] = {
+        {(const uint8_t **)&a.q, (size_t)n_tokens * n_head * D * (a.q_bf16 ? 2 : 4)},
+        {&a.k, src == PF_F16 ? (size_t)H * n_tiles * 128 * D : 0},
+        {&a.v, src == PF_F16 ? (size_t)H * n_tiles * 128 * D : 0}};
+    size_t copies = 0;
+    for (auto &b : src_buf) {
+        if (!((uintptr_t)*b.p & 15)) b.bytes = 0;
+        copies += up256(b.bytes);
+    }
+    const size_t total = 2 * kv_bytes + copies + part_o + part_ml;
     uint8_t *ws = nullptr;
     if (total) {
         ws = (uint8_t *)kvm_workspace(st, total);
@@ -1162,19 +1159,23 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     if (src == PF_STAGED) {
         sa.k = a.k;
         sa.v = a.v;
-        sa.cell_pos = w->cell_pos;
         sa.kh = ws;
         sa.vh = ws + kv_bytes;
-        sa.info = (int32_t *)(ws + 2 * kv_bytes);
         sa.n_tiles = n_tiles;
         a.k = sa.kh;
         a.v = sa.vh;
-        a.info = sa.info;
     }
-    a.ws_o = (float *)(ws + 2 * kv_bytes + info_bytes);
-    a.ws_ml = (float *)(ws + 2 * kv_bytes + info_bytes + part_o);
-
     KVM_HIP(st, hipSetDevice(st->device));
+    uint8_t *at = ws + 2 * kv_bytes;
+    for (auto &b : src_buf) {
+        if (!b.bytes) continue;
+        hipLaunchKernelGGL(k_pf_align, dim3(kvm_cdiv(b.bytes / 16, 256)), dim3(256), 0, st->stream, *b.p, at, (uint64_t)(b.bytes / 16));
+        *b.p = at;
+        at += up256(b.bytes);
+    }
+    a.ws_o = (float *)at;
+    a.ws_ml = (float *)(at + part_o);
+
     if (D == 256) pf_launch<256>(a, sa, src, rows, st->stream);
     else pf_launch<128>(a, sa, src, rows, st->stream);
     KVM_LAUNCH_CHECK(st, "fa_prefill");

@@ -326,3 +326,32 @@ def test_fa_prefill_edges(kvm_state, case, monkeypatch):
     assert np.isfinite(out).all() and np.all(out[0] == 0)
     toks = np.unique(np.r_[1, 2, T // 2, T - 2, T - 1])
     _prefill_check(out[toks], q.float().numpy()[toks], kr, vr, cp, pos[toks], H, G, D, kt, vt, D ** -0.5)
+
+
+def test_fa_prefill_two_segments(kvm_state):
+    """A window of more tiles than one list holds: two segments per unit, each cut
+    into pieces of its own; half of the first one empty."""
+    rng = np.random.default_rng(77)
+    H, G, D, T, n = 1, 8, 128, 5, 525312
+    w, kr, vr, cp = _window(kvm_state, rng, n, H, D, L.T_Q8_0, L.T_Q4_0)
+    cp[4096:266240] = -1
+    w.import_rows(0, dev(kr), dev(vr), dev(cp))
+    pos = np.arange(n - T, n, dtype=np.int32)
+    q = rng.standard_normal((T, H * G, D)).astype(np.float32)
+    out = host(api.fa_prefill(kvm_state, w, dev(q), dev(pos), H * G, D ** -0.5))
+    _prefill_check(out, q, kr, vr, cp, pos, H, G, D, L.T_Q8_0, L.T_Q4_0, D ** -0.5)
+
+
+@pytest.mark.parametrize("kt,vt,qdt", [(L.T_Q8_0, L.T_Q4_0, torch.bfloat16), (L.T_F16, L.T_F16, torch.float32)])
+def test_fa_prefill_query_alignment(kvm_state, kt, vt, qdt):
+    """A query that starts anywhere in memory gives the aligned one's output."""
+    rng = np.random.default_rng(19)
+    H, G, D, T, n = 2, 6, 256, 30, 1024
+    w, *_ = _window(kvm_state, rng, n, H, D, kt, vt)
+    q = torch.from_numpy(rng.standard_normal((T, H * G, D)).astype(np.float32)).to(qdt).cuda()
+    pos = dev(np.arange(n - T, n, dtype=np.int32))
+    want = host(api.fa_prefill(kvm_state, w, q, pos, H * G, D ** -0.5))
+    buf = torch.zeros(q.numel() + 1, dtype=qdt, device="cuda")
+    buf[1:] = q.reshape(-1)
+    got = host(api.fa_prefill(kvm_state, w, buf[1:].view(T, H * G, D), pos, H * G, D ** -0.5))
+    assert np.array_equal(got, want)
