@@ -236,6 +236,48 @@ __global__ void __launch_bounds__(D) k_query_terms(const float *q_sum, const uin
     if (d == 0) q_norm[(uint64_t)il * H + h] = ordered_sum<D>(s_sq);
 }
 
+// A few rows (at most KVM_QFEW_ROWS) and the terms they change in one launch: one
+// workgroup, a thread per (kv head, dim), which adds the rows of its group's heads
+// in order, the loads of four heads in flight, and then forms the terms as
+// k_query_terms does.  Two launches cost a decode step's four tokens 2.9 + 2.8 us
+// and ~9 of the host's time.
+#define KVM_QFEW_ROWS 8u
+template <int T, int D>
+__global__ void __launch_bounds__(1024) k_query_add_terms(qview_args a, float *q_vec, float *q_norm, uint32_t g) {
+    __shared__ __align__(16) float s_sq[1024];
+    const uint32_t tid = threadIdx.x, h = tid / D, d = tid % D;
+    const uint32_t qc = a.q_count[0] + a.n_kept, keep = a.keep[0];
+    float qh = 0.0f;
+    for (uint32_t g0 = 0; g0 < g; g0 += 4) {
+        float s[4];
+        uint32_t x[4][KVM_QFEW_ROWS];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t e = (h * g + (g0 + i < g ? g0 + i : g - 1)) * D + d;
+            const uint8_t *p = a.v.data + (size_t)a.t0 * a.v.nb2 + view_off(a.v, e);
+            s[i] = a.q_sum[e];
+#pragma unroll
+            for (uint32_t r = 0; r < KVM_QFEW_ROWS; ++r)
+                x[i][r] = view_raw<T>(p + (size_t)(r < a.n_rows ? r : a.n_rows - 1) * a.v.nb2);
+        }
+        __builtin_amdgcn_sched_barrier(0);           // all of them in flight
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            if (g0 + i >= g) break;
+#pragma unroll
+            for (uint32_t r = 0; r < KVM_QFEW_ROWS; ++r) s[i] = (keep >> r) & 1u ? kvm_fadd(s[i], raw_value<T>(x[i][r])) : s[i];
+            a.q_sum[(h * g + g0 + i) * D + d] = s[i];
+            qh = kvm_fadd(qh, s[i]);
+        }
+    }
+    const float qv = kvm_fmul(qh, kvm_recip_or0((float)(qc * (g > 1u ? g : 1u))));
+    q_vec[tid] = qv;
+    s_sq[tid] = kvm_fmul(qv, qv);
+    __syncthreads();                                 // every thread has read the count, too
+    if (d == 0) q_norm[h] = ordered_sum<D>(s_sq + tid);
+    if (tid == 0) a.q_count[0] = qc;
+}
+
 // An accumulator that carries the query terms: their buffers and grouping.
 static int query_terms_check(kvm_state *st, const kvm_query_acc *acc, const char *who) {
     if (!acc->q_vec) return KVM_OK;
@@ -306,6 +348,8 @@ extern "C" int kvm_query_add_view(kvm_state *st, const kvm_query_acc *acc, uint3
     if (rc) return rc;
     KVM_HIP(st, hipSetDevice(st->device));
     const bool rows_ok = query_rows_ok(q, n_embd);
+    const uint32_t n_kv = acc->n_head_kv * acc->head_dim;
+    const bool few = acc->q_vec && (uint64_t)q->ne2 <= KVM_QFEW_ROWS && n_kv <= 1024u;    // with the terms, one workgroup
     bool added = false;
     for (uint64_t t0 = 0; t0 < (uint64_t)q->ne2; t0 += KVM_QVIEW_ROWS) {
         // a launch covers its rows from the first kept one to the last
@@ -327,7 +371,15 @@ extern "C" int kvm_query_add_view(kvm_state *st, const kvm_query_acc *acc, uint3
             }
         auto go = [&](auto t) {
             constexpr int T = decltype(t)::value;
-            if (rows_ok && a.n_rows > KVM_QROWS_MIN)
+            if (few && acc->head_dim == 256)
+                hipLaunchKernelGGL((k_query_add_terms<T, 256>), dim3(1), dim3(n_kv), 0, st->stream, a,
+                                   acc->q_vec + (uint64_t)il * n_kv, acc->q_norm + (uint64_t)il * acc->n_head_kv,
+                                   acc->n_head / acc->n_head_kv);
+            else if (few)
+                hipLaunchKernelGGL((k_query_add_terms<T, 128>), dim3(1), dim3(n_kv), 0, st->stream, a,
+                                   acc->q_vec + (uint64_t)il * n_kv, acc->q_norm + (uint64_t)il * acc->n_head_kv,
+                                   acc->n_head / acc->n_head_kv);
+            else if (rows_ok && a.n_rows > KVM_QROWS_MIN)
                 hipLaunchKernelGGL(k_query_add_rows<T>, dim3(n_embd / 32), dim3(320), 0, st->stream, a);
             else
                 hipLaunchKernelGGL(k_query_add<T>, dim3(kvm_cdiv(n_embd, 64)), dim3(64), 0, st->stream, a);
@@ -338,7 +390,7 @@ extern "C" int kvm_query_add_view(kvm_state *st, const kvm_query_acc *acc, uint3
         KVM_LAUNCH_CHECK(st, "query_add");
         added = true;
     }
-    return added ? query_terms_launch(st, acc, il, 1) : KVM_OK;
+    return added && !few ? query_terms_launch(st, acc, il, 1) : KVM_OK;
 }
 
 extern "C" int kvm_query_add(kvm_state *st, const kvm_query_acc *acc, uint32_t il,

@@ -184,3 +184,29 @@ def test_view_shape_is_checked(kvm_state):
     v = api.view(k)
     v.type = api.L.T_Q8_0                            # a quantised view is not a captured output
     assert kvm_state.lib.kvm_meank_add_view(kvm_state.h, api.C.byref(ix.c), 0, 0, api.C.byref(v)) == api.L.KVM_EUNSUPPORTED
+
+
+@pytest.mark.parametrize("H,G,D", [(4, 6, 256), (8, 4, 128), (1, 5, 128), (8, 3, 256)])
+@pytest.mark.parametrize("n,dt", [(1, "f32"), (4, "bf16"), (8, "f16"), (9, "f32")])
+def test_query_add_few_rows_with_terms(kvm_state, H, G, D, n, dt):
+    """The one-launch form for a few rows and the general one past its limits (more
+    rows, more than 1,024 kv values): sums in row order, the mask's rows only, and
+    the terms that kvm_query_refresh forms from those sums, bit for bit."""
+    rng = np.random.default_rng(H * G + n)
+    qa = api.QueryAcc(kvm_state, 2, H * G, D, n_head_kv=H)
+    qa.reset()
+    total, want = 0, np.zeros(H * G * D, np.float32)
+    for rnd in range(2):
+        q = _captured(rng, n, H * G, D, dt, "heads_major" if rnd else "contiguous")
+        keep = None if rnd else np.arange(n) % 3 != 1
+        qa.add_view(1, q, keep)
+        rows = _f32_rows(q)
+        rows = rows if keep is None else rows[keep]
+        want = _ordered_sum(want, list(rows))
+        total += len(rows)
+    assert np.array_equal(host(qa.q_sum)[1].view(np.uint32), want.view(np.uint32))
+    assert not host(qa.q_sum)[0].any() and list(host(qa.q_count)) == [0, total]
+    vec, norm = qa.q_vec.clone(), qa.q_norm.clone()
+    qa.refresh()
+    assert torch.equal(vec.view(torch.int32), qa.q_vec.view(torch.int32))
+    assert torch.equal(norm.view(torch.int32), qa.q_norm.view(torch.int32))
