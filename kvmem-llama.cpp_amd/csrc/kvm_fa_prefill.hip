@@ -32,10 +32,10 @@
 // f16 tiles: K as kvm_kh_idx; V units of 8 keys of a dim (as kvm_vh_idx), in LDS
 // and in the workspace in the order [32-key half][16-dim tile][8-key group][dim].
 // What bounds it: large chunks, the matrix cores at the clock that the power limit
-// leaves (2,048 tokens x 34,816 cells: 1.10 -> 1.15 PFLOP/s, a large f16 matrix
-// product reaches 1.33); small ones, the attention waves' chain, the latencies of the
-// start and the piece traffic (37 tokens x 32,768 cells: 147 -> 54 us; 100 x 8,192:
-// 54.3 -> 40; 700 x 8,192 on an f16 cache of 2 heads x 128: 51.6 -> 41).
+// leaves (2,048 tokens x 34,816 cells, 16 rows a wave and this: 1.05 -> 1.14 PFLOP/s,
+// a large f16 matrix product reaches 1.33); small ones, the attention waves' chain, the
+// latencies of the start and the piece traffic (37 tokens x 32,768 cells: 152 -> 52 us;
+// 100 x 8,192: 54.3 -> 40; 700 x 8,192 on an f16 cache of 2 heads x 128: 48 -> 43).
 #include "kvm_internal.h"
 
 #include <type_traits>
