@@ -154,8 +154,20 @@ __global__ void __launch_bounds__(256) k_pf_stage(pf_stage_args a) {
 // The keys of U units (unit u: segment u % n_seg of row tile (u / n_seg) %
 // n_row_tiles of kv head u / n_seg / n_row_tiles), each counted as P, are dealt
 // to P workgroups in order: workgroup p has [p U, (p + 1) U) of U P.  The part of
-// a unit that a workgroup has is a piece; pieces of a unit with more than one go
-// to slot 2 p (the workgroup's first unit) or 2 p + 1 (its last).
+// a unit that a workgroup has is a piece; the pieces of a row tile and kv head that
+// has more than one (every one, if there are several segments) go to slots.
+// From one piece to the next the workgroup, the unit or both go on by one, so p + u
+// is another number for each.  With one segment and more units than workgroups
+// only a workgroup's first and last unit can be cut, and 2 p and 2 p + 1 are fewer.
+__host__ __device__ inline uint32_t pf_slot(uint32_t U, uint32_t P, uint32_t n_seg, uint32_t p, uint32_t u,
+                                            uint32_t u_first) {
+    return n_seg == 1 && U > P ? 2 * p + (u != u_first) : p + u;
+}
+__host__ inline uint64_t pf_slots(uint32_t U, uint32_t P, uint32_t n_seg) {
+    if (n_seg == 1 && U % P == 0) return 0;               // every unit whole
+    return n_seg == 1 && U > P ? 2ull * P : (uint64_t)P + U - 1;
+}
+
 struct pf_args {
     const uint8_t *k, *v;        // f16 operand tiles, f16 window tiles or quantised window tiles
     const int32_t *cell_pos;
@@ -565,7 +577,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
                 for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = quad(i) * inv;
             }
         } else if (active) {
-            const uint64_t slot = 2 * (uint64_t)p + (u != u_first);
+            const uint64_t slot = pf_slot(a.U, a.P, a.n_seg, p, u, u_first);
             float *o = a.ws_o + (slot * ROWS + 32 * w) * D + 4 * le;
 #pragma unroll
             for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 256 * i) = quad(i);
@@ -797,7 +809,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
                     for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = quad(i) * inv;
                 }
             } else if (rt_i * ROWS + 32 * rg < a.n_rows) {
-                const uint64_t slot = 2 * (uint64_t)p + (u != u_first);
+                const uint64_t slot = pf_slot(a.U, a.P, a.n_seg, p, u, u_first);
                 float *o = a.ws_o + (slot * ROWS + 32 * rg) * D + 4 * le;
 #pragma unroll
                 for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 256 * i) = quad(i);
@@ -952,15 +964,15 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     for (uint32_t u = u0; u < u1; ++u) {
         const uint32_t q0 = u * a.P / a.U, q1 = ((u + 1) * a.P - 1) / a.U;
         if (q0 == q1 && a.n_seg == 1) return;             // whole: the attention wrote it
-        // q0's piece is its last unit's unless it is also its first (u P = q0 U)
-        const uint32_t s0 = 2 * q0 + (q0 * a.U / a.P != u);
+        // u is the first unit of every workgroup after q0
+        const uint32_t s0 = pf_slot(a.U, a.P, a.n_seg, q0, u, q0 * a.U / a.P);
         for (uint32_t q = q0; q <= q1; q += NP * WS) {
             kvm_f32x4 x[NP];
             float m[NP], s[NP];
 #pragma unroll
             for (uint32_t j = 0; j < NP; ++j) {
                 const uint32_t qj = q + WS * j + ws, pj = min(qj, q1);
-                const uint64_t slot = pj == q0 ? s0 : 2 * pj;
+                const uint64_t slot = pj == q0 ? s0 : pf_slot(a.U, a.P, a.n_seg, pj, u, u);
                 x[j] = *(const kvm_f32x4 *)(a.ws_o + (slot * ROWS + 32 * rg) * D + 256 * i + 4 * l);
                 const kvm_f32x2 ml = *(const kvm_f32x2 *)(a.ws_ml + (slot * ROWS + 32 * rg + m2) * 2);
                 m[j] = qj <= q1 ? ml[0] : -INFINITY;
@@ -1083,6 +1095,47 @@ static double pf_piece_us(uint32_t D, uint64_t n_rows, uint32_t row_tiles) {
 // and 271; 700 x 144, 2 x 128: 48 and 41.
 #define PF_LONG 64.0
 
+struct pf_shape {
+    uint32_t src, rows, n_row_tiles, n_seg, U, P;
+    uint64_t slots;
+};
+static int pf_shape_of(bool quant, uint32_t D, uint32_t H, uint32_t n_tiles, uint64_t n_rows, uint32_t n_cu, pf_shape *s) {
+    s->n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
+    const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / n_cu >= PF_LONG;
+    s->rows = long_work ? 256u : 128u;
+    s->src = !quant ? PF_F16 : long_work ? PF_STAGED : PF_QUANT;
+    s->n_row_tiles = (uint32_t)kvm_cdiv(n_rows, s->rows);
+    const uint64_t units = (uint64_t)s->n_row_tiles * H * s->n_seg;
+    if (units > (1u << 30)) return KVM_ERANGE;
+    s->U = (uint32_t)units;
+    uint64_t P = pf_shares(units, kvm_cdiv(n_tiles, s->n_seg), pf_tile_us(D, s->src, s->rows),
+                           pf_piece_us(D, n_rows, s->n_row_tiles), n_cu);
+    // KVM_PF_SPLITS in the environment fixes the pieces per unit
+    if (const char *e = getenv("KVM_PF_SPLITS")) {
+        const int v = atoi(e);
+        if (v >= 1 && v <= 8) P = units * v < 65536u ? units * v : 65536u;
+    }
+    if (P * units > 0xffffffffu) P = 0xffffffffu / units;
+    s->P = (uint32_t)P;
+    s->slots = pf_slots(s->U, s->P, s->n_seg);
+    return KVM_OK;
+}
+
+// The launch's shape and the slot of a piece, for tests on the host (not part of the ABI).
+extern "C" int kvm_fa_prefill_shape(int k_type, uint32_t head_dim, uint32_t n_head_kv, uint32_t n_cells,
+                                    uint32_t n_tokens, uint32_t n_head, uint32_t n_cu, uint32_t out[7]) {
+    pf_shape s{};
+    const int rc = pf_shape_of(kvm_k_quant(k_type), head_dim, n_head_kv, n_cells / KVM_TILE_CELLS,
+                               (uint64_t)n_tokens * (n_head / n_head_kv), n_cu, &s);
+    const uint32_t v[7] = {s.src, s.rows, s.n_row_tiles, s.n_seg, s.U, s.P, (uint32_t)s.slots};
+    for (int i = 0; i < 7; ++i) out[i] = v[i];
+    return rc;
+}
+extern "C" uint32_t kvm_fa_prefill_slots(uint32_t U, uint32_t P, uint32_t n_seg) { return (uint32_t)pf_slots(U, P, n_seg); }
+extern "C" uint32_t kvm_fa_prefill_slot(uint32_t U, uint32_t P, uint32_t n_seg, uint32_t p, uint32_t u) {
+    return pf_slot(U, P, n_seg, p, u, (uint32_t)((uint64_t)p * U / P));
+}
+
 extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q, int q_type,
                               const int32_t *q_pos, uint32_t n_tokens, uint32_t n_head, float scale,
                               float *out) {
@@ -1099,32 +1152,22 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     const uint32_t D = w->head_dim, H = w->n_head_kv, n_tiles = w->n_cells / KVM_TILE_CELLS;
     const uint64_t n_rows = (uint64_t)n_tokens * G;
     if (n_rows > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
-    const bool quant = kvm_k_quant(w->k_type);
-    const uint32_t n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
-    const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / st->n_cu >= PF_LONG;
-    const uint32_t rows = long_work ? 256u : 128u;
-    const int src = !quant ? PF_F16 : long_work ? PF_STAGED : PF_QUANT;
+    pf_shape sh{};
+    if (pf_shape_of(kvm_k_quant(w->k_type), D, H, n_tiles, n_rows, st->n_cu, &sh))
+        return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
+    const int src = (int)sh.src;
+    const uint32_t rows = sh.rows;
 
     pf_args a{};
     a.n_tiles = n_tiles;
-    a.n_seg = n_seg;
+    a.n_seg = sh.n_seg;
     a.H = H;
     a.G = G;
     a.n_head = n_head;
     a.n_rows = (uint32_t)n_rows;
-    a.n_row_tiles = (uint32_t)kvm_cdiv(n_rows, rows);
-    const uint64_t units = (uint64_t)a.n_row_tiles * H * a.n_seg;
-    if (units > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
-    a.U = (uint32_t)units;
-    uint64_t P = pf_shares(units, kvm_cdiv(n_tiles, n_seg), pf_tile_us(D, src, rows),
-                           pf_piece_us(D, n_rows, a.n_row_tiles), st->n_cu);
-    // KVM_PF_SPLITS in the environment fixes the pieces per unit
-    if (const char *e = getenv("KVM_PF_SPLITS")) {
-        const int v = atoi(e);
-        if (v >= 1 && v <= 8) P = units * v < 65536u ? units * v : 65536u;
-    }
-    if (P * units > 0xffffffffu) P = 0xffffffffu / units;
-    a.P = (uint32_t)P;
+    a.n_row_tiles = sh.n_row_tiles;
+    a.U = sh.U;
+    a.P = sh.P;
     a.c = scale * 1.4426950408889634f;
     a.q_bf16 = q_type == KVM_TYPE_BF16;
     a.q = q;
@@ -1137,8 +1180,7 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     // workspace: the pieces, and for PF_STAGED the f16 K and V operand tiles
     auto up256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t kv_bytes = src == PF_STAGED ? up256((size_t)H * n_tiles * 64 * D * 2) : 0;
-    const bool pieces = a.n_seg > 1 || a.U % a.P != 0;
-    const size_t part_o = pieces ? (size_t)2 * a.P * rows * D * 4 : 0, part_ml = pieces ? (size_t)2 * a.P * rows * 8 : 0;
+    const size_t part_o = (size_t)sh.slots * rows * D * 4, part_ml = (size_t)sh.slots * rows * 8;
     // aligned copies (all sizes are multiples of 16)
     struct { const uint8_t **p; size_t bytes; } src_buf[3] = {
         {(const uint8_t **)&a.q, (size_t)n_tokens * n_head * D * (a.q_bf16 ? 2 : 4)},

@@ -355,3 +355,22 @@ def test_fa_prefill_query_alignment(kvm_state, kt, vt, qdt):
     buf[1:] = q.reshape(-1)
     got = host(api.fa_prefill(kvm_state, w, buf[1:].view(T, H * G, D), pos, H * G, D ** -0.5))
     assert np.array_equal(got, want)
+
+
+def test_fa_prefill_segments_with_more_units_than_workgroups(kvm_state):
+    """A window of two segments whose units outnumber the workgroups: a share then
+    spans more than one whole unit, and every one of its pieces has a place of its
+    own.  Few cells are live, in both segments; two tokens of each row tile, all
+    heads (so every unit is looked at)."""
+    rng = np.random.default_rng(78)
+    H, G, D, T, n, cut = 8, 4, 128, 1160, 525312, 524288
+    w = api.KVWindow(kvm_state, n, H, D, 128, L.T_Q8_0, L.T_Q4_0)
+    kr, vr = rand_rows(rng, 2048 + n - cut, H, D, L.T_Q8_0, L.T_Q4_0)
+    cp = np.arange(kr.shape[0], dtype=np.int32)
+    w.import_rows(0, dev(kr[:2048]), dev(vr[:2048]), dev(cp[:2048]))
+    w.import_rows(cut, dev(kr[2048:]), dev(vr[2048:]), dev(cp[2048:]))
+    pos = np.arange(cp.size - T, cp.size, dtype=np.int32)
+    q = rng.standard_normal((T, H * G, D)).astype(np.float32)
+    out = host(api.fa_prefill(kvm_state, w, dev(q), dev(pos), H * G, D ** -0.5))
+    toks = np.unique(np.r_[np.arange(0, T, 64), np.arange(63, T, 64), T - 1])
+    _prefill_check(out[toks], q[toks], kr, vr, cp, pos[toks], H, G, D, L.T_Q8_0, L.T_Q4_0, D ** -0.5)
