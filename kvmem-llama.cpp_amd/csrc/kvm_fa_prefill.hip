@@ -574,7 +574,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
                 const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
                 float *o = a.out + ((uint64_t)(row_e / a.G) * a.n_head + h * a.G + row_e % a.G) * D + 4 * ge;
 #pragma unroll
-                for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = quad(i) * inv;
+                for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = lr == 0.0f ? kvm_f32x4{0.f, 0.f, 0.f, 0.f} : quad(i) * inv;
             }
         } else if (active) {
             const uint64_t slot = pf_slot(a.U, a.P, a.n_seg, p, u, u_first);
@@ -806,7 +806,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
                     const float inv = lr > 0.0f ? 1.0f / lr : 0.0f;
                     float *o = a.out + ((uint64_t)(row_e / a.G) * a.n_head + h * a.G + row_e % a.G) * D + 4 * ge;
 #pragma unroll
-                    for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = quad(i) * inv;
+                    for (int i = 0; i < DT * 4; ++i) *(kvm_f32x4 *)(o + 8 * i) = lr == 0.0f ? kvm_f32x4{0.f, 0.f, 0.f, 0.f} : quad(i) * inv;
                 }
             } else if (rt_i * ROWS + 32 * rg < a.n_rows) {
                 const uint64_t slot = pf_slot(a.U, a.P, a.n_seg, p, u, u_first);
@@ -971,7 +971,7 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
             float m[NP], s[NP];
 #pragma unroll
             for (uint32_t j = 0; j < NP; ++j) {
-                const uint32_t qj = q + WS * j + ws, pj = min(qj, q1);
+                const uint32_t qj = q + WS * j + ws, pj = min(qj, q1);      // past q1 it is read again, but never added
                 const uint64_t slot = pj == q0 ? s0 : pf_slot(a.U, a.P, a.n_seg, pj, u, u);
                 x[j] = *(const kvm_f32x4 *)(a.ws_o + (slot * ROWS + 32 * rg) * D + 256 * i + 4 * l);
                 const kvm_f32x2 ml = *(const kvm_f32x2 *)(a.ws_ml + (slot * ROWS + 32 * rg + m2) * 2);
@@ -988,7 +988,8 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
             for (uint32_t j = 0; j < NP; ++j) {
                 const float wgt = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mb);
                 L += m[j] == -INFINITY ? 0.0f : s[j] * wgt;
-                acc += x[j] * wgt;
+                // (an infinite sum times the weight 0 would be no number)
+                acc += (q + WS * j + ws <= q1 ? x[j] : kvm_f32x4{0.f, 0.f, 0.f, 0.f}) * wgt;
             }
             M = mb;
         }
@@ -1004,6 +1005,7 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
         float mb = M;
 #pragma unroll
         for (int j = 1; j < WS; ++j) mb = fmaxf(mb, s_m[j][l]);
+        M = mb;
         L = 0.0f;
         acc = kvm_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1015,6 +1017,7 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     }
     if (row >= a.n_rows) return;
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    if (M == -INFINITY) acc = kvm_f32x4{0.f, 0.f, 0.f, 0.f};      // nothing visible: not 0 times what its tiles hold
     *(kvm_f32x4 *)(a.out + ((uint64_t)(row / a.G) * a.n_head + h * a.G + row % a.G) * D + 8 * i + 4 * (l >> 5)) = acc * inv;
 }
 

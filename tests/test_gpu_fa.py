@@ -374,3 +374,27 @@ def test_fa_prefill_segments_with_more_units_than_workgroups(kvm_state):
     out = host(api.fa_prefill(kvm_state, w, dev(q), dev(pos), H * G, D ** -0.5))
     toks = np.unique(np.r_[np.arange(0, T, 64), np.arange(63, T, 64), T - 1])
     _prefill_check(out[toks], q[toks], kr, vr, cp, pos[toks], H, G, D, L.T_Q8_0, L.T_Q4_0, D ** -0.5)
+
+
+@pytest.mark.parametrize("n_cells,splits", [(512, 2), (512, 3), (512, 5), (512, 8), (640, None), (1408, None), (128, None)])
+def test_fa_prefill_infinite_value(kvm_state, n_cells, splits, monkeypatch):
+    """An f16 V value that overflowed: the output that it enters is infinite and the
+    others are what they are without it, however many pieces are merged; a token
+    that sees nothing gets zeros."""
+    if splits is not None:
+        monkeypatch.setenv("KVM_PF_SPLITS", str(splits))
+    rng = np.random.default_rng(n_cells)
+    H, G, D, T = 1, 8, 128, 8
+    w, kr, vr, cp = _window(kvm_state, rng, n_cells, H, D, L.T_F16, L.T_F16)
+    vr.view(np.float16)[-1, 5] = np.inf
+    w.import_rows(0, dev(kr), dev(vr), dev(cp))
+    pos = np.full(T, n_cells - 1, np.int32)
+    pos[0] = -1
+    q = rng.standard_normal((T, H * G, D)).astype(np.float32)
+    out = host(api.fa_prefill(kvm_state, w, dev(q), dev(pos), H * G, D ** -0.5))
+    assert np.all(out[0] == 0)
+    assert np.all(out[1:, :, 5] == np.inf)
+    vr.view(np.float16)[-1, 5] = 0
+    out[:, :, 5] = 0
+    vr.view(np.float16)[:, 5] = 0
+    _prefill_check(out, q, kr, vr, cp, pos, H, G, D, L.T_F16, L.T_F16, D ** -0.5)
