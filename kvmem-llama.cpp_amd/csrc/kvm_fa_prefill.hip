@@ -182,6 +182,15 @@ struct pf_args {
     int q_bf16;
 };
 
+// The row tile of a unit.  With more units than workgroups a workgroup has several
+// after each other, and in a chunk that attends to itself the later rows see more
+// tiles: first and last row tiles take turns, so that shares have like numbers of
+// tiles.  32 heads on 8 x 128, 8,192 tokens (1,024 units, 4 a workgroup): 812 us in row
+// order, 551 here; 24 on 4 x 256, 4,096 tokens (384 units): 326 and 257.
+__device__ __forceinline__ uint32_t pf_row_tile(const pf_args &a, uint32_t i) {
+    return a.U > a.P ? (i & 1u ? a.n_row_tiles - 1 - (i >> 1) : i >> 1) : i;
+}
+
 // Q rows of a unit into LDS, coalesced (as operand loads, 32 rows of 32 bytes an
 // instruction, they took 4 us): unit c of 16 bytes of row r at slot c ^ r, so that a
 // column's reads use every bank; Q_UC units of each row a pass.  Rows past the last
@@ -328,7 +337,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
         const uint32_t u0 = u * a.P;
         const uint32_t f_lo = max(sh0, u0) - u0, f_hi = min(sh1 - u0, a.P);
         const uint32_t seg = u % a.n_seg, rest = u / a.n_seg;
-        const uint32_t rt_i = __builtin_amdgcn_readfirstlane(rest % a.n_row_tiles), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
+        const uint32_t rt_i = __builtin_amdgcn_readfirstlane(pf_row_tile(a, rest % a.n_row_tiles)), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
         const bool whole = f_lo == 0 && f_hi == a.P && a.n_seg == 1;
 
         const uint32_t row = rt_i * ROWS + 32 * w + m2;
@@ -633,7 +642,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
         const uint32_t u0 = u * a.P;
         const uint32_t f_lo = max(sh0, u0) - u0, f_hi = min(sh1 - u0, a.P);
         const uint32_t seg = u % a.n_seg, rest = u / a.n_seg;
-        const uint32_t rt_i = __builtin_amdgcn_readfirstlane(rest % a.n_row_tiles), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
+        const uint32_t rt_i = __builtin_amdgcn_readfirstlane(pf_row_tile(a, rest % a.n_row_tiles)), h = __builtin_amdgcn_readfirstlane(rest / a.n_row_tiles);
         const bool whole = f_lo == 0 && f_hi == a.P && a.n_seg == 1;
         const uint32_t row = rt_i * ROWS + 32 * rg + m2;
         const uint32_t t_begin = seg * KVM_PF_LIST;
@@ -954,7 +963,7 @@ template <int D, int ROWS, int WS, int NP>
 __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     constexpr uint32_t IB = 4 / WS;
     const uint32_t l = threadIdx.x & 63u, wv = threadIdx.x >> 6, ws = wv % WS, i = blockIdx.z * IB + wv / WS;
-    const uint32_t rg = blockIdx.y, m2 = l & 31u, rt_i = blockIdx.x % a.n_row_tiles, h = blockIdx.x / a.n_row_tiles;
+    const uint32_t rg = blockIdx.y, m2 = l & 31u, rt_i = pf_row_tile(a, blockIdx.x % a.n_row_tiles), h = blockIdx.x / a.n_row_tiles;
     const uint32_t row = rt_i * ROWS + 32 * rg + m2;
     // the unit's pieces: workgroups q0 .. q1 of each of its segments
     const uint32_t u0 = blockIdx.x * a.n_seg, u1 = u0 + a.n_seg;
