@@ -155,17 +155,19 @@ __global__ void __launch_bounds__(256) k_pf_stage(pf_stage_args a) {
 // n_row_tiles of kv head u / n_seg / n_row_tiles), each counted as P, are dealt
 // to P workgroups in order: workgroup p has [p U, (p + 1) U) of U P.  The part of
 // a unit that a workgroup has is a piece; the pieces of a row tile and kv head that
-// has more than one (every one, if there are several segments) go to slots.
-// From one piece to the next the workgroup, the unit or both go on by one, so p + u
-// is another number for each.  With one segment and more units than workgroups
-// only a workgroup's first and last unit can be cut, and 2 p and 2 p + 1 are fewer.
+// has more than one (every one, if there are several segments) go to slots.  With
+// one segment only a workgroup's first and last unit can be cut: slots 2 p and
+// 2 p + 1.  With several, from one piece to the next the workgroup, the unit or both
+// go on by one, so p + u is another number for each.  (p + u for one segment as well,
+// which leaves no slot out: 26.6 us where these take 26.0, 200 tokens in an empty
+// f16 window of 4 heads x 256.)
 __host__ __device__ inline uint32_t pf_slot(uint32_t U, uint32_t P, uint32_t n_seg, uint32_t p, uint32_t u,
                                             uint32_t u_first) {
-    return n_seg == 1 && U > P ? 2 * p + (u != u_first) : p + u;
+    return n_seg == 1 ? 2 * p + (u != u_first) : p + u;
 }
 __host__ inline uint64_t pf_slots(uint32_t U, uint32_t P, uint32_t n_seg) {
     if (n_seg == 1 && U % P == 0) return 0;               // every unit whole
-    return n_seg == 1 && U > P ? 2ull * P : (uint64_t)P + U - 1;
+    return n_seg == 1 ? 2ull * P : (uint64_t)P + U - 1;
 }
 
 struct pf_args {
@@ -980,12 +982,18 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
             float m[NP], s[NP];
 #pragma unroll
             for (uint32_t j = 0; j < NP; ++j) {
-                const uint32_t qj = q + WS * j + ws, pj = min(qj, q1);      // past q1 it is read again, but never added
+                const uint32_t qj = q + WS * j + ws, pj = min(qj, q1);
                 const uint64_t slot = pj == q0 ? s0 : pf_slot(a.U, a.P, a.n_seg, pj, u, u);
                 x[j] = *(const kvm_f32x4 *)(a.ws_o + (slot * ROWS + 32 * rg) * D + 256 * i + 4 * l);
                 const kvm_f32x2 ml = *(const kvm_f32x2 *)(a.ws_ml + (slot * ROWS + 32 * rg + m2) * 2);
                 m[j] = qj <= q1 ? ml[0] : -INFINITY;
                 s[j] = ml[1];
+            }
+            if (q + NP * WS > q1 + 1) {
+                // past q1 its piece was read again: an infinity there times the weight 0 is no number
+#pragma unroll
+                for (uint32_t j = 0; j < NP; ++j)
+                    if (q + WS * j + ws > q1) x[j] = kvm_f32x4{0.f, 0.f, 0.f, 0.f};
             }
             float mb = M;
 #pragma unroll
@@ -997,8 +1005,7 @@ __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
             for (uint32_t j = 0; j < NP; ++j) {
                 const float wgt = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mb);
                 L += m[j] == -INFINITY ? 0.0f : s[j] * wgt;
-                // (an infinite sum times the weight 0 would be no number)
-                acc += (q + WS * j + ws <= q1 ? x[j] : kvm_f32x4{0.f, 0.f, 0.f, 0.f}) * wgt;
+                acc += x[j] * wgt;
             }
             M = mb;
         }
