@@ -38,6 +38,7 @@
 // 100 x 8,192: 54.3 -> 40; 700 x 8,192 on an f16 cache of 2 heads x 128: 48 -> 43).
 #include "kvm_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #define KVM_PF_LAZY 8.0f         // log2 growth of a row max tolerated before a rescale
@@ -189,6 +190,7 @@ struct pf_args {
     uint32_t n_tiles, n_seg, H, G, n_head, n_rows, n_row_tiles;
     float c;                     // kq_scale * log2(e)
     int q_bf16;
+    int longest;                 // whole units, more than the CUs: pf_longest
 };
 
 // The row tile of a unit.  With more units than workgroups a workgroup has several
@@ -198,6 +200,14 @@ struct pf_args {
 // order, 551 here; 24 on 4 x 256, 4,096 tokens (384 units): 326 and 257.
 __device__ __forceinline__ uint32_t pf_row_tile(const pf_args &a, uint32_t i) {
     return a.U > a.P ? (i & 1u ? a.n_row_tiles - 1 - (i >> 1) : i >> 1) : i;
+}
+
+// The unit of the i-th workgroup where each has a whole one and they outnumber the
+// CUs: the last row tiles, which see the most, first, so that what is left at the
+// end is short; the heads of a row tile next to each other, so that an XCD (every
+// eighth workgroup) keeps to few of them.
+__device__ __forceinline__ uint32_t pf_longest(const pf_args &a, uint32_t i) {
+    return i % a.H * a.n_row_tiles + a.n_row_tiles - 1 - i / a.H;
 }
 
 // Q rows of a unit into LDS, coalesced (as operand loads, 32 rows of 32 bytes an
@@ -338,7 +348,8 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
     // Consecutive hardware workgroup ids go round robin over the 8 XCDs; regroup
     // them so one XCD runs consecutive shares, whose K/V tiles its L2 holds.
     uint32_t p = blockIdx.x;
-    if ((a.P & 7u) == 0) p = (p & 7u) * (a.P >> 3) + (p >> 3);
+    if (a.longest) p = pf_longest(a, p);
+    else if ((a.P & 7u) == 0) p = (p & 7u) * (a.P >> 3) + (p >> 3);
     const uint32_t sh0 = p * a.U, sh1 = sh0 + a.U;
     const uint32_t u_first = sh0 / a.P, u_last = (sh1 - 1) / a.P;
 
@@ -643,7 +654,8 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
     const bool consumer = w < 4;
     const uint32_t lds_mem = (uint32_t)(uintptr_t)(kvm_lds_ptr)&s_mem[0];
     uint32_t p = blockIdx.x;
-    if ((a.P & 7u) == 0) p = (p & 7u) * (a.P >> 3) + (p >> 3);       // as k_pf_attn
+    if (a.longest) p = pf_longest(a, p);
+    else if ((a.P & 7u) == 0) p = (p & 7u) * (a.P >> 3) + (p >> 3);       // as k_pf_attn
     const uint32_t sh0 = p * a.U, sh1 = sh0 + a.U;
     const uint32_t u_first = sh0 / a.P, u_last = (sh1 - 1) / a.P;
 
@@ -1090,16 +1102,21 @@ static double pf_tile_us(uint32_t D, int src, uint32_t rows) {
     return (rows == 256 ? 3.3 : src == PF_QUANT ? 1.75 : 1.6) * D / 256;
 }
 
-// Workgroups that U units of n_tiles tiles are dealt to, at most one per CU (LDS).
-// The same number s for every unit, so that none has two pieces (a second piece
-// costs its workgroup another start and end, PF_START us: 100 tokens over 32
-// tiles, 20 units, took 39.9 us on 256 workgroups, 29.3 on 220), unless so many
-// CUs would idle that the second piece is cheaper.  Each piece is written and read
-// once more, `piece` us of all (500 tokens over 16 tiles of 128 dims, 32 units:
-// 30.2 us in 256 pieces, 22.8 in 128).
+// Workgroups that U units of n_tiles tiles are dealt to: equal shares to one per CU
+// (LDS), or one whole unit each.  The same number s for every unit, so that none has
+// two pieces (a second piece costs its workgroup another start and end, PF_START us:
+// 100 tokens over 32 tiles, 20 units, took 39.9 us on 256 workgroups, 29.3 on 220),
+// unless so many CUs would idle that the second piece is cheaper.  Each piece is
+// written and read once more, `piece` us of all (500 tokens over 16 tiles of 128
+// dims, 32 units: 30.2 us in 256 pieces, 22.8 in 128): over few tiles that costs more
+// than a last round of whole units that does not fill the chip (64 heads on 8 x 128,
+// 1,500 tokens, 376 units: over 2,048 cells 112 us in shares, 92.6 whole; over 8,192
+// 399 and 426).  More units than CUs even out over the chip, so `seen` counts there:
+// the tiles that a unit sees on the average, if the chunk is the window's last cells.
 #define PF_START 8.0
-static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double t, double piece, uint32_t n_cu) {
-    double best = PF_START + t * n_tiles * U / n_cu + piece * (U < n_cu ? n_cu + U : 2.0 * n_cu);
+static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double seen, double t, double piece, uint32_t n_cu) {
+    double best = t * (U > n_cu ? seen : n_tiles) * U / n_cu;
+    if (U % n_cu) best += PF_START + piece * (U < n_cu ? n_cu + U : 2.0 * n_cu);
     uint32_t P = n_cu;
     for (uint64_t s = 1; s * U <= n_cu && s <= n_tiles; ++s) {
         const double c = t * kvm_cdiv(n_tiles, s) + (s > 1 ? piece * (s * U) : 0.0);
@@ -1108,6 +1125,7 @@ static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double t, double piece, 
             P = (uint32_t)(s * U);
         }
     }
+    if (U > n_cu && U < 65536 && t * std::max((double)n_tiles, seen * kvm_cdiv(U, n_cu)) < best) P = (uint32_t)U;
     return P;
 }
 // A piece's partial output, written and read at the rate that such launches reach.
@@ -1127,7 +1145,9 @@ struct pf_shape {
     uint32_t src, rows, n_row_tiles, n_seg, U, P;
     uint64_t slots;
 };
-static int pf_shape_of(bool quant, uint32_t D, uint32_t H, uint32_t n_tiles, uint64_t n_rows, uint32_t n_cu, pf_shape *s) {
+static int pf_shape_of(bool quant, uint32_t D, uint32_t H, uint32_t n_tiles, uint32_t n_tokens, uint32_t G, uint32_t n_cu,
+                       pf_shape *s) {
+    const uint64_t n_rows = (uint64_t)n_tokens * G;
     s->n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
     const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / n_cu >= PF_LONG;
     s->rows = long_work ? 256u : 128u;
@@ -1136,7 +1156,9 @@ static int pf_shape_of(bool quant, uint32_t D, uint32_t H, uint32_t n_tiles, uin
     const uint64_t units = (uint64_t)s->n_row_tiles * H * s->n_seg;
     if (units > (1u << 30)) return KVM_ERANGE;
     s->U = (uint32_t)units;
-    uint64_t P = pf_shares(units, kvm_cdiv(n_tiles, s->n_seg), pf_tile_us(D, s->src, s->rows),
+    const uint32_t seg_tiles = kvm_cdiv(n_tiles, s->n_seg);
+    const double own = std::min(1.0, (double)n_tokens / ((double)n_tiles * KVM_TILE_CELLS));
+    uint64_t P = pf_shares(units, seg_tiles, seg_tiles * (1.0 - own / 2), pf_tile_us(D, s->src, s->rows),
                            pf_piece_us(D, n_rows, s->n_row_tiles), n_cu);
     // KVM_PF_SPLITS in the environment fixes the pieces per unit
     if (const char *e = getenv("KVM_PF_SPLITS")) {
@@ -1154,7 +1176,7 @@ extern "C" int kvm_fa_prefill_shape(int k_type, uint32_t head_dim, uint32_t n_he
                                     uint32_t n_tokens, uint32_t n_head, uint32_t n_cu, uint32_t out[7]) {
     pf_shape s{};
     const int rc = pf_shape_of(kvm_k_quant(k_type), head_dim, n_head_kv, n_cells / KVM_TILE_CELLS,
-                               (uint64_t)n_tokens * (n_head / n_head_kv), n_cu, &s);
+                               n_tokens, n_head / n_head_kv, n_cu, &s);
     const uint32_t v[7] = {s.src, s.rows, s.n_row_tiles, s.n_seg, s.U, s.P, (uint32_t)s.slots};
     for (int i = 0; i < 7; ++i) out[i] = v[i];
     return rc;
@@ -1181,7 +1203,7 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     const uint64_t n_rows = (uint64_t)n_tokens * G;
     if (n_rows > (1u << 30)) return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
     pf_shape sh{};
-    if (pf_shape_of(kvm_k_quant(w->k_type), D, H, n_tiles, n_rows, st->n_cu, &sh))
+    if (pf_shape_of(kvm_k_quant(w->k_type), D, H, n_tiles, n_tokens, G, st->n_cu, &sh))
         return kvm_fail(st, KVM_ERANGE, "fa_prefill: %u tokens", n_tokens);
     const int src = (int)sh.src;
     const uint32_t rows = sh.rows;
@@ -1198,6 +1220,7 @@ extern "C" int kvm_fa_prefill(kvm_state *st, const kvm_window *w, const void *q,
     a.P = sh.P;
     a.c = scale * 1.4426950408889634f;
     a.q_bf16 = q_type == KVM_TYPE_BF16;
+    a.longest = a.U == a.P && a.P > st->n_cu && a.n_seg == 1;
     a.q = q;
     a.q_pos = q_pos;
     a.out = out;

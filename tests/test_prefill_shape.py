@@ -11,6 +11,13 @@ lib = L.load()
 lib.kvm_fa_prefill_slot.restype = lib.kvm_fa_prefill_slots.restype = C.c_uint32
 
 
+def prefill_shape(k_type, head_dim, n_head_kv, n_cells, n_tokens, n_head, n_cu):
+    """(source, rows of a unit, row tiles, segments, units, workgroups, slots) of a launch."""
+    out = (C.c_uint32 * 7)()
+    assert lib.kvm_fa_prefill_shape(k_type, head_dim, n_head_kv, n_cells, n_tokens, n_head, n_cu, out) == 0
+    return list(out)
+
+
 def _pieces(U, P):
     """(workgroup, unit, whole) of every piece: workgroup p has [p U, (p + 1) U) of U P, unit u [u P, (u + 1) P)."""
     for p in range(P):
@@ -43,9 +50,17 @@ def test_pieces_have_slots_of_their_own(n_seg):
 
 @pytest.mark.parametrize("n_cells,H,G,D,T", [(525312, 4, 6, 256, 2100), (525312, 8, 4, 128, 1160), (1048640, 4, 6, 256, 2048)])
 def test_segmented_windows_with_more_units_than_workgroups(n_cells, H, G, D, T):
-    out = (C.c_uint32 * 7)()
-    assert lib.kvm_fa_prefill_shape(L.T_Q8_0, D, H, n_cells, T, H * G, 256, out) == 0
-    src, rows, n_row_tiles, n_seg, U, P, slots = out
+    src, rows, n_row_tiles, n_seg, U, P, slots = prefill_shape(L.T_Q8_0, D, H, n_cells, T, H * G, 256)
     assert n_seg > 1 and U > P and U % P and U == n_row_tiles * H * n_seg
     assert slots == lib.kvm_fa_prefill_slots(U, P, n_seg)
     _check(U, P, n_seg)
+
+
+@pytest.mark.parametrize("n_cells,T,want", [(2048, 1500, 376), (4096, 1500, 376), (8192, 1500, 256), (2048, 2048, 256)])
+def test_units_that_outnumber_the_cus(n_cells, T, want):
+    """Whole units over few tiles (376 of 256 rows), equal shares over many and where
+    the units fill every round (512)."""
+    _, _, _, _, U, P, slots = prefill_shape(L.T_F16, 128, 8, n_cells, T, 64, 256)
+    assert P == want and U == (376 if T == 1500 else 512)
+    assert slots == (512 if U % P else 0)
+    _check(U, P, 1)
