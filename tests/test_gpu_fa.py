@@ -7,6 +7,7 @@ import torch
 import oracle as O
 from gpu_util import check_attention, dev, host, rand_rows
 from kvmem_amd import api, _lib as L
+from test_prefill_shape import prefill_shape
 
 pytestmark = pytest.mark.gpu
 
@@ -294,27 +295,41 @@ def test_fa_decode_rejects_wide_batches(kvm_state):
         api.fa_decode(kvm_state, w, q, dev(np.zeros(6, np.int32)), 24, 0.0625)
 
 
+STAGED, F16, QUANT = range(3)                            # where the tiles come from
+CUT, SHARES, WHOLE = "cut", "shares", "whole"             # units over the workgroups: U <= P, U > P, U = P > CUs
 PREFILL_EDGES = [
-    # n_cells, H, G, D, tokens, kt, vt, live cells (None = all), splits, q dtype
-    (128, 1, 11, 128, 3, L.T_Q8_0, L.T_Q4_0, None, None, "f32"),      # 33 rows over two tiles
-    (256, 2, 11, 256, 3, L.T_Q4_0, L.T_Q4_0, 130, None, "bf16"),      # a tile with two live cells
-    (1024, 1, 3, 256, 43, L.T_F16, L.T_F16, None, None, "f32"),       # 129 rows: a second, nearly empty row tile
-    (2048, 2, 8, 128, 32, L.T_F16, L.T_F16, 1100, None, "bf16"),      # 256 rows, half the window empty
-    (38400, 1, 6, 128, 10, L.T_Q8_0, L.T_Q4_0, 37000, None, "bf16"),  # more tiles than one look at the cells
-    (1024, 4, 6, 256, 200, L.T_Q8_0, L.T_Q4_0, None, None, "f32"),    # window converted ahead
-    (768, 2, 6, 256, 100, L.T_Q8_0, L.T_Q4_0, None, 8, "bf16"),       # more pieces of a unit than its rows see tiles
-    (4096, 8, 4, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16"),  # 256-row units, more of them than CUs
-    (4096, 8, 4, 256, 1100, L.T_F16, L.T_F16, 3900, None, "f32"),     # the same, Q in two passes
+    # n_cells, H, G, D, tokens, kt, vt, live cells (None = all), splits, q dtype, (source, rows of a unit, units)
+    (128, 1, 11, 128, 3, L.T_Q8_0, L.T_Q4_0, None, None, "f32", (QUANT, 128, CUT)),       # 33 rows over two tiles
+    (256, 2, 11, 256, 3, L.T_Q4_0, L.T_Q4_0, 130, None, "bf16", (QUANT, 128, CUT)),       # a tile with two live cells
+    (1024, 1, 3, 256, 43, L.T_F16, L.T_F16, None, None, "f32", (F16, 128, CUT)),          # 129 rows: a second, nearly empty row tile
+    (2048, 2, 8, 128, 32, L.T_F16, L.T_F16, 1100, None, "bf16", (F16, 128, CUT)),         # 256 rows, half the window empty
+    (38400, 1, 6, 128, 10, L.T_Q8_0, L.T_Q4_0, 37000, None, "bf16", (QUANT, 128, CUT)),   # more tiles than one look at the cells
+    (1024, 4, 6, 256, 200, L.T_Q8_0, L.T_Q4_0, None, None, "f32", (QUANT, 128, CUT)),     # f32 rows of 256 dims
+    (4096, 8, 4, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (STAGED, 256, CUT)),  # units cut at any place
+    (4096, 8, 4, 256, 1100, L.T_F16, L.T_F16, 3900, None, "f32", (F16, 256, CUT)),
+    (8192, 4, 6, 256, 700, L.T_Q8_0, L.T_Q4_0, None, None, "f32", (STAGED, 256, CUT)),    # window converted ahead, Q in two passes
+    (32768, 4, 6, 256, 200, L.T_Q8_0, L.T_Q4_0, 700, None, "bf16", (STAGED, 256, CUT)),   # the same, most of the window empty
+    (768, 2, 6, 256, 100, L.T_Q8_0, L.T_Q4_0, None, 8, "bf16", (QUANT, 128, CUT)),        # more pieces of a unit than its rows see tiles
+    (3712, 8, 4, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (QUANT, 128, SHARES)),  # 128-row units, more of them than CUs
+    (1536, 8, 4, 128, 1100, L.T_Q4_0, L.T_Q4_0, 1400, None, "f32", (QUANT, 128, WHOLE)),    # the same over few tiles
+    (8192, 8, 8, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (STAGED, 256, SHARES)),  # 256-row units, more of them than CUs
+    (4096, 8, 6, 256, 1400, L.T_F16, L.T_F16, 3900, None, "f32", (F16, 256, SHARES)),       # the same, Q in two passes
+    (2048, 8, 8, 128, 1500, L.T_F16, L.T_F16, None, None, "bf16", (F16, 256, WHOLE)),       # the same over few tiles
 ]
 
 
 @pytest.mark.parametrize("case", range(len(PREFILL_EDGES)))
 def test_fa_prefill_edges(kvm_state, case, monkeypatch):
-    """Row and key remainders, every source of the tiles and both unit sizes, at
-    sampled tokens; the first token sees nothing."""
-    n, H, G, D, T, kt, vt, live, splits, qdt = PREFILL_EDGES[case]
+    """Row and key remainders, every source of the tiles, both unit sizes and every way
+    the units are dealt, at sampled tokens; the first token sees nothing."""
+    n, H, G, D, T, kt, vt, live, splits, qdt, (want_src, want_rows, want_units) = PREFILL_EDGES[case]
     if splits is not None:
         monkeypatch.setenv("KVM_PF_SPLITS", str(splits))
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    src, rows, _, _, U, P, _ = prefill_shape(kt, D, H, n, T, H * G, n_cu)
+    if n_cu == 256:
+        units = SHARES if U > P else WHOLE if U == P > n_cu else CUT
+        assert (src, rows, units) == (want_src, want_rows, want_units) and (units != SHARES or U % P), (src, rows, U, P)
     rng = np.random.default_rng(300 + case)
     w, kr, vr, cp = _window(kvm_state, rng, n, H, D, kt, vt, live=live)
     last = n if live is None else live
@@ -324,7 +339,10 @@ def test_fa_prefill_edges(kvm_state, case, monkeypatch):
     q = q.to(torch.bfloat16) if qdt == "bf16" else q
     out = host(api.fa_prefill(kvm_state, w, q.cuda(), dev(pos), H * G, D ** -0.5))
     assert np.isfinite(out).all() and np.all(out[0] == 0)
-    toks = np.unique(np.r_[1, 2, T // 2, T - 2, T - 1])
+    # two tokens of each of some row tiles: the first, the last ones and some between
+    rt = np.unique(np.linspace(0, (T * G - 1) // rows, 9).astype(int))
+    toks = np.unique(np.r_[1, 2, T // 2, T - 2, T - 1, np.minimum(T - 1, -(-rt * rows // G))])
+    toks = toks[toks > 0]
     _prefill_check(out[toks], q.float().numpy()[toks], kr, vr, cp, pos[toks], H, G, D, kt, vt, D ** -0.5)
 
 
