@@ -1139,7 +1139,18 @@ static double pf_piece_us(uint32_t D, uint64_t n_rows, uint32_t row_tiles) {
 // 256 rows, 944 with 128; 1,000 x 128, 4 x 256: 201 and 215; 300 x 128, 4 x 256: 87
 // and 78; 37 x 544, 4 x 256: 99 and 54; on an f16 window 1,000 x 256, 8 x 128: 255
 // and 271; 700 x 144, 2 x 128: 48 and 41.
+// - PF_TIGHT instead, where the 256-row units fill the chip with one or two workgroups
+//   each: the last row tiles then bound the call, and smaller units leave their
+//   workgroups less (1,024 x 64, 8 x 128, 128 units: 87 and 84, and in a chunk that
+//   is alone in the window 43 and 29; 2,048 x 32, 256 units: 70 and 58; from twice
+//   that many tiles on 256 rows win, 1,024 x 128: 147 and 160).
+// - A quantised window keeps 128 rows up to PF_FEW row tiles of 256: converting it
+//   ahead costs more than so few of them save (32 heads, no groups, 128 dims: 200
+//   x 256, one row tile, 144 and 98; 1,024 x 128, four, 182 and 166; 1,500 x 128,
+//   six, 241 and 243).
 #define PF_LONG 64.0
+#define PF_TIGHT 112.0
+#define PF_FEW 4u
 
 struct pf_shape {
     uint32_t src, rows, n_row_tiles, n_seg, U, P;
@@ -1149,7 +1160,10 @@ static int pf_shape_of(bool quant, uint32_t D, uint32_t H, uint32_t n_tiles, uin
                        pf_shape *s) {
     const uint64_t n_rows = (uint64_t)n_tokens * G;
     s->n_seg = kvm_cdiv(n_tiles, KVM_PF_LIST);
-    const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / n_cu >= PF_LONG;
+    const uint64_t rt256 = kvm_cdiv(n_rows, 256), wgs = rt256 * H <= n_cu ? n_cu / (rt256 * H) : 0;      // workgroups a unit
+    const bool tight = (wgs == 1 || wgs == 2) && wgs * rt256 * H * 8 >= 7u * n_cu;
+    const bool long_work = (double)kvm_cdiv(n_rows, 128) * H * n_tiles / n_cu >= (tight ? PF_TIGHT : PF_LONG) &&
+                           !(quant && rt256 <= PF_FEW);
     s->rows = long_work ? 256u : 128u;
     s->src = !quant ? PF_F16 : long_work ? PF_STAGED : PF_QUANT;
     s->n_row_tiles = (uint32_t)kvm_cdiv(n_rows, s->rows);

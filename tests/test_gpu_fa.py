@@ -375,13 +375,17 @@ def test_fa_prefill_query_alignment(kvm_state, kt, vt, qdt):
     assert np.array_equal(got, want)
 
 
-def test_fa_prefill_segments_with_more_units_than_workgroups(kvm_state):
+@pytest.mark.parametrize("H,G,T,rows", [(8, 4, 1160, 256), (20, 1, 1000, 128)])
+def test_fa_prefill_segments_with_more_units_than_workgroups(kvm_state, H, G, T, rows):
     """A window of two segments whose units outnumber the workgroups: a share then
     spans more than one whole unit, and every one of its pieces has a place of its
     own.  Few cells are live, in both segments; two tokens of each row tile, all
     heads (so every unit is looked at)."""
     rng = np.random.default_rng(78)
-    H, G, D, T, n, cut = 8, 4, 128, 1160, 525312, 524288
+    D, n, cut = 128, 525312, 524288
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    _, got, _, n_seg, U, P, _ = prefill_shape(L.T_Q8_0, D, H, n, T, H * G, n_cu)
+    assert n_cu != 256 or (got == rows and n_seg == 2 and U > P and U % P)
     w = api.KVWindow(kvm_state, n, H, D, 128, L.T_Q8_0, L.T_Q4_0)
     kr, vr = rand_rows(rng, 2048 + n - cut, H, D, L.T_Q8_0, L.T_Q4_0)
     cp = np.arange(kr.shape[0], dtype=np.int32)

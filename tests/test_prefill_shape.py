@@ -64,3 +64,16 @@ def test_units_that_outnumber_the_cus(n_cells, T, want):
     assert P == want and U == (376 if T == 1500 else 512)
     assert slots == (512 if U % P else 0)
     _check(U, P, 1)
+
+
+@pytest.mark.parametrize("kt,D,H,G,n_cells,T,rows", [
+    (L.T_Q8_0, 128, 8, 4, 4096, 1024, 128), (L.T_Q8_0, 128, 8, 4, 8192, 1024, 256),      # two workgroups a unit
+    (L.T_F16, 128, 8, 4, 2048, 2048, 128), (L.T_F16, 128, 8, 4, 8192, 2048, 256),        # one
+    (L.T_Q4_0, 256, 4, 6, 32768, 170, 128), (L.T_Q4_0, 256, 4, 6, 32768, 171, 256),      # four row tiles of 256 rows, five
+    (L.T_F16, 256, 4, 6, 32768, 170, 256),
+])
+def test_rows_of_a_unit(kt, D, H, G, n_cells, T, rows):
+    """Both sides of the rules that choose between 128- and 256-row units."""
+    src, got, *_ = prefill_shape(kt, D, H, n_cells, T, H * G, 256)
+    assert got == rows
+    assert src == (1 if kt == L.T_F16 else 0 if rows == 256 else 2)       # f16 window, converted ahead, by the attention
