@@ -260,21 +260,26 @@ __device__ __forceinline__ void import_v_f16(const import_args &a, uint64_t i) {
         x[j] = load_any<kvm_u32x4>(a.v_rows + ((t * g.H + h) * D + 8 * u) * 2);
     }
     uint16_t *dst = (uint16_t *)(g.v + ((uint64_t)h * g.n_tiles + tile) * g.vtile);
-    const bool full = c0 >= a.cell0 && c0 + 8 <= end;
+    uint16_t *o[8];
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
-        uint16_t *o = dst + kvm_vh_idx((uint32_t)(c0 % 64), 8 * u + d);
-        if (full) {
+    for (int d = 0; d < 8; ++d) o[d] = dst + kvm_vh_idx((uint32_t)(c0 % 64), 8 * u + d);
+    if (c0 >= a.cell0 && c0 + 8 <= end) {
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
             kvm_u32x4 y;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 y[j] = __builtin_amdgcn_perm(x[2 * j + 1][d >> 1], x[2 * j][d >> 1], d & 1 ? 0x07060302u : 0x05040100u);
-            *(kvm_u32x4 *)o = y;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (c0 + j >= a.cell0 && c0 + j < end) o[j] = (uint16_t)(x[j][d >> 1] >> (16 * (d & 1)));
+            *(kvm_u32x4 *)o[d] = y;
         }
+    } else {
+        // the first or last group: a branch for each cell, not for each value
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (c0 + j >= a.cell0 && c0 + j < end) {
+#pragma unroll
+                for (int d = 0; d < 8; ++d) o[d][j] = (uint16_t)(x[j][d >> 1] >> (16 * (d & 1)));
+            }
     }
 }
 
