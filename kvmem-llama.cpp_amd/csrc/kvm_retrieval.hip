@@ -72,13 +72,12 @@ __device__ __forceinline__ float ordered_sum(const float *x) {
     return s;
 }
 
-// Any view: one thread per embedding, its rows in order.  The loads of 16 rows
+// Any view: one thread per embedding, its rows in order.  The loads of B rows
 // are issued together (unconditional: rows past the last re-read it, and rows
-// the mask leaves out are read but not added), one memory round trip per 16
-// rows instead of one per row.
-template <int T>
+// the mask leaves out are read but not added), one memory round trip per B rows
+// instead of one per row: 16, or 4 for up to 4 rows.
+template <int T, uint32_t B>
 __global__ void __launch_bounds__(64) k_query_add(qview_args a) {
-    constexpr uint32_t B = 16;
     const uint32_t e = blockIdx.x * 64u + threadIdx.x;
     if (e < a.n_embd) {
         const uint8_t *p = a.v.data + (size_t)a.t0 * a.v.nb2 + view_off(a.v, e);
@@ -381,8 +380,10 @@ extern "C" int kvm_query_add_view(kvm_state *st, const kvm_query_acc *acc, uint3
                                    acc->n_head / acc->n_head_kv);
             else if (rows_ok && a.n_rows > KVM_QROWS_MIN)
                 hipLaunchKernelGGL(k_query_add_rows<T>, dim3(n_embd / 32), dim3(320), 0, st->stream, a);
+            else if (a.n_rows <= 4u)
+                hipLaunchKernelGGL((k_query_add<T, 4>), dim3(kvm_cdiv(n_embd, 64)), dim3(64), 0, st->stream, a);
             else
-                hipLaunchKernelGGL(k_query_add<T>, dim3(kvm_cdiv(n_embd, 64)), dim3(64), 0, st->stream, a);
+                hipLaunchKernelGGL((k_query_add<T, 16>), dim3(kvm_cdiv(n_embd, 64)), dim3(64), 0, st->stream, a);
         };
         if (q->type == KVM_TYPE_F16) go(std::integral_constant<int, KVM_TYPE_F16>{});
         else if (q->type == KVM_TYPE_BF16) go(std::integral_constant<int, KVM_TYPE_BF16>{});
@@ -422,13 +423,17 @@ extern "C" size_t kvm_meank_k_sum_floats(const kvm_meank_index *ix) {
 // One block's share (chunk ci = blockIdx.y of the positions pos0 .. pos0+n-1)
 // of 256 embeddings per workgroup; the view's token pos - pos0 + tok0 holds
 // position pos.  What bounds it is the memory round trips of a block's ordered
-// rows, so the loads of 64 rows are issued together (unconditional: rows past
-// the share re-read its last one): two round trips for a 128-token block.  TD:
+// rows, so the loads of B rows are issued together (unconditional: rows past
+// the share re-read its last one): 64, two round trips for a 128-token block; 8 in
+// calls of up to KVM_MEANK_FEW tokens, where reading the last row again up to 64
+// times takes longer than more trips (4 x 256 f32 values without terms: 1 token 4.03
+// us with 64, 2.23 with 8; 24 tokens 4.05 and 2.85; a trip 0.31); 2 up to 2 tokens.  TD:
 // 0, or the head_dim (128, 256) of an index that carries the block terms, whose
 // new nk the workgroup then forms from its sums (256 / TD heads) as
 // k_meank_terms does, without a launch of its own.  A 2,048-token bf16 chunk of
 // 4 x 256 values took 40 us with a load in flight at a time, and 4.8 for the
 // terms' launch.
+#define KVM_MEANK_FEW 48u
 struct meank_add_args {
     float *k_sum;
     uint32_t *mean_tokens;
@@ -437,9 +442,8 @@ struct meank_add_args {
     view_args v;
     uint32_t cap, n_embd, bt, pos0, n, tok0;
 };
-template <int T, int TD>
+template <int T, int TD, uint32_t B>
 __global__ void __launch_bounds__(256) k_meank_add(meank_add_args a) {
-    constexpr uint32_t B = 64;
     const uint32_t tid = threadIdx.x, e = blockIdx.x * 256u + tid;
     const uint32_t ci = blockIdx.y;                  // chunk = one block's share
     const uint32_t bid = a.pos0 / a.bt + ci;
@@ -563,9 +567,15 @@ static int meank_add_view(kvm_state *st, const kvm_meank_index *ix, uint32_t il,
     const dim3 grid(kvm_cdiv(n_embd, 256), n_chunks);
     auto go = [&](auto t) {
         constexpr int T = decltype(t)::value;
-        if (!ix->k_norm) hipLaunchKernelGGL((k_meank_add<T, 0>), grid, dim3(256), 0, st->stream, a);
-        else if (ix->head_dim == 256) hipLaunchKernelGGL((k_meank_add<T, 256>), grid, dim3(256), 0, st->stream, a);
-        else hipLaunchKernelGGL((k_meank_add<T, 128>), grid, dim3(256), 0, st->stream, a);
+        auto go_b = [&](auto rows) {
+            constexpr uint32_t B = decltype(rows)::value;
+            if (!ix->k_norm) hipLaunchKernelGGL((k_meank_add<T, 0, B>), grid, dim3(256), 0, st->stream, a);
+            else if (ix->head_dim == 256) hipLaunchKernelGGL((k_meank_add<T, 256, B>), grid, dim3(256), 0, st->stream, a);
+            else hipLaunchKernelGGL((k_meank_add<T, 128, B>), grid, dim3(256), 0, st->stream, a);
+        };
+        if (n <= 2u) go_b(std::integral_constant<uint32_t, 2>{});
+        else if (n <= KVM_MEANK_FEW) go_b(std::integral_constant<uint32_t, 8>{});
+        else go_b(std::integral_constant<uint32_t, 64>{});
     };
     if (k->type == KVM_TYPE_F16) go(std::integral_constant<int, KVM_TYPE_F16>{});
     else if (k->type == KVM_TYPE_BF16) go(std::integral_constant<int, KVM_TYPE_BF16>{});

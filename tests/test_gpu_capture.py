@@ -87,6 +87,24 @@ def test_query_add_view_long_runs(kvm_state, dt, n, offset):
     assert int(qa.q_count[0]) == int(keep.sum())
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 16, 17, 31])
+def test_query_add_view_few_rows(kvm_state, n):
+    """Row counts around the general form's loads in flight (4, 16), with and without
+    a mask whose last row is kept."""
+    rng = np.random.default_rng(n)
+    qa = api.QueryAcc(kvm_state, 1, 3, 128)
+    qa.reset()
+    q = _captured(rng, n, 3, 128, "bf16", "heads_major")
+    keep = rng.random(n) < 0.5
+    keep[-1] = True
+    qa.add_view(0, q, keep)
+    qa.add_view(0, q)
+    rows = _f32_rows(q)
+    want = _ordered_sum(np.zeros(384, np.float32), list(rows[keep]) + list(rows))
+    assert np.array_equal(host(qa.q_sum)[0].view(np.uint32), want.view(np.uint32))
+    assert int(host(qa.q_count)[0]) == int(keep.sum()) + n
+
+
 def test_query_add_view_more_rows_than_one_launch(kvm_state):
     rng = np.random.default_rng(5)
     qa = api.QueryAcc(kvm_state, 1, 2, 128)
@@ -142,6 +160,30 @@ def test_meank_add_forms_block_terms(kvm_state, H, D, bt, dt):
     assert bool((got[0, :, 5] == -1.0).all())
     ix.refresh()
     assert torch.equal(got[0, :, :5].contiguous().view(torch.int32), ix.k_norm[0, :, :5].contiguous().view(torch.int32))
+
+
+@pytest.mark.parametrize("norms", [False, True])
+@pytest.mark.parametrize("n", [1, 2, 3, 8, 9, 47, 48, 49, 64, 65])
+def test_meank_add_token_counts(kvm_state, n, norms):
+    """Token counts around the kernel's loads in flight (2, 8, 64), across the end of
+    a block: the sums in token order, the counts, and the terms of a refresh."""
+    rng = np.random.default_rng(n)
+    H, D, bt = 2, 256, 64
+    ix = api.MeanKIndex(kvm_state, 1, 4, H, D, bt, norms=norms)
+    first = _captured(rng, bt - n // 2, H, D, "f32", "contiguous")
+    k = _captured(rng, n, H, D, "bf16", "strided_dim")
+    ix.add_view(0, 0, first)
+    ix.add_view(0, bt - n // 2, k)
+    rows = np.concatenate([_f32_rows(first), _f32_rows(k)])
+    got = host(ix.block_sums())[0]
+    for b in range(2):
+        want = _ordered_sum(np.zeros(H * D, np.float32), rows[b * bt:(b + 1) * bt])
+        assert np.array_equal(got[b].view(np.uint32), want.view(np.uint32)), b
+    assert list(host(ix.mean_tokens)[0][:2]) == [bt, len(rows) - bt]
+    if norms:
+        terms = ix.k_norm.clone()
+        ix.refresh()
+        assert torch.equal(terms.view(torch.int32), ix.k_norm.view(torch.int32))
 
 
 def test_meank_decode_running_sum_and_flush(kvm_state):
