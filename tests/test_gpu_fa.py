@@ -375,6 +375,27 @@ def test_fa_prefill_query_alignment(kvm_state, kt, vt, qdt):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("D,T", [(128, 9), (256, 300)])
+def test_fa_prefill_window_alignment(kvm_state, D, T):
+    """An f16 window whose buffers start anywhere in memory (a copy of it is read)
+    gives the aligned one's output."""
+    rng = np.random.default_rng(20)
+    H, G, n = 2, 6, 4096
+    w, *_ = _window(kvm_state, rng, n, H, D, L.T_F16, L.T_F16, holes=50)
+    q = dev(rng.standard_normal((T, H * G, D)).astype(np.float32))
+    pos = dev(np.arange(n - T, n, dtype=np.int32))
+    want = host(api.fa_prefill(kvm_state, w, q, pos, H * G, D ** -0.5))
+    for dk, dv in ((2, 0), (0, 4), (8, 6)):
+        bufs = []
+        for src, off in ((w.k, dk), (w.v, dv)):
+            bufs.append(torch.zeros(src.numel() + 16, dtype=torch.uint8, device="cuda"))
+            bufs[-1][off:off + src.numel()] = src
+        w.c.k, w.c.v = bufs[0].data_ptr() + dk, bufs[1].data_ptr() + dv
+        got = host(api.fa_prefill(kvm_state, w, q, pos, H * G, D ** -0.5))
+        w.c.k, w.c.v = w.k.data_ptr(), w.v.data_ptr()
+        assert np.array_equal(got, want), (dk, dv)
+
+
 @pytest.mark.parametrize("H,G,T,rows", [(8, 4, 1160, 256), (20, 1, 1000, 128)])
 def test_fa_prefill_segments_with_more_units_than_workgroups(kvm_state, H, G, T, rows):
     """A window of two segments whose units outnumber the workgroups: a share then
