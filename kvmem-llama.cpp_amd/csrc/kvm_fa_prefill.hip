@@ -632,6 +632,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
 // cells 61.6 -> 54 us, 64 x 4,096 of 8 heads x 128 28 -> 22.5.)
 template <int D, int SRC, bool BF16>
 __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
+    static_assert(SRC == PF_F16 || SRC == PF_QUANT, "a window is converted ahead for 256-row units only");
     constexpr int ROWS = 128;
     constexpr int KS = D / 16, DT = D / 32, NB = D / 32;  // k-steps of a score; MFMAs of a sub tile's P V: 2 DT = KS
     constexpr uint32_t TILE_B = 128u * D;                 // bytes of an f16 K (or V) tile
@@ -856,7 +857,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
             const int pw = w - 4;
             auto tile = [&](uint32_t k) { return t_begin + (__builtin_amdgcn_readfirstlane((uint32_t)s_front.list[k < n_t ? k : n_t - 1]) & 0x7fffu); };
             auto cells_to = [&](uint32_t t) { return a.cell_pos[(uint64_t)t * 64 + l]; };
-            if constexpr (SRC != PF_QUANT) {
+            if constexpr (SRC == PF_F16) {
                 // Copies go global -> LDS directly (global_load_lds_dwordx4: lane l
                 // writes 16 bytes at M0 + 16 l), issued from asm so the compiler adds
                 // no wait for them; the wait is before the barrier.  The asm restores
@@ -879,8 +880,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
 #pragma unroll
                     for (int i = 0; i < NC; ++i) {
                         const uint32_t x = pw * NC + i;   // key half, dim tile
-                        const uint8_t *src = SRC == PF_F16 ? vt + (x % (D / 16)) * 2048u + (x / (D / 16)) * 16u : vt + x * 1024u;
-                        copy((SRC == PF_F16 ? 32u : 16u) * opaque(l), dst + TILE_B + x * 1024u, src);
+                        copy(32u * opaque(l), dst + TILE_B + x * 1024u, vt + (x % (D / 16)) * 2048u + (x / (D / 16)) * 16u);
                     }
                 };
                 if constexpr (!Q_EARLY) KVM_LDS_BARRIER();
