@@ -33,10 +33,11 @@
 // f16 tiles: K as kvm_kh_idx; V units of 8 keys of a dim (as kvm_vh_idx), in LDS
 // and in the workspace in the order [32-key half][16-dim tile][8-key group][dim].
 // What bounds it: large chunks, the matrix cores at the clock that the power limit
-// leaves (2,048 tokens x 34,816 cells, 16 rows a wave and this: 1.05 -> 1.14 PFLOP/s,
-// a large f16 matrix product reaches 1.33); small ones, the attention waves' chain, the
-// latencies of the start and the piece traffic (37 tokens x 32,768 cells: 152 -> 52 us;
-// 100 x 8,192: 54.3 -> 40; 700 x 8,192 on an f16 cache of 2 heads x 128: 48 -> 43).
+// leaves (2,048 tokens x 34,816 cells, 16 rows a wave and this: 1.02 -> 1.10 PFLOP/s on
+// one card, where a large f16 matrix product reaches 1.33; the matrix cores are busy 0.66
+// of the cycles, the LDS 0.33); small ones, the attention waves' chain, the latencies of
+// the start and the piece traffic (37 tokens x 32,768 cells: 152 -> 53 us; 700 x 8,192 on
+// an f16 cache of 2 heads x 128: 49 -> 44).
 #include "kvm_internal.h"
 
 #include <algorithm>
@@ -198,7 +199,7 @@ struct pf_args {
 // after each other, and in a chunk that attends to itself the later rows see more
 // tiles: first and last row tiles take turns, so that shares have like numbers of
 // tiles.  32 heads on 8 x 128, 8,192 tokens (1,024 units, 4 a workgroup): 812 us in row
-// order, 551 here; 24 on 4 x 256, 4,096 tokens (384 units): 326 and 257.
+// order, 551 here; 24 on 4 x 256, 8,192 over 16,384 cells (768 units): 2,414 and 2,117.
 __device__ __forceinline__ uint32_t pf_row_tile(const pf_args &a, uint32_t i) {
     return a.U > a.P ? (i & 1u ? a.n_row_tiles - 1 - (i >> 1) : i >> 1) : i;
 }
@@ -629,7 +630,7 @@ __global__ void __launch_bounds__(512) k_pf_attn(pf_args a) {
 // softmax of a 32-key sub tile is taken between the MFMAs of the next scores or of
 // the P V before.  (Converting between the MFMAs of eight attention waves took 5,300:
 // their LDS writes, 64 bytes a cycle, held up the operand reads.  37 tokens x 32,768
-// cells 61.6 -> 54 us, 64 x 4,096 of 8 heads x 128 28 -> 22.5.)
+// cells 61.6 -> 52.3 us, 64 x 4,096 of 8 heads x 128 28 -> 22.5.)
 template <int D, int SRC, bool BF16>
 __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
     static_assert(SRC == PF_F16 || SRC == PF_QUANT, "a window is converted ahead for 256-row units only");
@@ -1139,10 +1140,12 @@ static double pf_piece_us(uint32_t D, uint64_t n_rows, uint32_t row_tiles) {
 
 // Rows of a unit, and with them the kernel: 256 (k_pf_attn; a quantised window is
 // converted ahead) once a workgroup would have PF_LONG tiles of 128 rows, 128
-// (k_pf_attn_split) below.  1,500 tokens x 512 tiles, 8 heads x 128: 770 us with
-// 256 rows, 944 with 128; 1,000 x 128, 4 x 256: 201 and 215; 300 x 128, 4 x 256: 87
-// and 78; 37 x 544, 4 x 256: 99 and 54; on an f16 window 1,000 x 256, 8 x 128: 255
-// and 271; 700 x 144, 2 x 128: 48 and 41.
+// (k_pf_attn_split) below.  Full windows, us with 256 and with 128 rows: 1,500 tokens x
+// 512 tiles, 4 heads x 256, 1,055 and 1,215; 1,024 x 128, 210 and 236; 400 x 256, 179 and
+// 190; 400 x 128, 106 and 106; 1,024 x 64, 120 and 122; 200 x 256, 114 and 106; on an f16
+// window of 8 x 128, 1,024 x 256, 261 and 285; 1,024 x 32, 51 and 44.  What is live in the
+// window is not known here: chunks that start a large one would rather have 128 rows
+// (1,024 tokens alone in 8,192 cells of 8 x 128: 44 and 29, full 150 and 160).
 // - PF_TIGHT instead, where the 256-row units fill the chip with one or two workgroups
 //   each: the last row tiles then bound the call, and smaller units leave their
 //   workgroups less (1,024 x 64, 8 x 128, 128 units: 87 and 84, and in a chunk that

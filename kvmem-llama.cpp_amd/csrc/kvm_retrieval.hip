@@ -97,14 +97,16 @@ __global__ void __launch_bounds__(64) k_query_add(qview_args a) {
 
 // Many rows of a view whose heads are contiguous and 16-byte aligned
 // (query_rows_ok): a workgroup takes 32 embeddings, and wave 0's lanes add one
-// each, in row order.  What bounds it is that chain (2,048 dependent adds of ~5
-// cycles), so wave 0 does nothing else: waves 1 - 4 load the rows two buffers
-// ahead, convert them and lay them in LDS four rows of an embedding together, and
-// the chain reads 32 rows with 8 loads while it adds the 32 before.  2,048 bf16
-// rows of 24 heads x 256 dims: 23.4 us with the conversions and a load per value
-// in the chain, 18.2 here (678 for one thread per embedding with a load in
-// flight at a time).  The row quads' columns are rotated (by xor) so that the
-// stores of a wave spread over the banks.
+// each, in row order.  Waves 1 - 4 load the rows two buffers ahead, convert them
+// and lay them in LDS four rows of an embedding together, so that wave 0 reads 32
+// rows with 8 loads and only adds.  2,048 bf16 rows of 24 heads x 256 dims: 23.4 us
+// with the conversions and a load per value in the chain, 18.2 here (678 for one
+// thread per embedding with a load in flight at a time).  What bounds it is wave 0:
+// the 2,048 dependent adds are about 4.3 us of it, the rest an LDS and a scalar round
+// trip for every 32 rows.  The reads of the next 32 are issued before these are
+// added, but a keep word's scalar load shares the LDS reads' wait counter, and the
+// compiler waits for both ahead of the adds.  The row quads' columns are rotated (by
+// xor) so that the stores of a wave spread over the banks.
 template <int T>
 __global__ void __launch_bounds__(320) k_query_add_rows(qview_args a) {
     constexpr uint32_t ES = T == KVM_TYPE_F32 ? 4u : 2u, VPU = 16u / ES, UPR = 32u / VPU;   // values of a 16-byte unit, units of a row
