@@ -13,9 +13,9 @@
 // query heads of a kv head share every K/V tile.  A wave has 32 rows: the 32x32x16
 // MFMA reads half the LDS bytes per flop of 16 rows a wave.  A unit is 256 rows of a
 // kv head (k_pf_attn: eight such waves) or 128 (k_pf_attn_split: four, and four that
-// bring the tiles).  The units' keys are dealt to the workgroups in equal shares
-// (pf_shares), so the CUs have the same work whatever the shape; k_pf_combine merges
-// the units that several workgroups share.
+// bring the tiles).  The units' keys are dealt to the workgroups in equal shares, or
+// whole units over few tiles (pf_shares); k_pf_combine merges the units that several
+// workgroups share.
 // S^T = K Q^T and O^T += V^T P^T.  Key order: score row i of a 32-key sub tile is
 // key i with bits 2 and 3 swapped (the lane that supplies K row i reads that key),
 // so that the accumulator holds for each lane the 8 consecutive keys that the P V
@@ -28,7 +28,8 @@
 //             global -> LDS, double buffered;
 //   PF_STAGED the same from a workspace into which k_pf_stage converted the
 //             quantised window: one conversion for all row tiles (256-row units);
-//   PF_QUANT  the quantised tiles, converted by the attention's own waves (128).
+//   PF_QUANT  the quantised tiles, converted by the attention's own waves (128-row
+//             units).
 // f16 tiles: K as kvm_kh_idx; V units of 8 keys of a dim (as kvm_vh_idx), in LDS
 // and in the workspace in the order [32-key half][16-dim tile][8-key group][dim].
 // What bounds it: large chunks, the matrix cores at the clock that the power limit
@@ -979,8 +980,7 @@ __global__ void __launch_bounds__(512) k_pf_attn_split(pf_args a) {
 
 // Merge the pieces of a unit's 32-row group: a lane has 4 dims of a row.  WS waves
 // share the pieces, each with NP pieces' loads in flight, and meet in LDS: what
-// bounds a unit of many pieces is the round trips of its loads (32 pieces of 128
-// rows x 256 dims: 8.1 us with one wave, four trips).
+// bounds a unit of many pieces is the round trips of its loads.
 template <int D, int ROWS, int WS, int NP>
 __global__ void __launch_bounds__(256) k_pf_combine(pf_args a) {
     constexpr uint32_t IB = 4 / WS;
@@ -1077,8 +1077,19 @@ static void pf_attn(const pf_args &a, hipStream_t stream) {
     if (a.q_bf16) go(std::true_type{});
     else go(std::false_type{});
     if (a.n_seg == 1 && a.U % a.P == 0) return;           // every unit whole
+    // The form by the most pieces of a unit (of one of its segments): a call's time, us,
+    // with (waves, loads in flight) = (1, 2), (1, 4), (1, 8), (4, 4), (4, 8).
+    //    2 pieces, 32 units of 128 dims   40.4  40.6  41.1  42.2  44.0
+    //    2, 64 units (shares) of 128      33.1  33.4  34.9  38.7  43.7
+    //    4, 12 units of 256 dims          36.1  35.9  36.6  36.8  38.1
+    //    8, 4 units of 256 dims           25.5  24.8  24.5  24.8  25.3
+    //    8, 2 units of 128 dims           15.4  14.7  14.3  14.4  14.8
+    //   16, 2 units of 128 dims           16.1  14.8  14.2  13.5  14.0
+    //   16, 12 units of 256 dims          25.0  24.1  24.3  24.1  24.9
+    //   32, 1 unit of 128 dims            17.8  15.7  14.6  12.9  12.4
+    //   64, 4 units of 256 dims           33.9  29.4  27.4  25.7  26.0
+    // (A kernel trace does not show it: there every launch takes 4.5 us and more.)
     const dim3 g1(a.n_row_tiles * a.H, ROWS / 32, D / 32), g4(a.n_row_tiles * a.H, ROWS / 32, D / 8), t(256);
-    // most pieces of a unit (of one of its segments)
     const uint32_t n = a.P % a.U == 0 ? a.P / a.U : a.P / a.U + 2;
     if (n <= 2) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 1, 2>), g1, t, 0, stream, a);
     else if (n <= 4) hipLaunchKernelGGL((k_pf_combine<D, ROWS, 1, 4>), g1, t, 0, stream, a);
@@ -1097,8 +1108,10 @@ static void pf_launch(const pf_args &a, const pf_stage_args &sa, int src, uint32
     pf_attn<D, 256, PF_STAGED>(a, stream);
 }
 
-// ---- the launch's shape, from measured costs (us; D 256, half of it at D 128)
-// A 64-cell tile of a unit.
+// ---- the launch's shape, from estimated costs (us)
+// A 64-cell tile of a unit, as measured at D 256; at D 128 half of it is taken, where
+// 1.1 - 1.25 (128 rows) and 2.0 - 2.2 (256) are measured: the lines below were found
+// with these values.
 static double pf_tile_us(uint32_t D, int src, uint32_t rows) {
     return (rows == 256 ? 3.3 : src == PF_QUANT ? 1.75 : 1.6) * D / 256;
 }
