@@ -155,3 +155,39 @@ def test_back_to_back_replays_follow_changing_inputs(kvm_state, monkeypatch, mod
     torch.cuda.synchronize()
     for r in range(n_rep):
         assert torch.equal(outs[r], api.fa_decode(st, w, qs[r], q_pos, H * G, D ** -0.5)), r
+
+
+@pytest.mark.parametrize("kt,vt,D,H,G,n,T,filled", [
+    (L.T_Q8_0, L.T_Q4_0, 256, 4, 6, 8192, 40, 8000),       # pieces, tiles converted by the attention
+    (L.T_Q8_0, L.T_Q4_0, 256, 4, 6, 32768, 200, 3000),     # tiles converted ahead, most of the window empty
+    (L.T_F16, L.T_F16, 128, 8, 8, 2048, 1500, 2048),       # whole units, more than the CUs
+])
+def test_prefill_graph_replays_equal_eager(kvm_state, kt, vt, D, H, G, n, T, filled):
+    """A captured prefill reads the window and the query of each replay: cells filled
+    and emptied between replays, and a new query, give the eager call's bits."""
+    st = kvm_state
+    rng = np.random.default_rng(n + T)
+    w = api.KVWindow(st, n, H, D, 128, kt, vt)
+    kr, vr = rand_rows(rng, min(n, filled + 1000), H, D, kt, vt)
+    w.import_rows(0, dev(kr[:filled]), dev(vr[:filled]), dev(np.arange(filled, dtype=np.int32)))
+    pos = dev(np.arange(filled - T, filled, dtype=np.int32))
+    q = dev(rng.standard_normal((T, H * G, D)).astype(np.float32))
+    out = torch.empty((T, H * G, D), dtype=torch.float32, device="cuda")
+    api.fa_prefill(st, w, q, pos, H * G, D ** -0.5, out)               # sizes the workspace
+    g = st.capture(lambda: api.fa_prefill(st, w, q, pos, H * G, D ** -0.5, out))
+    for r in range(4):
+        q.copy_(dev(rng.standard_normal((T, H * G, D)).astype(np.float32)))
+        if r == 1:                                                     # cells of tiles that were empty, seen by every row
+            m = kr.shape[0] - filled
+            if m:
+                w.import_rows(filled, dev(kr[filled:]), dev(vr[filled:]), dev(np.zeros(m, np.int32)))
+        if r == 2:
+            w.cell_pos[64:640] = -1
+        torch.cuda.synchronize()
+        out.zero_()
+        g.replay()
+        got = out.clone()
+        want = api.fa_prefill(st, w, q, pos, H * G, D ** -0.5)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), r
+        assert bool(torch.isfinite(got).all())
