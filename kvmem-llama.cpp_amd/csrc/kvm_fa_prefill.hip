@@ -1139,7 +1139,11 @@ static uint32_t pf_shares(uint64_t U, uint32_t n_tiles, double seen, double t, d
             P = (uint32_t)(s * U);
         }
     }
-    if (U > n_cu && U < 65536 && t * std::max((double)n_tiles, seen * kvm_cdiv(U, n_cu)) < best) P = (uint32_t)U;
+    // Whole units, longest first: the shortest fill a part of the last round's gap (0.6 as
+    // measured: 32 heads on 8 x 128, 3,000 tokens over 8,192 cells, 376 units, 360 us in
+    // shares and 369 whole; alone in the window 130 and 101).
+    const double least = 2 * seen - n_tiles, gap = kvm_cdiv(U, n_cu) - (double)U / n_cu;
+    if (U > n_cu && U < 65536 && t * std::max((double)n_tiles, seen * U / n_cu + 0.6 * gap * least) < best) P = (uint32_t)U;
     return P;
 }
 // A piece's partial output, written and read at the rate that such launches reach.

@@ -310,11 +310,13 @@ PREFILL_EDGES = [
     (8192, 4, 6, 256, 700, L.T_Q8_0, L.T_Q4_0, None, None, "f32", (STAGED, 256, CUT)),    # window converted ahead, Q in two passes
     (32768, 4, 6, 256, 200, L.T_Q8_0, L.T_Q4_0, 700, None, "bf16", (STAGED, 256, CUT)),   # the same, most of the window empty
     (768, 2, 6, 256, 100, L.T_Q8_0, L.T_Q4_0, None, 8, "bf16", (QUANT, 128, CUT)),        # more pieces of a unit than its rows see tiles
-    (3712, 8, 4, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (QUANT, 128, SHARES)),  # 128-row units, more of them than CUs
-    (1536, 8, 4, 128, 1100, L.T_Q4_0, L.T_Q4_0, 1400, None, "f32", (QUANT, 128, WHOLE)),    # the same over few tiles
+    (8192, 36, 1, 128, 1000, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (QUANT, 128, SHARES)),  # 128-row units, more of them than CUs
+    (3712, 8, 4, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (QUANT, 128, WHOLE)),   # the same over few tiles
+    (1536, 8, 4, 128, 1100, L.T_Q4_0, L.T_Q4_0, 1400, None, "f32", (QUANT, 128, WHOLE)),
     (8192, 8, 8, 128, 1100, L.T_Q8_0, L.T_Q4_0, None, None, "bf16", (STAGED, 256, SHARES)),  # 256-row units, more of them than CUs
-    (4096, 8, 6, 256, 1400, L.T_F16, L.T_F16, 3900, None, "f32", (F16, 256, SHARES)),       # the same, Q in two passes
-    (2048, 8, 8, 128, 1500, L.T_F16, L.T_F16, None, None, "bf16", (F16, 256, WHOLE)),       # the same over few tiles
+    (8192, 8, 6, 256, 1400, L.T_F16, L.T_F16, 7900, None, "f32", (F16, 256, SHARES)),       # the same, Q in two passes
+    (4096, 8, 6, 256, 1400, L.T_F16, L.T_F16, 3900, None, "f32", (F16, 256, WHOLE)),        # the same over few tiles
+    (2048, 8, 8, 128, 1500, L.T_F16, L.T_F16, None, None, "bf16", (F16, 256, WHOLE)),
 ]
 
 
